@@ -1,6 +1,7 @@
 """Build the gfx950 shared library libgdremc.so in-tree with hipcc.
 
-The library holds the HIP kernels (csrc/gd_kernels.hip), the host image of a
+The library holds the HIP kernels (csrc/gd_kernels.hip; FP64 re-score:
+csrc/gd_rescore.hip), the host image of a
 complex (csrc/gd_image.cpp), the engine and the C ABI entry points
 (csrc/gd_engine.cpp), the serving loop (csrc/gd_server.cpp), shared host utilities
 (csrc/gd_host.cpp), the host preparation / parameter parsing
@@ -36,7 +37,8 @@ def build(verbose=True):
     objdir = os.path.join(HERE, "_build")
     os.makedirs(objdir, exist_ok=True)
     objs = []
-    for src, dev in (("gd_kernels.hip", True), ("gd_image.cpp", False), ("gd_engine.cpp", False),
+    for src, dev in (("gd_kernels.hip", True), ("gd_rescore.hip", True),
+                     ("gd_image.cpp", False), ("gd_engine.cpp", False),
                      ("gd_server.cpp", False), ("gd_host.cpp", False), ("gd_prep.cpp", False),
                      ("gd_load.cpp", False)):
         obj = os.path.join(objdir, src + ".o")

@@ -158,6 +158,24 @@ typedef struct gd_task {
   int r_count;
 } gd_task;
 
+/* One workgroup task of the FP64 re-score: `count` poses of one protein
+ * conformer, places begin .. of the launch's pose order or replicas begin ..
+ * of the complex, whose energies go to rows out .. */
+typedef struct gd_r64_task {
+  int cx;
+  int prt;
+  int begin;
+  int count;
+  int out;
+} gd_r64_task;
+
+/* LDS of one pose of the FP64 re-score: its atoms (x, y, z, KDE weight) and
+ * eight slices' sums of eight terms, in double. */
+static inline __host__ __device__ int gd_r64_area_bytes(int max_lna)
+{
+  return max_lna * 32 + 8 * 8 * 8;
+}
+
 /* One temperature chain: (complex, protein conformer * n_lig + ligand conformer). */
 typedef struct gd_chain {
   int cx;

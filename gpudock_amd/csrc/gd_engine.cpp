@@ -904,8 +904,9 @@ int gd_engine::collect_async(GdCollect *cs, int n, hipEvent_t *done)
   int rc = ensure_built();   /* current cx indices; initial energies queued */
   if (rc)
     return rc;
-  std::vector<int2> items;
   std::vector<GdSlot *> ss(n);
+  size_t nitem = 0;
+  int max_lna = 1;
   for (int i = 0; i < n; ++i) {
     GdSlot *s = find(cs[i].handle);
     if (!s)
@@ -913,11 +914,22 @@ int gd_engine::collect_async(GdCollect *cs, int n, hipEvent_t *done)
     if (!cs[i].host || cs[i].host_bytes < collect_bytes(cs[i].handle))
       return gd_fail(GD_ERR_ARG, "read-back buffer too small");
     ss[i] = s;
-    for (int r = 0; r < s->img->P.n_rep; ++r)
-      items.push_back(make_int2(s->cx_index, r));
+    nitem += s->img->P.n_rep;
+    max_lna = std::max(max_lna, s->img->P.lna);
   }
-  const size_t nitem = items.size();
-  const size_t ib = GdArena::round(nitem * sizeof(int2));
+  const int split = gd_rescore64_split((long long) nitem, n_cu);
+  std::vector<gd_r64_task> items;
+  std::vector<gd_task> runs;
+  int lds = 0, row = 0;
+  for (GdSlot *s : ss) {
+    runs.clear();
+    gd_complex_tasks(*s->img, s->cx_index, 8 / split, runs);
+    for (const gd_task &t : runs)
+      items.push_back(gd_r64_task{t.cx, t.prt, t.r_begin, t.r_count, row + t.r_begin});
+    row += s->img->P.n_rep;
+    lds = std::max(lds, gd_rescore64_lds(s->img->P, split, max_lna, max_lds));
+  }
+  const size_t ib = GdArena::round(items.size() * sizeof(gd_r64_task));
   const size_t eb = GdArena::round(nitem * 10 * sizeof(double));
   const size_t ioff = arena_take(*this, ib, true);
   const size_t eoff = ioff == (size_t) -1 ? (size_t) -1 : arena_take(*this, eb, true);
@@ -927,11 +939,12 @@ int gd_engine::collect_async(GdCollect *cs, int n, hipEvent_t *done)
     return gd_fail(GD_ERR_NOMEM, "arena too small for the FP64 re-score");
   }
   const double *e64 = (const double *) (arena.base() + eoff);
-  rc = upload(arena.base() + ioff, items.data(), nitem * sizeof(int2));
+  rc = upload(arena.base() + ioff, items.data(), vbytes(items));
   hipError_t he = rc ? hipSuccess
-                     : gd_launch_rescore64_best((const gd_pack *) (arena.base() + packs_off),
-                                                (const int2 *) (arena.base() + ioff),
-                                                (int) nitem, (double *) e64, stream);
+                     : gd_launch_rescore64((const gd_pack *) (arena.base() + packs_off),
+                                           (const gd_r64_task *) (arena.base() + ioff),
+                                           (int) items.size(), split, max_lna, lds, max_lds,
+                                           nullptr, nullptr, nullptr, (double *) e64, stream);
   size_t first = 0;
   for (int i = 0; i < n && !rc && he == hipSuccess; ++i) {
     GdSlot *s = ss[i];
@@ -1510,14 +1523,24 @@ extern "C" int gd_batch_run(int n_jobs, const gd_job *jobs, const gd_batch_confi
 /* ------------------------------------------------------------------------ */
 namespace {
 
-/* Device layout of one pose-scoring call inside one region: the complex
- * image, the task list, the pose order and arrays, the FP32 and FP64
- * energies, each at a 256-byte aligned offset. */
-struct ScoreLayout {
-  size_t img, tasks, order, lc, pc, mv, e, e64, total;
+/* One pose-scoring call: the host image of the complex, the poses ordered by
+ * protein conformer and the workgroup tasks over that order. */
+struct ScoreJob {
+  GdImage I;
+  std::vector<int> order;
+  std::vector<gd_task> tasks;          /* FP32: up to 8 poses each */
+  std::vector<gd_r64_task> tasks64;    /* FP64: up to 8 / split64 poses each */
+  int split64 = 1, lds64 = 0, max_lds = 65536;
 };
 
-ScoreLayout score_layout(size_t img_bytes, size_t n_tasks, int n_pose)
+/* Its device layout inside one region: the complex image, the task lists,
+ * the pose order and arrays, the FP32 and FP64 energies, each at a 256-byte
+ * aligned offset. */
+struct ScoreLayout {
+  size_t img, tasks, tasks64, order, lc, mv, e, e64, total;
+};
+
+ScoreLayout score_layout(const ScoreJob &J, int n_pose)
 {
   ScoreLayout L;
   size_t off = 0;
@@ -1526,11 +1549,11 @@ ScoreLayout score_layout(size_t img_bytes, size_t n_tasks, int n_pose)
     off += GdArena::round(bytes);
     return o;
   };
-  L.img = take(img_bytes);
-  L.tasks = take(n_tasks * sizeof(gd_task));
+  L.img = take(gd_image_footprint(J.I));
+  L.tasks = take(vbytes(J.tasks));
+  L.tasks64 = take(vbytes(J.tasks64));
   L.order = take((size_t) n_pose * 4);
   L.lc = take((size_t) n_pose * 4);
-  L.pc = take((size_t) n_pose * 4);
   L.mv = take((size_t) n_pose * 24);
   L.e = take((size_t) n_pose * 40);
   L.e64 = take((size_t) n_pose * 80);
@@ -1538,15 +1561,27 @@ ScoreLayout score_layout(size_t img_bytes, size_t n_tasks, int n_pose)
   return L;
 }
 
+/* What a call counts against the static workspace: the image, one task list
+ * and 156 bytes a pose (conformers, order, move, both energies).  The
+ * workspace holds GD_SCRATCH_SLACK more than that limit for the FP64 tasks:
+ * at most 20 bytes a conformer of at least 1.8 KB of image, and 2.5 a pose
+ * against the 4 counted for its protein conformer. */
+size_t score_counted(const ScoreJob &J, int n_pose)
+{
+  size_t b = GdArena::round(gd_image_footprint(J.I)) + GdArena::round(vbytes(J.tasks));
+  for (int per : {4, 4, 4, 24, 40, 80})
+    b += GdArena::round((size_t) n_pose * per);
+  return b;
+}
+
 /* Argument checks, the host image of the complex (the pose arrays ride in it
- * as a one-temperature replica set) and the workgroup tasks: runs of up to 8
- * poses on one protein conformer, poses ordered by conformer. */
+ * as a one-temperature replica set) and the workgroup tasks: runs of poses on
+ * one protein conformer, poses ordered by conformer. */
 int score_prepare(const gd_ligand *lig, const gd_protein *prt, const gd_psp *psp,
                   const gd_kde *kde, const gd_mcs *mcs, const gd_enepara *enepara,
                   gd_complex_size size, int n_pose, const int *lig_conf, const int *prt_conf,
                   const float *move, int term_order, int device, float *energy,
-                  double *energy_fp64, GdImage &I, std::vector<int> &order,
-                  std::vector<gd_task> &tasks)
+                  double *energy_fp64, ScoreJob &J)
 {
   int rc = gd_check_inputs(lig, prt, psp, kde, mcs, enepara, size);
   if (rc)
@@ -1562,69 +1597,82 @@ int score_prepare(const gd_ligand *lig, const gd_protein *prt, const gd_psp *psp
   const int ndev = gd_device_count();
   if (ndev > 0 && (device < 0 || device >= ndev))
     return gd_fail(GD_ERR_ARG, "device %d of %d", device, ndev);
-  int max_lds = 65536;
-  if (ndev > 0)
-    GD_HIP_TRY(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock,
+  int n_cu = 256;
+  if (ndev > 0) {
+    GD_HIP_TRY(hipDeviceGetAttribute(&J.max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock,
                                      device));
+    GD_HIP_TRY(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, device));
+  }
   gd_options o = default_opts(nullptr);
   o.term_order = term_order;
   o.device = device;
   gd_complex_size sz1 = size;
   sz1.n_tmp = 1;
   sz1.n_rep = size.n_lig * size.n_prt;
-  rc = gd_build_image(I, lig, prt, psp, kde, mcs, enepara, nullptr, nullptr, nullptr, sz1, o,
-                      max_lds, 0);
+  rc = gd_build_image(J.I, lig, prt, psp, kde, mcs, enepara, nullptr, nullptr, nullptr, sz1, o,
+                      J.max_lds, 0);
   if (rc)
     return rc;
-  order.resize(n_pose);
+  J.order.resize(n_pose);
   for (int i = 0; i < n_pose; ++i)
-    order[i] = i;
-  std::stable_sort(order.begin(), order.end(),
+    J.order[i] = i;
+  std::stable_sort(J.order.begin(), J.order.end(),
                    [&](int a, int b) { return prt_conf[a] < prt_conf[b]; });
-  tasks.clear();
-  for (int i = 0; i < n_pose;) {
-    int j = i;
-    while (j < n_pose && prt_conf[order[j]] == prt_conf[order[i]] && j - i < 8)
-      ++j;
-    tasks.push_back(gd_task{0, prt_conf[order[i]], i, j - i});
-    i = j;
+  auto runs = [&](int most, auto &&put) {
+    for (int i = 0; i < n_pose;) {
+      const int p = prt_conf[J.order[i]];
+      int j = i;
+      while (j < n_pose && prt_conf[J.order[j]] == p && j - i < most)
+        ++j;
+      put(p, i, j - i);
+      i = j;
+    }
+  };
+  J.tasks.clear();
+  runs(8, [&](int p, int i, int n) { J.tasks.push_back(gd_task{0, p, i, n}); });
+  J.tasks64.clear();
+  if (energy_fp64 && n_pose > 0) {
+    J.split64 = gd_rescore64_split(n_pose, n_cu);
+    J.lds64 = gd_rescore64_lds(J.I.P, J.split64, J.I.P.lna, J.max_lds);
+    runs(8 / J.split64,
+         [&](int p, int i, int n) { J.tasks64.push_back(gd_r64_task{0, p, i, n, 0}); });
   }
   return GD_OK;
 }
 
 /* Uploads, launches and read-back, all ordered on st, into the device
  * region at B laid out as L; returns after st has drained. */
-int score_run(char *B, const ScoreLayout &L, GdImage &I, const std::vector<gd_task> &tasks,
-              const std::vector<int> &order, int n_pose, const int *lig_conf,
-              const int *prt_conf, const float *move, float *energy, double *energy_fp64,
-              hipStream_t st)
+int score_run(char *B, const ScoreLayout &L, ScoreJob &J, int n_pose, const int *lig_conf,
+              const float *move, float *energy, double *energy_fp64, hipStream_t st)
 {
-  const size_t img = gd_image_footprint(I);
+  const size_t img = gd_image_footprint(J.I);
   std::vector<char> host(img);
   GdBlock b;
-  gd_pack_image(I, host.data(), B + L.img, b);
+  gd_pack_image(J.I, host.data(), B + L.img, b);
   const gd_pack *pack_dev = (const gd_pack *) (B + L.img + b.pack);
   /* the host buffers outlive the final synchronisation */
   hipError_t he = hipMemcpyAsync(B + L.img, host.data(), img, hipMemcpyHostToDevice, st);
   auto put = [&](const void *src, size_t bytes, size_t off) {
-    if (he == hipSuccess)
+    if (he == hipSuccess && bytes)
       he = hipMemcpyAsync(B + off, src, bytes, hipMemcpyHostToDevice, st);
   };
-  put(tasks.data(), vbytes(tasks), L.tasks);
-  put(order.data(), (size_t) n_pose * 4, L.order);
+  put(J.tasks.data(), vbytes(J.tasks), L.tasks);
+  put(J.tasks64.data(), vbytes(J.tasks64), L.tasks64);
+  put(J.order.data(), (size_t) n_pose * 4, L.order);
   put(lig_conf, (size_t) n_pose * 4, L.lc);
-  put(prt_conf, (size_t) n_pose * 4, L.pc);
   put(move, (size_t) n_pose * 24, L.mv);
   if (he == hipSuccess && energy) {
-    he = gd_set_kernel_attrs(I.P.lds_bytes);
+    he = gd_set_kernel_attrs(J.I.P.lds_bytes);
     if (he == hipSuccess)
-      he = gd_launch_score(pack_dev, (const gd_task *) (B + L.tasks), (int) tasks.size(),
+      he = gd_launch_score(pack_dev, (const gd_task *) (B + L.tasks), (int) J.tasks.size(),
                            (const int *) (B + L.order), (const int *) (B + L.lc),
-                           (const float *) (B + L.mv), I.P.lds_bytes, (float *) (B + L.e), st);
+                           (const float *) (B + L.mv), J.I.P.lds_bytes, (float *) (B + L.e), st);
   }
   if (he == hipSuccess && energy_fp64)
-    he = gd_launch_rescore64(pack_dev, 0, (const int *) (B + L.lc), (const int *) (B + L.pc),
-                             (const float *) (B + L.mv), 6, n_pose, (double *) (B + L.e64), st);
+    he = gd_launch_rescore64(pack_dev, (const gd_r64_task *) (B + L.tasks64),
+                             (int) J.tasks64.size(), J.split64, J.I.P.lna, J.lds64, J.max_lds,
+                             (const int *) (B + L.order), (const int *) (B + L.lc),
+                             (const float *) (B + L.mv), (double *) (B + L.e64), st);
   if (he == hipSuccess && energy)
     he = hipMemcpyAsync(energy, B + L.e, (size_t) n_pose * 40, hipMemcpyDeviceToHost, st);
   if (he == hipSuccess && energy_fp64)
@@ -1647,11 +1695,9 @@ extern "C" int gd_score_poses(const gd_ligand *lig, const gd_protein *prt,
                               const float *move, int term_order, int device,
                               float *energy, double *energy_fp64)
 {
-  GdImage I;
-  std::vector<int> order;
-  std::vector<gd_task> tasks;
+  ScoreJob J;
   int rc = score_prepare(lig, prt, psp, kde, mcs, enepara, size, n_pose, lig_conf, prt_conf,
-                         move, term_order, device, energy, energy_fp64, I, order, tasks);
+                         move, term_order, device, energy, energy_fp64, J);
   if (rc)
     return rc;
   if (gd_device_count() < 1)
@@ -1659,7 +1705,7 @@ extern "C" int gd_score_poses(const gd_ligand *lig, const gd_protein *prt,
   if (n_pose == 0)
     return GD_OK;
   GD_HIP_TRY(hipSetDevice(device));
-  const ScoreLayout L = score_layout(gd_image_footprint(I), tasks.size(), n_pose);
+  const ScoreLayout L = score_layout(J, n_pose);
   GdArena arena;
   GD_HIP_TRY(arena.init(L.total));
   struct StreamGuard {
@@ -1667,8 +1713,7 @@ extern "C" int gd_score_poses(const gd_ligand *lig, const gd_protein *prt,
     ~StreamGuard() { if (s) (void) hipStreamDestroy(s); }
   } sg;
   GD_HIP_TRY(hipStreamCreateWithFlags(&sg.s, hipStreamNonBlocking));
-  return score_run(arena.base(), L, I, tasks, order, n_pose, lig_conf, prt_conf, move, energy,
-                   energy_fp64, sg.s);
+  return score_run(arena.base(), L, J, n_pose, lig_conf, move, energy, energy_fp64, sg.s);
 }
 
 /* The same scoring with no device allocation: the region is the static
@@ -1680,20 +1725,19 @@ extern "C" int gd_score_poses_noalloc(const gd_ligand *lig, const gd_protein *pr
                                       const int *prt_conf, const float *move, int term_order,
                                       int device, float *energy, double *energy_fp64)
 {
-  GdImage I;
-  std::vector<int> order;
-  std::vector<gd_task> tasks;
+  ScoreJob J;
   int rc = score_prepare(lig, prt, psp, kde, mcs, enepara, size, n_pose, lig_conf, prt_conf,
-                         move, term_order, device, energy, energy_fp64, I, order, tasks);
+                         move, term_order, device, energy, energy_fp64, J);
   if (rc)
     return rc;
-  const ScoreLayout L = score_layout(gd_image_footprint(I), tasks.size(), n_pose);
-  if (L.total > GD_SCRATCH_BYTES)
+  const ScoreLayout L = score_layout(J, n_pose);
+  const size_t need = score_counted(J, n_pose);
+  if (need > GD_SCRATCH_BYTES || L.total > GD_SCRATCH_BYTES + GD_SCRATCH_SLACK)
     return gd_fail(GD_ERR_ARG,
                    "gd_score_poses_noalloc: %d poses of this complex need %zu bytes of "
                    "workspace; the static workspace holds %zu (use gd_score_poses, or fewer "
                    "poses per call)",
-                   n_pose, L.total, (size_t) GD_SCRATCH_BYTES);
+                   n_pose, need, (size_t) GD_SCRATCH_BYTES);
   if (gd_device_count() < 1)
     return gd_fail(GD_ERR_NODEV, "no HIP device visible");
   if (n_pose == 0)
@@ -1701,8 +1745,7 @@ extern "C" int gd_score_poses_noalloc(const gd_ligand *lig, const gd_protein *pr
   GD_HIP_TRY(hipSetDevice(device));
   char *base = nullptr;
   GD_HIP_TRY(gd_scratch_region(device, &base));
-  return score_run(base, L, I, tasks, order, n_pose, lig_conf, prt_conf, move, energy,
-                   energy_fp64, nullptr);
+  return score_run(base, L, J, n_pose, lig_conf, move, energy, energy_fp64, nullptr);
 }
 
 /* ------------------------------------------------------------------------ */

@@ -14,9 +14,7 @@
  *   gd_advance_kernel  advances each complex's device step counter after a
  *                      cycle and re-arms the work queue.
  *   gd_score_kernel    energies of caller-given poses (FP32).
- *   gd_rescore64_kernel FP64 energies of caller-given poses.
- *   gd_rescore64_best_kernel FP64 energies of the best poses of listed
- *                      replicas of many complexes (result read-back).
+ * (FP64 energies: gd_rescore.hip.)
  *
  * Execution model: a workgroup takes a task -- up to WPG replicas of one
  * protein conformer of one complex -- either by its block index or, in the
@@ -102,14 +100,6 @@ __device__ __forceinline__ float gd_wave_sum(float v)
   v += gd_dpp<0x142>(v);   /* rows 1 and 3 are the ones read */
   v += gd_dpp<0x143>(v);   /* row 3 is the one read */
   return gd_bcast(v, 63);
-}
-
-__device__ __forceinline__ double gd_wave_sum64(double v)
-{
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1)
-    v += __shfl_xor(v, off, GD_WAVE);
-  return v;
 }
 
 /* ------------------------------------------------------------------------ */
@@ -1524,229 +1514,6 @@ gd_score_kernel(const gd_pack *__restrict__ packs, const gd_task *__restrict__ t
 }
 
 /* ------------------------------------------------------------------------ */
-/* FP64 re-score: the reference formulas (calcenergy_d.cu:69-309) in double, */
-/* one wavefront per pose, reading the pack straight from HBM.              */
-/* ------------------------------------------------------------------------ */
-/* The Bayesian total in FP64: the same fitted pdfs and the same floor (1e-8
- * for a zero or non-finite pdf or an exponential factor below e^-86). */
-__device__ double gd_pdf64(int family, double x, double loc, double scale)
-{
-  const double pi = 3.14159265358979323846;
-  double v, arg = 0.0;
-  if (family == 0) {
-    const double d = x - loc;
-    arg = -d * d / (2.0 * scale * scale);
-    v = exp(arg) / (scale * sqrt(2.0 * pi));
-  } else if (family == 1) {
-    const double t = (x - loc) / scale;
-    v = 1.0 / (pi * scale * (1.0 + t * t));
-  } else if (family == 2) {
-    arg = -fabs((x - loc) / scale);
-    const double e = exp(arg);
-    v = e / ((1.0 + e) * (1.0 + e)) / scale;
-  } else {
-    const double nx = (x - loc) / scale;
-    if (!(nx > 0.0))
-      return 1e-8;
-    arg = -(nx - 1.0) * (nx - 1.0) / (2.0 * nx);
-    v = exp(arg) / (sqrt(2.0 * pi * nx * nx * nx) * scale);
-  }
-  return (v > 0.0 && v < HUGE_VAL && arg >= -86.0) ? v : 1e-8;
-}
-
-__device__ double gd_bayes_total64(const double nf[9])
-{
-  const float hi[9][2] = GD_BAYES_HIGH_INIT;
-  const float lo[9][2] = GD_BAYES_LOW_INIT;
-  const int fam[9] = GD_BAYES_FAMILY_INIT;
-  double ph = 0.0, pl = 0.0;
-  for (int k = 0; k < 9; ++k) {
-    ph += log10(gd_pdf64(fam[k], nf[k], hi[k][0], hi[k][1]));
-    pl += log10(gd_pdf64(fam[k], nf[k], lo[k][0], lo[k][1]));
-  }
-  return pl - ph;
-}
-
-__device__ void gd_energy64_wave(const gd_pack &P, int lconf, int pconf, const float *move,
-                                 double *__restrict__ out)
-{
-  const int lane = threadIdx.x & (GD_WAVE - 1);
-  const int lna = P.lna, pnp = P.pnp;
-  double m[6];
-  for (int k = 0; k < 6; ++k)
-    m[k] = (double) move[k];
-  const double s1 = sin(m[3]), c1 = cos(m[3]);
-  const double s2 = sin(m[4]), c2 = cos(m[4]);
-  const double s3 = sin(m[5]), c3 = cos(m[5]);
-  const double R[9] = {c1 * c2, c1 * s2 * s3 - c3 * s1, s1 * s3 + c1 * c3 * s2,
-                       c2 * s1, c1 * c3 + s1 * s2 * s3, c3 * s1 * s2 - c1 * s3,
-                       -s2,     c2 * s3,                c2 * c3};
-  const double cen[3] = {(double) P.center[0] + m[0], (double) P.center[1] + m[1],
-                         (double) P.center[2] + m[2]};
-  const float4 *cx = P.lig_xyz + (size_t) lconf * lna;
-  const float4 *pp = P.pt_pos + (size_t) pconf * P.pnp_pad;
-  const float2 *pe = P.pt_eh + (size_t) pconf * P.pnp_pad;
-  const double lj0 = P.sc.lj0, lj1 = P.sc.lj1, el0 = P.sc.el0, el1 = P.sc.el1;
-  const double a1 = 4.0 - 3.0 * el0, b1 = 2.0 * el0 - 3.0;
-
-  double evdw = 0, eele = 0, epmf = 0, epsp = 0, ehdb = 0, ehpc = 0, ekde = 0, elhm = 0;
-  for (int l = 0; l < lna; ++l) {
-    const float4 o = cx[l];
-    const double lx = R[0] * o.x + R[1] * o.y + R[2] * o.z + cen[0];
-    const double ly = R[3] * o.x + R[4] * o.y + R[5] * o.z + cen[1];
-    const double lz = R[6] * o.x + R[7] * o.y + R[8] * o.z + cen[2];
-    const int row = P.lig_row[l];
-    const int lt = P.lig_type[l];
-    const double lq = P.lig_q[l];
-    const gd_pair_param *trow = P.tab + row * GD_ROW_STRIDE;
-    double hpc1 = 0.0;
-    for (int p = lane; p < pnp; p += GD_WAVE) {
-      const float4 q = pp[p];
-      const float2 eh = pe[p];
-      const uint32_t bits = __float_as_uint(q.w);
-      const gd_pair_param tp = trow[bits >> GD_PT_TYPE_SHIFT];
-      const double dx = lx - q.x, dy = ly - q.y, dz = lz - q.z;
-      const double d2 = dx * dx + dy * dy + dz * dz;
-      const double d = sqrt(d2);
-      if (eh.y != 0.0f && d2 <= 81.0) {
-        const double u = d2 / 81.0;
-        hpc1 += (double) eh.y * (1.0 - (3.5 * u - 4.5 * u * u + 2.5 * u * u * u - 0.5 * u * u * u * u));
-      }
-      const double p1 = (double) tp.p1a / (d2 * d2 * d2 * d2 * d);
-      const double p2 = (double) tp.p2a / (d2 * d2 * d2);
-      const double p4 = p1 * lj0 * (1.0 + lj1 * d2) + 1.0;
-      evdw += (p1 - p2) / p4;
-      const double s = el1 * d;
-      const double g = s < 1.0 ? el0 + a1 * s * s + b1 * s * s * s : 1.0 / s;
-      eele += lq * (double) eh.x * g;
-      const double dm = d - (double) tp.pmf0;
-      epmf += (double) tp.pmf1 / (1.0 + exp((-0.5 * d + 6.0) * dm));
-      if (dm <= 0.0)
-        epsp += (double) P.psp_pt[((size_t) pconf * P.n_rows + row) * P.pnp_pad + p];
-      if (tp.hdb0 > 0.1f) {
-        const double h = (d - (double) tp.hdb0) * (double) tp.hdb1;
-        ehdb += (double) tp.hdb1 * exp(-0.5 * h * h);
-      }
-    }
-    hpc1 = gd_wave_sum64(hpc1);
-    const double z = (hpc1 - (double) P.hpl0[lt]) / (double) P.hpl1[lt];
-    ehpc += 0.5 * z * z - (double) P.hpl2[lt];
-
-    const int k0 = P.kde_seg[2 * row], k1 = P.kde_seg[2 * row + 1];
-    double v = 0.0;
-    for (int k = k0 + lane; k < k1; k += GD_WAVE) {
-      const float4 q = P.kde[k];
-      const double ex = lx - q.x, ey = ly - q.y, ez = lz - q.z;
-      v += exp((double) P.kde2 * (ex * ex + ey * ey + ez * ez));
-    }
-    v = gd_wave_sum64(v);
-    if (k1 > k0)
-      ekde += v / (double) (k1 - k0);
-  }
-  evdw = gd_wave_sum64(evdw);
-  eele = gd_wave_sum64(eele);
-  epmf = gd_wave_sum64(epmf);
-  epsp = gd_wave_sum64(epsp);
-  ehdb = gd_wave_sum64(ehdb);
-  ekde = ekde / (double) P.kde3;
-
-  for (int mm = 0; mm < P.pos; ++mm) {
-    double s = 0.0, c = 0.0;
-    for (int l = lane; l < lna; l += GD_WAVE) {
-      const float4 t = P.mcs[(size_t) mm * lna + l];
-      if (t.w != 0.0f) {
-        const float4 o = cx[l];
-        const double lx = R[0] * o.x + R[1] * o.y + R[2] * o.z + cen[0];
-        const double ly = R[3] * o.x + R[4] * o.y + R[5] * o.z + cen[1];
-        const double lz = R[6] * o.x + R[7] * o.y + R[8] * o.z + cen[2];
-        const double dx = lx - t.x, dy = ly - t.y, dz = lz - t.z;
-        s += dx * dx + dy * dy + dz * dz;
-        c += 1.0;
-      }
-    }
-    s = gd_wave_sum64(s);
-    c = gd_wave_sum64(c);
-    if (c > 0.0)
-      elhm += (double) P.mcs_tcc[mm] * sqrt(s / c);
-  }
-  elhm = P.pos > 0 ? log(elhm / (double) P.pos) : 0.0;
-  const double ddx = cen[0] - P.pocket_center[0], ddy = cen[1] - P.pocket_center[1],
-               ddz = cen[2] - P.pocket_center[2];
-  const double edst = sqrt(ddx * ddx + ddy * ddy + ddz * ddz);
-
-  if (lane == 0) {
-    const double fl = (double) lna;
-    double raw[9];
-    raw[GD_F_VDW] = evdw / fl;
-    raw[GD_F_ELE] = eele / fl;
-    raw[GD_F_PMF] = epmf / fl;
-    raw[GD_F_HPC] = ehpc / fl;
-    raw[GD_F_HDB] = -ehdb / fl / sqrt(2.0 * 3.14159265358979323846);
-    raw[GD_F_DST] = edst;
-    raw[GD_F_PSP] = epsp / fl;
-    raw[GD_F_KDE] = ekde / fl;
-    raw[GD_F_LHM] = elhm;
-    const int f2s[9] = GD_FILE_TO_SLOT_INIT;
-    double slot[10];
-    for (int k = 0; k < 9; ++k)
-      slot[f2s[k]] = raw[k];
-    double total = 0.0;
-    if (P.term_order == 0) {
-      for (int k = 0; k < 9; ++k) {
-        const double v = (double) P.a_para[k] * raw[k] + (double) P.b_para[k];
-        slot[f2s[k]] = v;
-        total += (double) P.w[k] * v;
-      }
-    } else {
-      for (int k = 0; k < 9; ++k) {
-        const double v = (double) P.a_para[k] * slot[k] + (double) P.b_para[k];
-        slot[k] = v;
-        total += (double) P.w[k] * v;
-      }
-    }
-    if (P.combine == 1) {
-      double nf[9];
-      for (int k = 0; k < 9; ++k)
-        nf[k] = slot[f2s[k]];
-      total = gd_bayes_total64(nf);
-    }
-    slot[9] = total;
-    for (int k = 0; k < 10; ++k)
-      out[k] = slot[k];
-  }
-}
-
-
-/* FP64 energies of caller-given poses of one complex. */
-__global__ void __launch_bounds__(GD_WAVE)
-gd_rescore64_kernel(const gd_pack *__restrict__ packs, int cx_index,
-                    const int *__restrict__ lig_conf, const int *__restrict__ prt_conf,
-                    const float *__restrict__ move, int move_stride, int n_pose,
-                    double *__restrict__ energy)
-{
-  const int i = blockIdx.x;
-  if (i >= n_pose)
-    return;
-  gd_energy64_wave(packs[cx_index], lig_conf[i], prt_conf[i], move + (size_t) i * move_stride,
-                   energy + (size_t) i * 10);
-}
-
-/* FP64 energies of the best poses of listed replicas (complex, replica) of
- * many complexes, one launch: the read-back of finished jobs. */
-__global__ void __launch_bounds__(GD_WAVE)
-gd_rescore64_best_kernel(const gd_pack *__restrict__ packs, const int2 *__restrict__ items,
-                         int n, double *__restrict__ energy)
-{
-  const int i = blockIdx.x;
-  if (i >= n)
-    return;
-  const int2 it = items[i];
-  const gd_pack &P = packs[it.x];
-  gd_energy64_wave(P, P.rep_lig[it.y], P.rep_prt[it.y], P.S.mv_best + (size_t) it.y * 8,
-                   energy + (size_t) i * 10);
-}
-
-/* ------------------------------------------------------------------------ */
 /* host-callable launch wrappers                                             */
 /* ------------------------------------------------------------------------ */
 template <int WPG, int MINW>
@@ -1845,27 +1612,6 @@ hipError_t gd_launch_score(const gd_pack *packs, const gd_task *tasks, int n_tas
   return hipGetLastError();
 }
 
-hipError_t gd_launch_rescore64_best(const gd_pack *packs, const int2 *items, int n,
-                                    double *energy, hipStream_t st)
-{
-  if (n <= 0)
-    return hipSuccess;
-  hipLaunchKernelGGL(gd_rescore64_best_kernel, dim3(n), dim3(GD_WAVE), 0, st, packs, items, n,
-                     energy);
-  return hipGetLastError();
-}
-
-hipError_t gd_launch_rescore64(const gd_pack *packs, int cx_index, const int *lig_conf,
-                               const int *prt_conf, const float *move, int move_stride,
-                               int n_pose, double *energy, hipStream_t st)
-{
-  if (n_pose <= 0)
-    return hipSuccess;
-  hipLaunchKernelGGL(gd_rescore64_kernel, dim3(n_pose), dim3(GD_WAVE), 0, st, packs,
-                     cx_index, lig_conf, prt_conf, move, move_stride, n_pose, energy);
-  return hipGetLastError();
-}
-
 template <int WPG, int MINW>
 static hipError_t set_attr_var(int bytes)
 {
@@ -1961,7 +1707,7 @@ hipError_t gd_mc_occupancy(const gd_launch_cfg &C, int stage_bytes, int *blocks_
 /* array's name as an address: gd_scratch_region resolves each device's     */
 /* own copy once, with that device current, and hands out that address.     */
 /* ------------------------------------------------------------------------ */
-static __device__ __align__(256) char scratch[GD_SCRATCH_BYTES];
+static __device__ __align__(256) char scratch[GD_SCRATCH_BYTES + GD_SCRATCH_SLACK];
 
 #define GD_SCRATCH_MAX_DEVICES 64
 

@@ -33,21 +33,26 @@ hipError_t gd_launch_advance(const gd_pack *packs, int n_cx, int *queue, int n_q
 hipError_t gd_launch_score(const gd_pack *packs, const gd_task *tasks, int n_tasks,
                            const int *pose_ids, const int *lig_conf, const float *move,
                            int stage_bytes, float *energy, hipStream_t st);
-/* pose i: movematrix at move[i * move_stride .. +6] */
 /* blocks x 256 lanes, each 128 x iters FMAs; out holds blocks x 256 floats */
 hipError_t gd_launch_valu_probe(float *out, int blocks, int iters, hipStream_t st);
 /* one kind of gd_valu_probe_kinds (0 .. GD_VALU_KINDS - 1) */
 hipError_t gd_launch_valu_kind(int kind, float *out, int blocks, int iters, hipStream_t st);
-hipError_t gd_launch_rescore64(const gd_pack *packs, int cx_index, const int *lig_conf,
-                               const int *prt_conf, const float *move, int move_stride,
-                               int n_pose, double *energy, hipStream_t st);
-/* items[i] = (complex index in packs, replica): FP64 energy of its best pose */
-hipError_t gd_launch_rescore64_best(const gd_pack *packs, const int2 *items, int n,
-                                    double *energy, hipStream_t st);
+/* FP64 re-score (gd_rescore.hip): wavefronts per pose for n_pose poses, the
+ * dynamic LDS a complex wants (less is enough: the pocket is then read
+ * through the caches), and the launch -- poses of order[] (energies at row
+ * pose id), or with order null the best poses of the tasks' replicas. */
+int gd_rescore64_split(long long n_pose, int n_cu);
+int gd_rescore64_lds(const gd_pack &P, int split, int max_lna, int max_lds);
+hipError_t gd_launch_rescore64(const gd_pack *packs, const gd_r64_task *tasks, int n_tasks,
+                               int split, int max_lna, int lds_bytes, int max_lds,
+                               const int *order, const int *lig_conf, const float *move,
+                               double *energy, hipStream_t st);
 hipError_t gd_set_kernel_attrs(int stage_bytes);
 
 /* Bytes of the static per-GPU workspace of gd_score_poses_noalloc. */
 #define GD_SCRATCH_BYTES ((size_t) 64 << 20)
+/* room in it beyond what a call is counted for (score_counted) */
+#define GD_SCRATCH_SLACK ((size_t) 1 << 20)
 /* Device address of that workspace on `device`, which must be the current
  * device; resolved once per device (hipGetSymbolAddress) and kept. */
 hipError_t gd_scratch_region(int device, char **ptr);
