@@ -207,37 +207,60 @@ int gd_engine::upload_image(GdImage &I, size_t off, GdBlock &b)
   return GD_OK;
 }
 
-/* Wavefronts per replica.  One, unless the resident replicas are too few to
- * give every SIMD of the device two wavefronts: then 16, 8 or 4 per replica
- * (the most that keeps the total within that), one replica per workgroup.
- * Complexes with more position restraints than the split area holds keep
- * one wavefront per replica. */
-/* Split launches stage every table, the pair list, the restraint targets
- * and the PSP rows in LDS beside the area: restraints beyond the area's
- * slots, a complex whose extras do not fit, or KDE points kept in HBM mean
- * one wavefront per replica. */
+/* Split launches keep the area beside the staged tables: restraints beyond
+ * its slots, or tables that leave no room for it, mean one wavefront per
+ * replica. */
+int gd_engine::stage_of(const GdImage &I) const
+{
+  return std::max(16, kde_global && I.P.kde_in_lds ? I.P.off_kde : I.P.lds_bytes);
+}
+
 bool gd_engine::can_split(const GdImage &I) const
 {
-  const gd_pack &P = I.P;
-  return P.pos <= GD_SPLIT_MAX_POS && P.split_extra && !kde_global &&
-         P.split_lds_bytes + GD_WSLOT_FLOATS * 4 + (int) GD_SPLIT_AREA_BYTES <= max_lds;
+  return I.P.pos <= GD_SPLIT_MAX_POS &&
+         stage_of(I) + GD_SPLIT_LDS_BYTES <= max_lds;
+}
+
+/* Wavefronts per replica for one of the resident complexes, n_rep replicas
+ * in all.  A wavefront issues a dependent instruction every 4 ns and a SIMD
+ * one every 1.06 ns, so one wavefront per replica wants four of them on
+ * every SIMD.  With fewer -- too few replicas, or tables so large that one
+ * workgroup fills a CU's LDS -- a replica is split over a workgroup: 16
+ * wavefronts, or 8 where two such workgroups share a CU and each covers the
+ * other's serial part, once there are more replicas than CUs.  Cycle of 10
+ * steps, one wavefront per replica | split: 592 replicas of 61 atoms x 1,037
+ * points 2.68 | 0.88 ms; 2,048 of 46 x 800 1.51 | 1.17 ms; 2,048 of
+ * 96 x 1,500 (one workgroup a CU) 5.09 | 4.02 ms; 4,096 of 46 x 800 (four
+ * wavefronts a SIMD) 2.2 | 2.3 ms. */
+int gd_engine::split_of(const GdImage &I, long long n_rep) const
+{
+  if (!can_split(I))
+    return 1;
+  if (lc.split == 1 || lc.split == 4 || lc.split == 8 || lc.split == 16)
+    return lc.split;
+  const int stage = stage_of(I);
+  const int groups = std::min(max_lds / (stage + lc.wpg * GD_WSLOT_FLOATS * 4), 20 / lc.wpg);
+  const long long waves = std::min<long long>(std::max(groups, 1) * lc.wpg, n_rep / n_cu);
+  if (waves >= 14)
+    return 1;
+  return n_rep > n_cu && 2 * (stage + GD_SPLIT_LDS_BYTES) <= max_lds ? 8 : 16;
+}
+
+long long gd_engine::replicas() const
+{
+  long long n = 0;
+  for (auto *s : slots)
+    n += s->img->P.n_rep;
+  return n;
 }
 
 int gd_engine::choose_split() const
 {
-  long long reps = 0;
-  for (auto *s : slots) {
-    if (!can_split(*s->img))
-      return 1;
-    reps += s->img->P.n_rep;
-  }
-  if (lc.split == 1 || lc.split == 4 || lc.split == 8 || lc.split == 16)
-    return lc.split;
-  const long long waves = 2LL * 4 * n_cu;
-  for (int s : {16, 8, 4})
-    if (reps > 0 && reps * s <= waves)
-      return s;
-  return 1;
+  const long long n_rep = replicas();
+  int most = 1;
+  for (auto *s : slots)
+    most = std::max(most, split_of(*s->img, n_rep));
+  return most;
 }
 
 /* New device copies of the pack, task and chain arrays for the current
@@ -247,20 +270,21 @@ int gd_engine::rebuild()
 {
   drop_graph();
   split_eff = choose_split();
+  const long long n_rep = replicas();
   gd_launch_cfg lce = lc;
-  lce.split = split_eff;
   std::vector<gd_pack> packs;
   std::vector<gd_chain> chains;
   /* occupancy class of every complex: workgroups per CU at its LDS need */
-  std::map<int, int> occ_cache;
-  auto per_cu_of = [&](int stage) -> int {
-    auto it = occ_cache.find(stage);
+  std::map<std::pair<int, int>, int> occ_cache;
+  auto per_cu_of = [&](int split, int stage) -> int {
+    auto it = occ_cache.find({split, stage});
     if (it != occ_cache.end())
       return it->second;
     int k = 0;
+    lce.split = split;
     if (gd_mc_occupancy(lce, stage, &k) != hipSuccess || k < 1)
       k = 1;
-    occ_cache[stage] = k;
+    occ_cache[{split, stage}] = k;
     return k;
   };
   struct Pending {
@@ -268,7 +292,8 @@ int gd_engine::rebuild()
     std::vector<double> cost;
     int stage = 16;
   };
-  std::map<int, Pending> by_class;   /* key: workgroups per CU */
+  /* key: wavefronts per replica, workgroups per CU */
+  std::map<std::pair<int, int>, Pending> by_class;
   std::vector<gd_task> t1;
   for (auto *s : slots) {
     const int cx = (int) packs.size();
@@ -277,16 +302,14 @@ int gd_engine::rebuild()
     if (kde_global && p.kde_in_lds) {
       p.kde_in_lds = 0;
       p.lds_bytes = p.off_kde;
-      p.split_extra = 0;
-      p.split_lds_bytes = p.lds_bytes;
     }
     packs.push_back(p);
-    const int stage = std::max(16, split_eff > 1 ? std::max(p.lds_bytes, p.split_lds_bytes)
-                                                 : p.lds_bytes);
-    Pending &cl = by_class[per_cu_of(stage)];
+    const int stage = std::max(16, p.lds_bytes);
+    const int split = split_of(*s->img, n_rep);
+    Pending &cl = by_class[{split, per_cu_of(split, stage)}];
     cl.stage = std::max(cl.stage, stage);
     t1.clear();
-    gd_complex_tasks(*s->img, cx, split_eff > 1 ? 1 : lc.wpg, t1);
+    gd_complex_tasks(*s->img, cx, split > 1 ? 1 : lc.wpg, t1);
     for (const gd_task &t : t1) {
       cl.tasks.push_back(t);
       cl.cost.push_back((double) t.r_count * p.lna * p.pnp_pad);
@@ -299,7 +322,7 @@ int gd_engine::rebuild()
    * small ones; classes with the most work launch first */
   std::vector<gd_task> sorted;
   classes.clear();
-  std::vector<std::pair<double, int>> order_cls;
+  std::vector<std::pair<double, std::pair<int, int>>> order_cls;
   for (auto &kv : by_class) {
     double w = 0.0;
     for (double c : kv.second.cost)
@@ -319,7 +342,8 @@ int gd_engine::rebuild()
     c.stage = cl.stage;
     c.off = (int) sorted.size();
     c.n = (int) order.size();
-    c.per_cu = oc.second;
+    c.split = oc.second.first;
+    c.per_cu = oc.second.second;
     c.grid = lc.persistent ? std::min(c.n, c.per_cu * n_cu) : c.n;
     for (int i : order)
       sorted.push_back(cl.tasks[i]);
@@ -424,7 +448,7 @@ static hipError_t launch_classes(gd_engine &E, int *queue_base)
   for (size_t i = 0; i < E.classes.size(); ++i) {
     const gd_engine::Class &c = E.classes[i];
     gd_launch_cfg C = E.lc;
-    C.split = E.split_eff;
+    C.split = c.split;
     C.stage_bytes = c.stage;
     hipError_t e = gd_launch_mc(C, packs, tasks + c.off, c.n,
                                 E.lc.persistent ? queue_base + i : nullptr, c.grid, 0,

@@ -105,17 +105,17 @@ struct gd_engine {
   size_t packs_off = 0, packs_bytes = 0, tasks_off = 0, tasks_bytes = 0, chains_off = 0,
          chains_bytes = 0;
   int n_cx = 0, n_tasks = 0, n_chain = 0;
-  /* MC launches of a cycle: complexes whose LDS need gives the same
-   * workgroups per CU share one launch (tasks [off, off + n) of the task
+  /* MC launches of a cycle: complexes with as many wavefronts per replica
+   * whose LDS need gives the same workgroups per CU share one launch (tasks [off, off + n) of the task
    * list, queue counter = class index), so a large pocket does not lower
    * the occupancy of the small ones */
   struct Class {
-    int stage, off, n, grid, per_cu;
+    int stage, off, n, grid, per_cu, split;
   };
   std::vector<Class> classes;
   int kde_global = 0;               /* 1: every complex reads KDE points from HBM */
-  int split_eff = 1;                /* wavefronts per replica of the current launches
-                                       (lc.split 0 = chosen at each rebuild) */
+  int split_eff = 1;                /* most wavefronts per replica of the current
+                                       launches (lc.split 0 = chosen at each rebuild) */
   int timing = 0;
   std::vector<hipEvent_t> ev_mc, ev_x;
   double mc_ms = 0.0, x_ms = 0.0;
@@ -185,7 +185,12 @@ private:
   int upload_image(GdImage &I, size_t off, GdBlock &b);
   int enqueue_cycle();
   int trial_cycle();
-  /* wavefronts per replica for the resident complexes under lc.split */
+  /* LDS staging bytes of a complex */
+  int stage_of(const GdImage &I) const;
+  long long replicas() const;
+  /* wavefronts per replica of one complex, n_rep replicas resident in all,
+   * and the most over the resident complexes */
+  int split_of(const GdImage &I, long long n_rep) const;
   int choose_split() const;
 };
 typedef gd_engine gd_engine_t;

@@ -378,7 +378,14 @@ int gd_build_image(GdImage &I, const gd_ligand *lig, const gd_protein *prt,
   }
   P.off_kde = al16(P.off_tab + tab_bytes);
   const int with_kde = al16(P.off_kde + (P.pnk + 1) * 16);   /* with the padding point */
-  if (kde_policy != GD_KDE_GLOBAL && with_kde + reserve <= max_lds) {
+  /* the KDE points too, unless that keeps one of two split workgroups off a
+   * CU: read through the caches they cost no measurable time (16,384 replicas
+   * of 48 x 800 with 2,000 KDE points 8.43 ms a cycle staged, 8.36 read
+   * through the caches; 592 of 61 x 1,037 split over 8 wavefronts 1.33 ms at
+   * one workgroup a CU, 0.91 at two) */
+  auto split_groups = [&](int stage) { return std::min(2, max_lds / (stage + GD_SPLIT_LDS_BYTES)); };
+  if (kde_policy != GD_KDE_GLOBAL && with_kde + reserve <= max_lds &&
+      split_groups(with_kde) == split_groups(P.off_kde)) {
     P.kde_in_lds = 1;
     P.lds_bytes = with_kde;
   } else {
@@ -388,15 +395,6 @@ int gd_build_image(GdImage &I, const gd_ligand *lig, const gd_protein *prt,
   if (P.lds_bytes + reserve > max_lds)
     return gd_fail(GD_ERR_ARG, "%d ligand atom types need %d B of LDS (device has %d)",
                    P.n_rows, P.lds_bytes + reserve, max_lds);
-  /* split launches: pair list, restraint targets and PSP rows after the KDE
-   * points, beside the wave slot and the partial-sum area of one replica */
-  const int split_reserve = GD_WSLOT_FLOATS * 4 + (int) GD_SPLIT_AREA_BYTES + 64;
-  P.off_pairs = with_kde;
-  P.off_mcs = al16(P.off_pairs + (int) I.kde_pairs.size() * 4);
-  P.off_psp = al16(P.off_mcs + P.pos * P.lna * 16);
-  const int split_bytes = al16(P.off_psp + P.n_rows * pnp_pad * 4);
-  P.split_extra = P.pocket_in_lds && P.kde_in_lds && split_bytes + split_reserve <= max_lds;
-  P.split_lds_bytes = P.split_extra ? split_bytes : P.lds_bytes;
   return GD_OK;
 }
 

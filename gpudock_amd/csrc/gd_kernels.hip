@@ -133,27 +133,6 @@ __device__ __forceinline__ void gd_stage(const gd_pack &P, int prt, char *smem)
   }
 }
 
-/* Split launches (one replica per workgroup) with split_extra: the
- * (atom, KDE point) pair list, the restraint targets and the PSP rows of
- * protein conformer prt, read every step by every item, staged once. */
-__device__ __forceinline__ void gd_stage_split_extra(const gd_pack &P, int prt, char *smem)
-{
-  const int n_words = ((P.kde_n_lo + GD_WAVE - 1) / GD_WAVE +
-                       (P.kde_n_hi + GD_WAVE - 1) / GD_WAVE) * GD_WAVE;
-  uint32_t *s_pairs = (uint32_t *) (smem + P.off_pairs);
-  for (int i = threadIdx.x; i < n_words; i += blockDim.x)
-    s_pairs[i] = P.kde_pairs[i];
-  float4 *s_mcs = (float4 *) (smem + P.off_mcs);
-  const int n_mcs = P.pos * P.lna;
-  for (int i = threadIdx.x; i < n_mcs; i += blockDim.x)
-    s_mcs[i] = P.mcs[i];
-  float *s_psp = (float *) (smem + P.off_psp);
-  const float *g_psp = P.psp_pt + (size_t) prt * P.n_rows * P.pnp_pad;
-  const int n_psp = P.n_rows * P.pnp_pad;
-  for (int i = threadIdx.x; i < n_psp; i += blockDim.x)
-    s_psp[i] = g_psp[i];
-}
-
 /* ------------------------------------------------------------------------ */
 /* Energy of one pose (calcenergy_d.cu:22-374), in summation blocks          */
 /* (gd_block_size in gd_canon.h): atom blocks of the pair loop, blocks of    */
@@ -169,10 +148,7 @@ struct gd_blk {
 /* Pair loop + hydrophobic restraint (calcenergy_d.cu:56-149) over ligand
  * atoms [l0, l1): lane partials from +0 into blk, the block's restraint sum
  * (uniform) into *ehpc_b, MCC confusion counts (uniform) added to tp/fp/fn.
- * XL (split launches, whose complexes all stage the extras): pocket points,
- * KDE points and PSP rows are all in LDS; else the PSP rows come from HBM
- * and the pocket from LDS or HBM as staged. */
-template <bool XL>
+ * The PSP rows come from HBM, the pocket from LDS or HBM as staged. */
 __device__ __forceinline__ void gd_atoms_block(
     const gd_pack &P, const char *smem, int prt, float ax0, float ay0, float az0, float ax1,
     float ay1, float az1, int l0, int l1, gd_blk &blk, float *ehpc_b, int &tp, int &fp,
@@ -208,7 +184,6 @@ __device__ __forceinline__ void gd_atoms_block(
       (void *) (P.pt_pos + (size_t) prt * P.pnp_pad), 0, P.pnp_pad * 16, GD_BUFFER_DWORD3);
   const __amdgpu_buffer_rsrc_t eh_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       (void *) (P.pt_eh + (size_t) prt * P.pnp_pad), 0, P.pnp_pad * 8, GD_BUFFER_DWORD3);
-  const gd_lds_f32 *psp_lds = (const gd_lds_f32 *) (smem + P.off_psp);
 
   /* the atom loops, for one way of reading the pocket: the choice is made
    * once per call, not per atom */
@@ -248,13 +223,9 @@ __device__ __forceinline__ void gd_atoms_block(
             /* the PSP read (chunk base uniform, lane offset fixed) is consumed
              * at the end of the pair; points outside class 2 hold PSP 0 */
             float pv = 0.0f;
-            if (decltype(psp_tag)::value) {
-              if (XL)
-                pv = psp_lds[row * P.pnp_pad + k * GD_WAVE + lane];
-              else
-                pv = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                    psp_rsrc, ulane * 4u, k * GD_WAVE * 4, 0));
-            }
+            if (decltype(psp_tag)::value)
+              pv = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                  psp_rsrc, ulane * 4u, k * GD_WAVE * 4, 0));
             const float d2 = gd_dist2(lx - q.x, ly - q.y, lz - q.z);
             if (decltype(hpc_tag)::value)
               hacc = gd_hpc_acc2(d2, eh.y, hacc);
@@ -295,7 +266,7 @@ __device__ __forceinline__ void gd_atoms_block(
       }
     }
   };
-  if (XL || pocket_lds) {
+  if (pocket_lds) {
     atoms([&](int k, float4 &q, float2 &eh) {
       const float2 *__restrict__ c = (const float2 *) (smem + k * GD_LDS_CHUNK_BYTES) + lane;
       const float2 xy = c[0], zw = c[GD_WAVE];
@@ -331,7 +302,6 @@ __device__ __forceinline__ void gd_atoms_block(
  * of weight 0 after the segments, so they add exact zeros (the sums are
  * never -0) and every lane keeps its sum.  Returns this lane's sum over
  * rounds [r0, r1) from +0. */
-template <bool XL>
 __device__ __forceinline__ float gd_kde_rounds(const gd_pack &P, const char *smem, float ax0,
                                                float ay0, float az0, float ax1, float ay1,
                                                float az1, int r0, int r1)
@@ -348,10 +318,7 @@ __device__ __forceinline__ float gd_kde_rounds(const gd_pack &P, const char *sme
     /* rounds [ra, rb) of one group, whose atoms lanes hold in (gx, gy, gz);
      * padding entries name lane 0 and the zero-weight point */
     auto entry = [&](int r) -> uint32_t {
-      return XL ? ((const __attribute__((address_space(3))) uint32_t *) (smem + P.off_pairs))
-                      [r * GD_WAVE + ulane]
-                : __builtin_amdgcn_raw_buffer_load_b32(pairs_rsrc, ulane * 4u,
-                                                       r * GD_WAVE * 4, 0);
+      return __builtin_amdgcn_raw_buffer_load_b32(pairs_rsrc, ulane * 4u, r * GD_WAVE * 4, 0);
     };
     auto group = [&](int ra, int rb, float gx, float gy, float gz) {
       if (ra >= rb)
@@ -376,7 +343,7 @@ __device__ __forceinline__ float gd_kde_rounds(const gd_pack &P, const char *sme
     group(r0, r1 < rounds_lo ? r1 : rounds_lo, ax0, ay0, az0);
     group(r0 > rounds_lo ? r0 : rounds_lo, r1, ax1, ay1, az1);
   };
-  if (XL || P.kde_in_lds) {
+  if (P.kde_in_lds) {
     const __attribute__((address_space(3))) char *pts =
         (const __attribute__((address_space(3))) char *) (smem + P.off_kde);
     rounds([&](uint32_t off) {
@@ -402,33 +369,22 @@ __device__ __forceinline__ int gd_kde_round_count(const gd_pack &P)
 
 /* Position restraint m (calcenergy_d.cu:240-258): tcc_m sqrt(mean squared
  * distance of the atoms it names), 0 when it names none (uniform). */
-template <bool XL>
-__device__ __forceinline__ float gd_lhm_one(const gd_pack &P, const char *smem, float ax0,
-                                            float ay0, float az0, float ax1, float ay1,
-                                            float az1, int m)
+__device__ __forceinline__ float gd_lhm_one(const gd_pack &P, float ax0, float ay0, float az0,
+                                            float ax1, float ay1, float az1, int m)
 {
-  typedef const __attribute__((address_space(3))) gd_f4 *lds_f4;
   const int lane = threadIdx.x & (GD_WAVE - 1);
   const int lna = P.lna;
   float s = 0.0f, c = 0.0f;
   const float4 *tm = P.mcs + (size_t) m * lna;
-  const lds_f4 tl = (lds_f4) (smem + P.off_mcs) + m * lna;
-  auto target = [&](int a) -> float4 {
-    if (XL) {
-      const gd_f4 v = tl[a];
-      return make_float4(v.x, v.y, v.z, v.w);
-    }
-    return tm[a];
-  };
   if (lane < lna) {
-    const float4 t = target(lane);
+    const float4 t = tm[lane];
     if (t.w != 0.0f) {
       s += gd_dist2(ax0 - t.x, ay0 - t.y, az0 - t.z);
       c += 1.0f;
     }
   }
   if (lane + GD_WAVE < lna) {
-    const float4 t = target(lane + GD_WAVE);
+    const float4 t = tm[lane + GD_WAVE];
     if (t.w != 0.0f) {
       s += gd_dist2(ax1 - t.x, ay1 - t.y, az1 - t.z);
       c += 1.0f;
@@ -514,7 +470,7 @@ __device__ __forceinline__ void gd_energy_wave(
   for (int l0 = 0; l0 < lna; l0 += bs) {
     gd_blk blk;
     float eb;
-    gd_atoms_block<false>(P, smem, prt, ax0, ay0, az0, ax1, ay1, az1, l0, min(l0 + bs, lna),
+    gd_atoms_block(P, smem, prt, ax0, ay0, az0, ax1, ay1, az1, l0, min(l0 + bs, lna),
                           blk, &eb, tp, fp, fn);
     tot.vdw += blk.vdw;
     tot.pmf += blk.pmf;
@@ -527,11 +483,11 @@ __device__ __forceinline__ void gd_energy_wave(
   const int kbs = gd_block_size(n_rounds > 0 ? n_rounds : 1);
   float kde_lane = 0.0f;
   for (int r0 = 0; r0 < n_rounds; r0 += kbs)
-    kde_lane += gd_kde_rounds<false>(P, smem, ax0, ay0, az0, ax1, ay1, az1, r0,
+    kde_lane += gd_kde_rounds(P, smem, ax0, ay0, az0, ax1, ay1, az1, r0,
                                      min(r0 + kbs, n_rounds));
   float elhm = 0.0f;
   for (int m = 0; m < P.pos; ++m)
-    elhm += gd_lhm_one<false>(P, smem, ax0, ay0, az0, ax1, ay1, az1, m);
+    elhm += gd_lhm_one(P, ax0, ay0, az0, ax1, ay1, az1, m);
   gd_energy_tail(P, tot, ehpc, kde_lane, elhm, tp, fp, fn, cen, out, cmcc);
 }
 
@@ -672,7 +628,6 @@ __device__ __forceinline__ gd_split_sizes gd_split_sizes_of(const gd_pack &P)
   return z;
 }
 
-template <bool XL>
 __device__ __forceinline__ void gd_energy_items(
     const gd_pack &P, const char *smem, gd_lds_f32 *A, int prt, const gd_split_sizes &Z,
     float ax0, float ay0, float az0, float ax1, float ay1, float az1)
@@ -695,7 +650,7 @@ __device__ __forceinline__ void gd_energy_items(
       gd_blk blk;
       float eb;
       int tp = 0, fp = 0, fn = 0;
-      gd_atoms_block<XL>(P, smem, prt, ax0, ay0, az0, ax1, ay1, az1, i * bs,
+      gd_atoms_block(P, smem, prt, ax0, ay0, az0, ax1, ay1, az1, i * bs,
                          min(i * bs + bs, lna), blk, &eb, tp, fp, fn);
       gd_lds_f32 *pb = A + GD_SA_PART + i * 5 * GD_WAVE + lane;
       pb[0 * GD_WAVE] = blk.vdw;
@@ -712,11 +667,11 @@ __device__ __forceinline__ void gd_energy_items(
     } else if (i < nb + nbk) {
       const int kb = i - nb;
       A[GD_SA_KPART + kb * GD_WAVE + lane] =
-          gd_kde_rounds<XL>(P, smem, ax0, ay0, az0, ax1, ay1, az1, kb * kbs,
+          gd_kde_rounds(P, smem, ax0, ay0, az0, ax1, ay1, az1, kb * kbs,
                             min(kb * kbs + kbs, n_rounds));
     } else {
       const int m = i - nb - nbk;
-      const float v = gd_lhm_one<XL>(P, smem, ax0, ay0, az0, ax1, ay1, az1, m);
+      const float v = gd_lhm_one(P, ax0, ay0, az0, ax1, ay1, az1, m);
       if (lane == 0)
         A[GD_SA_LHM + m] = v;
     }
@@ -1072,7 +1027,7 @@ __device__ __forceinline__ void gd_pose_put(const gd_pack &P, gd_lds_f32 *pb, co
   }
 }
 
-/* Items of the pose in buffer pb (split launches stage the extras). */
+/* Items of the pose in buffer pb. */
 __device__ __forceinline__ void gd_pose_items(const gd_pack &P, const char *smem,
                                               gd_lds_f32 *A, const gd_lds_f32 *pb, int prt,
                                               const gd_split_sizes &Z)
@@ -1082,7 +1037,7 @@ __device__ __forceinline__ void gd_pose_items(const gd_pack &P, const char *smem
 #pragma unroll
   for (int k = 0; k < 6; ++k)
     xyz[k] = pb[k * GD_WAVE + lane];
-  gd_energy_items<true>(P, smem, A, prt, Z, xyz[0], xyz[1], xyz[2], xyz[3], xyz[4], xyz[5]);
+  gd_energy_items(P, smem, A, prt, Z, xyz[0], xyz[1], xyz[2], xyz[3], xyz[4], xyz[5]);
 }
 
 /* n_steps MC steps from step s0 of replica r on the SPLIT wavefronts of the
@@ -1464,13 +1419,12 @@ gd_mc_split_kernel(const gd_pack *__restrict__ packs, const gd_task *__restrict_
       if (task.cx != staged_cx || task.prt != staged_prt) {
         __syncthreads();
         gd_stage(P, task.prt, smem);
-        gd_stage_split_extra(P, task.prt, smem);
         __syncthreads();
         staged_cx = task.cx;
         staged_prt = task.prt;
       }
       gd_replica_cycle_split<SPLIT>(P, smem, ws, A, role, task.r_begin, task.prt, s0,
-                                    n_steps);
+                                        n_steps);
     }
     if (!queue)
       t = -2;
@@ -1546,12 +1500,13 @@ static hipError_t launch_mc_wpg(const gd_launch_cfg &C, const gd_pack *packs,
 }
 
 template <int SPLIT>
-static hipError_t launch_split(const gd_pack *packs, const gd_task *tasks, int n_tasks,
-                               int *queue, int grid, int stage_bytes, int prio, hipStream_t st)
+static hipError_t launch_split(const gd_launch_cfg &C, const gd_pack *packs,
+                               const gd_task *tasks, int n_tasks, int *queue, int grid,
+                               hipStream_t st)
 {
-  const int lds = stage_bytes + GD_WSLOT_FLOATS * 4 + (int) GD_SPLIT_AREA_BYTES;
+  const int lds = C.stage_bytes + GD_SPLIT_LDS_BYTES - 64;
   hipLaunchKernelGGL(gd_mc_split_kernel<SPLIT>, dim3(grid), dim3(GD_WAVE * SPLIT), lds, st,
-                     packs, tasks, n_tasks, queue, stage_bytes, prio);
+                     packs, tasks, n_tasks, queue, C.stage_bytes, C.prio);
   return hipGetLastError();
 }
 
@@ -1562,10 +1517,9 @@ hipError_t gd_launch_mc(const gd_launch_cfg &C, const gd_pack *packs, const gd_t
     return hipSuccess;
   if (mode == 0 && C.split > 1) {
     switch (C.split) {
-    case 4: return launch_split<4>(packs, tasks, n_tasks, queue, grid, C.stage_bytes, C.prio, st);
-    case 8: return launch_split<8>(packs, tasks, n_tasks, queue, grid, C.stage_bytes, C.prio, st);
-    case 16:
-      return launch_split<16>(packs, tasks, n_tasks, queue, grid, C.stage_bytes, C.prio, st);
+    case 4: return launch_split<4>(C, packs, tasks, n_tasks, queue, grid, st);
+    case 8: return launch_split<8>(C, packs, tasks, n_tasks, queue, grid, st);
+    case 16: return launch_split<16>(C, packs, tasks, n_tasks, queue, grid, st);
     default: return hipErrorInvalidValue;
     }
   }
@@ -1632,19 +1586,19 @@ static hipError_t set_attr_wpg(int bytes)
 template <int SPLIT>
 static hipError_t set_attr_split(int bytes)
 {
-  /* a complex whose staging and split area exceed the device's LDS never
-   * runs split (the engine checks the same sum), so it needs no attribute */
+  /* at most the device's LDS, less the 64 bytes of room: a complex whose
+   * staging and split area exceed it does not run split (the engine checks
+   * the same sum), but others in the engine may */
   int dev = 0, max_lds = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e == hipSuccess)
     e = hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
   if (e != hipSuccess)
     return e;
-  const int want = bytes + GD_WSLOT_FLOATS * 4 + (int) GD_SPLIT_AREA_BYTES;
-  if (want > max_lds)
-    return hipSuccess;
+  const int want = bytes + GD_SPLIT_LDS_BYTES;
   return hipFuncSetAttribute((const void *) gd_mc_split_kernel<SPLIT>,
-                             hipFuncAttributeMaxDynamicSharedMemorySize, want);
+                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                             (want < max_lds ? want : max_lds) - 64);
 }
 
 hipError_t gd_set_kernel_attrs(int stage_bytes)
@@ -1683,7 +1637,7 @@ static hipError_t occ_split(int stage_bytes, int *blocks)
 {
   return hipOccupancyMaxActiveBlocksPerMultiprocessor(
       blocks, gd_mc_split_kernel<SPLIT>, GD_WAVE * SPLIT,
-      stage_bytes + GD_WSLOT_FLOATS * 4 + (int) GD_SPLIT_AREA_BYTES);
+      stage_bytes + GD_SPLIT_LDS_BYTES - 64);
 }
 
 hipError_t gd_mc_occupancy(const gd_launch_cfg &C, int stage_bytes, int *blocks_per_cu)

@@ -530,7 +530,6 @@ extern "C" int gd_server_create(const gd_server_config *cfg, gd_server **out)
         return gd_fail(GD_ERR_ARG, "lane_split[%d] = %d: 0, 1, 4, 8 or 16", k,
                        s->cfg.lane_split[k]);
       ec.split = s->cfg.lane_split[k];
-      ec.kde_policy = GD_KDE_STAGE_AUTO;   /* split launches read KDE points from LDS */
       l->split_lane = true;
     } else if (s->cfg.lane_split[k] == 1) {
       ec.split = 1;

@@ -397,15 +397,15 @@ typedef struct gd_engine_config {
   int occ;             /* MC kernel register budget: 0 (compiler's choice),
                           6 or 8 waves per SIMD */
   int split;           /* wavefronts per replica in the MC cycles: 0 = chosen
-                          from the resident replica count (several when they
-                          are fewer than the device's SIMDs), 1 = one, or 4, 8,
-                          16 (one replica per workgroup); the energies are the
-                          same bits for every choice.  One wavefront per
-                          replica is used whatever is asked when a resident
-                          complex has more than 64 position restraints, its
-                          pair list, restraint targets and PSP rows do not fit
-                          in LDS beside the split area, or the KDE points are
-                          kept in HBM */
+                          for each resident complex (16 or 8 where one
+                          wavefront per replica would leave a SIMD fewer than
+                          four: few replicas, or tables that fill a CU's
+                          LDS), 1 = one, or 4, 8, 16 (one replica per
+                          workgroup); the energies are the same bits for
+                          every choice.  A complex with more than 64 position
+                          restraints, or whose staged tables leave no room in
+                          LDS for the split area, has one wavefront per
+                          replica whatever is asked */
   int prio;            /* 0-3: issue priority of the MC launches' wavefronts in
                           their SIMD against other streams' launches on the
                           device (s_setprio); 0 = the default */
@@ -434,7 +434,7 @@ typedef struct gd_engine_layout_info {
   int n_classes;       /* MC launches per cycle (occupancy classes) */
   int kde_global;      /* 1: KDE points read from HBM for every complex */
   int occ;             /* MC kernel register budget (waves per SIMD, 0 = default) */
-  int split;           /* wavefronts per replica in the MC cycles */
+  int split;           /* most wavefronts per replica of a resident complex */
 } gd_engine_layout_info;
 
 int gd_engine_create(const gd_engine_config *cfg, gd_engine **out);
@@ -531,9 +531,8 @@ typedef struct gd_server_config {
    * lanes two of them shared a queue and their launches ran in turn; with 8
    * queues they did not, but four lanes served no better than three.
    * lane_split[k] > 1 runs lane k with that many wavefronts per replica (4,
-   * 8 or 16) and KDE points staged in LDS: a few small jobs then fill the
-   * device, so they are done in a few cycles of their own instead of waiting
-   * in a large resident set.  A job that lane cannot split (more than 64
+   * 8 or 16): a few small jobs then fill the device, so they are done in a
+   * few cycles of their own instead of waiting in a large resident set.  A job that lane cannot split (more than 64
    * restraints, or its tables do not fit in LDS beside the split area) goes
    * to the next lane.  0 = split as above.
    * lane_max_jobs[k] > 0: lane k takes a job only while fewer jobs than
