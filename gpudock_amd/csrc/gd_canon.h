@@ -328,13 +328,10 @@ GD_HD float gd_exchange_draw(int fixed_draws, uint32_t w)
 /* ------------------------------------------------------------------ */
 /* Rigid move (reference move_d.cu:79-132)                              */
 /* ------------------------------------------------------------------ */
-/* R = Rz(a) Ry(b) Rx(g) for (a, b, g) = (m[3], m[4], m[5]). */
-GD_HD void gd_rotation(const float m[6], float rot[9])
+/* R = Rz(a) Ry(b) Rx(g) from the sines and cosines of a, b, g. */
+GD_HD void gd_rotation_sc(float s1, float c1, float s2, float c2, float s3, float c3,
+                          float rot[9])
 {
-  float s1, c1, s2, c2, s3, c3;
-  gd_sincos(m[3], &s1, &c1);
-  gd_sincos(m[4], &s2, &c2);
-  gd_sincos(m[5], &s3, &c3);
   rot[0] = c1 * c2;
   rot[1] = c1 * s2 * s3 - c3 * s1;
   rot[2] = s1 * s3 + c1 * c3 * s2;
@@ -344,6 +341,16 @@ GD_HD void gd_rotation(const float m[6], float rot[9])
   rot[6] = -s2;
   rot[7] = c2 * s3;
   rot[8] = c2 * c3;
+}
+
+/* The same for (a, b, g) = (m[3], m[4], m[5]). */
+GD_HD void gd_rotation(const float m[6], float rot[9])
+{
+  float s1, c1, s2, c2, s3, c3;
+  gd_sincos(m[3], &s1, &c1);
+  gd_sincos(m[4], &s2, &c2);
+  gd_sincos(m[5], &s3, &c3);
+  gd_rotation_sc(s1, c1, s2, c2, s3, c3, rot);
 }
 
 /* x' = R x + t + c, summed left to right as in the reference. */

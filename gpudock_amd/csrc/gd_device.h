@@ -184,18 +184,36 @@ typedef struct gd_chain {
 #define GD_WS_ENEW 22
 #define GD_WS_CMCC 32     /* energy_old.cmcc */
 
-/* A replica split over several wavefronts keeps the partial sums of its
- * summation blocks in LDS beside its slot, with three placed poses and
- * the conformer: this many bytes (atom and KDE blocks, restraint values,
- * poses, conformer, sums);
- * complexes with more position restraints than GD_SPLIT_MAX_POS run one
- * wavefront per replica. */
+/* A replica split over several wavefronts keeps beside its slot, in LDS: the
+ * lane partials of its atom blocks (5 terms) and KDE blocks, per atom block
+ * the restraint sum and the MCC counts, the position-restraint values, three
+ * placed poses, the normalised terms, its MCC counts and the
+ * draws of GD_SPLIT_DRAWS steps (offsets in floats).  Complexes with more
+ * position restraints than GD_SPLIT_MAX_POS run one wavefront per replica. */
 #define GD_SPLIT_MAX_POS 64
-#define GD_SPLIT_AREA_BYTES \
-  ((GD_MAX_BLOCKS * 6 * 64 + GD_MAX_BLOCKS * 4 + GD_SPLIT_MAX_POS + 3 * (6 * 64 + 16) + \
-    6 * 64 + 16) * 4)
-/* what a split workgroup takes beside the staged tables: the slot and the
- * area, and 64 bytes of room for its static LDS */
-#define GD_SPLIT_LDS_BYTES ((int) (GD_WSLOT_FLOATS * 4 + GD_SPLIT_AREA_BYTES) + 64)
+#define GD_SPLIT_DRAWS 32
+/* most replicas that share a split workgroup */
+#define GD_SPLIT_MAX_SHARE 4
+#define GD_SA_PART GD_WSLOT_FLOATS
+#define GD_SA_KPART (GD_SA_PART + GD_MAX_BLOCKS * 5 * GD_WAVE)
+#define GD_SA_EHPC (GD_SA_KPART + GD_MAX_BLOCKS * GD_WAVE)
+#define GD_SA_MCC (GD_SA_EHPC + GD_MAX_BLOCKS)
+#define GD_SA_LHM (GD_SA_MCC + GD_MAX_BLOCKS * 3)
+/* pose buffer i: atoms k * 64 + lane (x0 y0 z0 x1 y1 z1), movematrix at
+ * GD_PB_M, centre at GD_PB_CEN */
+#define GD_PB_M (6 * GD_WAVE)
+#define GD_PB_CEN (GD_PB_M + 6)
+#define GD_PB_FLOATS (6 * GD_WAVE + 12)
+#define GD_SA_POSE (GD_SA_LHM + GD_SPLIT_MAX_POS)
+#define GD_SA_TERM (GD_SA_POSE + 3 * GD_PB_FLOATS)   /* terms by parameter index */
+#define GD_SA_CNT (GD_SA_TERM + 12)       /* MCC counts (int) */
+#define GD_SA_SEL (GD_SA_CNT + 3)         /* the pose buffer of the step (int) */
+#define GD_SA_DRAW (GD_SA_CNT + 4)        /* d[6], u, u2 of each step */
+#define GD_SA_FLOATS (GD_SA_DRAW + GD_SPLIT_DRAWS * 8)
+#define GD_SPLIT_AREA_BYTES (GD_SA_FLOATS * 4)
+/* room for a split workgroup's static LDS */
+#define GD_SPLIT_ROOM 64
+/* what a split workgroup of `share` replicas takes beside the staged tables */
+#define GD_SPLIT_LDS_BYTES(share) ((share) * GD_SPLIT_AREA_BYTES + GD_SPLIT_ROOM)
 
 #endif /* GD_DEVICE_H */

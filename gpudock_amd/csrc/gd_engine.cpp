@@ -23,6 +23,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -59,6 +60,7 @@ int gd_engine::init(const gd_engine_config *cfg)
   lc.persistent = c.persistent ? 1 : 0;
   lc.occ = (c.occ == 6 || c.occ == 8) ? c.occ : 0;
   lc.split = (c.split == 1 || c.split == 4 || c.split == 8 || c.split == 16) ? c.split : 0;
+  lc.share = 1;
   lc.prio = c.prio > 0 ? std::min(c.prio, 3) : 0;
   lc.stage_bytes = 16;
   GD_HIP_TRY(hipSetDevice(c.device));
@@ -207,43 +209,65 @@ int gd_engine::upload_image(GdImage &I, size_t off, GdBlock &b)
   return GD_OK;
 }
 
-/* Split launches keep the area beside the staged tables: restraints beyond
- * its slots, or tables that leave no room for it, mean one wavefront per
- * replica. */
+/* Split launches keep their replicas' areas beside the staged tables:
+ * restraints beyond an area's slots, or tables that leave no room for one,
+ * mean one wavefront per replica. */
 int gd_engine::stage_of(const GdImage &I) const
 {
   return std::max(16, kde_global && I.P.kde_in_lds ? I.P.off_kde : I.P.lds_bytes);
 }
 
-bool gd_engine::can_split(const GdImage &I) const
+int gd_engine::max_share(const GdImage &I) const
 {
-  return I.P.pos <= GD_SPLIT_MAX_POS &&
-         stage_of(I) + GD_SPLIT_LDS_BYTES <= max_lds;
+  if (I.P.pos > GD_SPLIT_MAX_POS)
+    return 0;
+  const int room = max_lds - stage_of(I) - GD_SPLIT_LDS_BYTES(0);
+  return std::max(0, std::min(GD_SPLIT_MAX_SHARE, room / GD_SPLIT_AREA_BYTES));
 }
 
-/* Wavefronts per replica for one of the resident complexes, n_rep replicas
- * in all.  A wavefront issues a dependent instruction every 4 ns and a SIMD
- * one every 1.06 ns, so one wavefront per replica wants four of them on
- * every SIMD.  With fewer -- too few replicas, or tables so large that one
- * workgroup fills a CU's LDS -- a replica is split over a workgroup: 16
- * wavefronts, or 8 where two such workgroups share a CU and each covers the
- * other's serial part, once there are more replicas than CUs.  Cycle of 10
- * steps, one wavefront per replica | split: 592 replicas of 61 atoms x 1,037
- * points 2.68 | 0.88 ms; 2,048 of 46 x 800 1.51 | 1.17 ms; 2,048 of
- * 96 x 1,500 (one workgroup a CU) 5.09 | 4.02 ms; 4,096 of 46 x 800 (four
- * wavefronts a SIMD) 2.2 | 2.3 ms. */
-int gd_engine::split_of(const GdImage &I, long long n_rep) const
+bool gd_engine::can_split(const GdImage &I) const { return max_share(I) > 0; }
+
+/* The workgroups of one of the resident complexes, n_rep replicas in all.
+ * A wavefront alone issues an instruction every 6-8 cycles and a SIMD one
+ * every 2.5, so one wavefront per replica wants four of them on every SIMD.
+ * With fewer -- too few replicas, or tables so large that one workgroup fills
+ * a CU's LDS -- replicas are split over workgroups of 16 wavefronts, one a CU.
+ * Up to four share one and its staged tables: they take turns on the same
+ * SIMDs, but the serial end of a step (sums, decision; some 4,000 cycles) is
+ * paid once for all, and a last round of workgroups is not left half empty.
+ * So of the shares that fit, the one with the least rounds x (share + 1).
+ * Cycle of 10 steps of 592 replicas of 61 atoms x 1,037 points: one wavefront
+ * per replica 2.68 ms, two workgroups of 8 a CU, two rounds 0.82 ms, three
+ * replicas a workgroup, one round 0.70 ms; 2,048 of 46 x 800, one wavefront
+ * per replica 1.51 ms, split 1.17 ms; 4,096 of 46 x 800 (four
+ * wavefronts a SIMD) 2.2 ms, split 2.3 ms. */
+gd_engine::Split gd_engine::split_of(const GdImage &I, long long n_rep) const
 {
-  if (!can_split(I))
-    return 1;
-  if (lc.split == 1 || lc.split == 4 || lc.split == 8 || lc.split == 16)
-    return lc.split;
+  const int most = max_share(I);
+  if (most < 1 || lc.split == 1)
+    return {1, 1};
+  if (lc.split > 1) {
+    /* asked for: workgroups of 16 where the areas of 16 / split replicas
+     * fit, else of `split` wavefronts with one */
+    const int share = 16 / lc.split;
+    return share <= most ? Split{16, share} : Split{lc.split, 1};
+  }
   const int stage = stage_of(I);
   const int groups = std::min(max_lds / (stage + lc.wpg * GD_WSLOT_FLOATS * 4), 20 / lc.wpg);
   const long long waves = std::min<long long>(std::max(groups, 1) * lc.wpg, n_rep / n_cu);
   if (waves >= 14)
-    return 1;
-  return n_rep > n_cu && 2 * (stage + GD_SPLIT_LDS_BYTES) <= max_lds ? 8 : 16;
+    return {1, 1};
+  Split best{16, 1};
+  long long best_cost = 0;
+  for (int share = 1; share <= most; ++share) {
+    const long long per_round = (long long) share * n_cu;
+    const long long cost = (n_rep + per_round - 1) / per_round * (share + 1);
+    if (share == 1 || cost < best_cost) {
+      best_cost = cost;
+      best.share = share;
+    }
+  }
+  return best;
 }
 
 long long gd_engine::replicas() const
@@ -259,7 +283,7 @@ int gd_engine::choose_split() const
   const long long n_rep = replicas();
   int most = 1;
   for (auto *s : slots)
-    most = std::max(most, split_of(*s->img, n_rep));
+    most = std::max(most, split_of(*s->img, n_rep).per_replica());
   return most;
 }
 
@@ -275,16 +299,18 @@ int gd_engine::rebuild()
   std::vector<gd_pack> packs;
   std::vector<gd_chain> chains;
   /* occupancy class of every complex: workgroups per CU at its LDS need */
-  std::map<std::pair<int, int>, int> occ_cache;
-  auto per_cu_of = [&](int split, int stage) -> int {
-    auto it = occ_cache.find({split, stage});
+  typedef std::array<int, 3> Key;
+  std::map<Key, int> occ_cache;
+  auto per_cu_of = [&](Split sp, int stage) -> int {
+    auto it = occ_cache.find(Key{sp.waves, sp.share, stage});
     if (it != occ_cache.end())
       return it->second;
     int k = 0;
-    lce.split = split;
+    lce.split = sp.waves;
+    lce.share = sp.share;
     if (gd_mc_occupancy(lce, stage, &k) != hipSuccess || k < 1)
       k = 1;
-    occ_cache[{split, stage}] = k;
+    occ_cache[Key{sp.waves, sp.share, stage}] = k;
     return k;
   };
   struct Pending {
@@ -292,8 +318,9 @@ int gd_engine::rebuild()
     std::vector<double> cost;
     int stage = 16;
   };
-  /* key: wavefronts per replica, workgroups per CU */
-  std::map<std::pair<int, int>, Pending> by_class;
+  /* key: wavefronts of a workgroup (1: one per replica), replicas that share
+   * it, workgroups per CU */
+  std::map<Key, Pending> by_class;
   std::vector<gd_task> t1;
   for (auto *s : slots) {
     const int cx = (int) packs.size();
@@ -305,11 +332,11 @@ int gd_engine::rebuild()
     }
     packs.push_back(p);
     const int stage = std::max(16, p.lds_bytes);
-    const int split = split_of(*s->img, n_rep);
-    Pending &cl = by_class[{split, per_cu_of(split, stage)}];
+    const Split sp = split_of(*s->img, n_rep);
+    Pending &cl = by_class[Key{sp.waves, sp.share, per_cu_of(sp, stage)}];
     cl.stage = std::max(cl.stage, stage);
     t1.clear();
-    gd_complex_tasks(*s->img, cx, split > 1 ? 1 : lc.wpg, t1);
+    gd_complex_tasks(*s->img, cx, sp.waves > 1 ? sp.share : lc.wpg, t1);
     for (const gd_task &t : t1) {
       cl.tasks.push_back(t);
       cl.cost.push_back((double) t.r_count * p.lna * p.pnp_pad);
@@ -322,7 +349,7 @@ int gd_engine::rebuild()
    * small ones; classes with the most work launch first */
   std::vector<gd_task> sorted;
   classes.clear();
-  std::vector<std::pair<double, std::pair<int, int>>> order_cls;
+  std::vector<std::pair<double, Key>> order_cls;
   for (auto &kv : by_class) {
     double w = 0.0;
     for (double c : kv.second.cost)
@@ -342,8 +369,9 @@ int gd_engine::rebuild()
     c.stage = cl.stage;
     c.off = (int) sorted.size();
     c.n = (int) order.size();
-    c.split = oc.second.first;
-    c.per_cu = oc.second.second;
+    c.split = oc.second[0];
+    c.share = oc.second[1];
+    c.per_cu = oc.second[2];
     c.grid = lc.persistent ? std::min(c.n, c.per_cu * n_cu) : c.n;
     for (int i : order)
       sorted.push_back(cl.tasks[i]);
@@ -449,6 +477,7 @@ static hipError_t launch_classes(gd_engine &E, int *queue_base)
     const gd_engine::Class &c = E.classes[i];
     gd_launch_cfg C = E.lc;
     C.split = c.split;
+    C.share = c.share;
     C.stage_bytes = c.stage;
     hipError_t e = gd_launch_mc(C, packs, tasks + c.off, c.n,
                                 E.lc.persistent ? queue_base + i : nullptr, c.grid, 0,
@@ -775,7 +804,7 @@ int gd_engine::autotune(gd_tune_report *rep)
     for (int pers = 0; pers < 2; ++pers)
       trial(wpgs[wi], pers, kg0, occ0, 1);
   if (split_auto > 1)
-    for (int sp : {4, 8, 16})
+    for (int sp : {4, 5, 8, 16})
       for (int pers = 0; pers < 2; ++pers)
         trial(lc.wpg, pers, kg0, occ0, sp);
   {

@@ -110,7 +110,7 @@ struct gd_engine {
    * list, queue counter = class index), so a large pocket does not lower
    * the occupancy of the small ones */
   struct Class {
-    int stage, off, n, grid, per_cu, split;
+    int stage, off, n, grid, per_cu, split, share;
   };
   std::vector<Class> classes;
   int kde_global = 0;               /* 1: every complex reads KDE points from HBM */
@@ -190,7 +190,13 @@ private:
   long long replicas() const;
   /* wavefronts per replica of one complex, n_rep replicas resident in all,
    * and the most over the resident complexes */
-  int split_of(const GdImage &I, long long n_rep) const;
+  /* a complex's workgroups: wavefronts (1: one per replica) and replicas */
+  struct Split {
+    int waves, share;
+    int per_replica() const { return waves / share; }
+  };
+  int max_share(const GdImage &I) const;
+  Split split_of(const GdImage &I, long long n_rep) const;
   int choose_split() const;
 };
 typedef gd_engine gd_engine_t;

@@ -378,14 +378,16 @@ int gd_build_image(GdImage &I, const gd_ligand *lig, const gd_protein *prt,
   }
   P.off_kde = al16(P.off_tab + tab_bytes);
   const int with_kde = al16(P.off_kde + (P.pnk + 1) * 16);   /* with the padding point */
-  /* the KDE points too, unless that keeps one of two split workgroups off a
-   * CU: read through the caches they cost no measurable time (16,384 replicas
-   * of 48 x 800 with 2,000 KDE points 8.43 ms a cycle staged, 8.36 read
-   * through the caches; 592 of 61 x 1,037 split over 8 wavefronts 1.33 ms at
-   * one workgroup a CU, 0.91 at two) */
-  auto split_groups = [&](int stage) { return std::min(2, max_lds / (stage + GD_SPLIT_LDS_BYTES)); };
+  /* the KDE points too, unless that keeps a replica out of a split workgroup:
+   * read through the caches they cost no measurable time (16,384 replicas of
+   * 48 x 800 with 2,000 KDE points 8.43 ms a cycle staged, 8.36 read through
+   * the caches) */
+  auto split_areas = [&](int stage) {
+    return std::min(GD_SPLIT_MAX_SHARE,
+                    (max_lds - stage - GD_SPLIT_LDS_BYTES(0)) / GD_SPLIT_AREA_BYTES);
+  };
   if (kde_policy != GD_KDE_GLOBAL && with_kde + reserve <= max_lds &&
-      split_groups(with_kde) == split_groups(P.off_kde)) {
+      split_areas(with_kde) == split_areas(P.off_kde)) {
     P.kde_in_lds = 1;
     P.lds_bytes = with_kde;
   } else {

@@ -6,8 +6,8 @@
  *                      (montecarlo_d.cu:59-106 with move_d.cu:73-134,
  *                      calcenergy_d.cu:22-374, accept_d.cu:12-52), or the
  *                      initial energies (MonteCarlo_Init_d, :12-55).
- *   gd_mc_split_kernel the same cycle with one replica split over 4, 8 or
- *                      16 wavefronts (launches with few replicas).
+ *   gd_mc_split_kernel the same cycle with one to four replicas split over
+ *                      a workgroup's wavefronts (launches with few replicas).
  *   gd_exchange1_kernel / gd_exchange_kernel temperature swaps, one
  *                      wavefront per chain, one lane per temperature pair
  *                      (exchangereplicas_d.cu:7-136), then the advance.
@@ -140,31 +140,158 @@ __device__ __forceinline__ void gd_stage(const gd_pack &P, int prt, char *smem)
 /* j and j + 64 in (ax0..az0) and (ax1..az1).  prt = the protein conformer   */
 /* staged in smem.                                                           */
 /* ------------------------------------------------------------------------ */
+/* What the energy loops need of a complex and a protein conformer, read once
+ * per cycle and kept in scalar registers.  Read where it is used instead, the
+ * loads are repeated after every barrier and atomic, six of them one behind
+ * the other (some 2,000 cycles) before an atom block's first pair. */
+struct gd_hot {
+  int lna, nchunk, pnp_pad;
+  int kp;                           /* chunks that hold a class-2 point */
+  int off_tab, off_kde, pocket_in_lds, kde_in_lds;
+  int pnk, rounds_lo, n_rounds;     /* KDE rounds of atoms < 64, in all */
+  float kde2, ea1, eb1, lj0, lj01, el01, dcut2;
+  const gd_atom_rec *atom;
+  const float *psp;
+  const float4 *pos;
+  const float2 *eh;
+  const unsigned long long *mref;   /* null: no MCC */
+  const uint32_t *kde_pairs;
+  const float4 *kde;
+  const float4 *mcs;
+  const float *mcs_tcc;
+};
+
+__device__ __forceinline__ gd_hot gd_hot_of(const gd_pack &P, int prt)
+{
+  gd_hot H;
+  H.lna = P.lna;
+  H.pnp_pad = P.pnp_pad;
+  H.nchunk = P.pnp_pad / GD_WAVE;   /* padding points add exact zeros */
+  H.kp = gd_uload(P.chunk_bounds + 2 * prt + 1);
+  H.off_tab = P.off_tab;
+  H.off_kde = P.off_kde;
+  H.pocket_in_lds = P.pocket_in_lds;
+  H.kde_in_lds = P.kde_in_lds;
+  H.pnk = P.pnk;
+  H.rounds_lo = (P.kde_n_lo + GD_WAVE - 1) / GD_WAVE;
+  H.n_rounds = H.rounds_lo + (P.kde_n_hi + GD_WAVE - 1) / GD_WAVE;
+  H.kde2 = P.kde2;
+  H.ea1 = P.sc.ea1;
+  H.eb1 = P.sc.eb1;
+  H.lj0 = P.sc.lj0;
+  H.lj01 = P.sc.lj01;
+  H.el01 = P.sc.el01;
+  H.dcut2 = P.sc.dcut2;
+  H.atom = P.atom;
+  H.psp = P.psp_pt + (size_t) prt * P.n_rows * P.pnp_pad;
+  H.pos = P.pt_pos + (size_t) prt * P.pnp_pad;
+  H.eh = P.pt_eh + (size_t) prt * P.pnp_pad;
+  H.mref = P.mcc_ref ? P.mcc_ref + (size_t) prt * P.lna * H.nchunk : nullptr;
+  H.kde_pairs = P.kde_pairs;
+  H.kde = P.kde;
+  H.mcs = P.mcs;
+  H.mcs_tcc = P.mcs_tcc;
+  return H;
+}
+
 /* Lane partials of the directly summed terms over one atom block. */
 struct gd_blk {
   float vdw, pmf, psp, hdb, ele;
 };
 
+/* Fewest chunks of a pocket that a split replica takes two at a time. */
+#define GD_PAIR_CHUNKS 12
+
+/* Two consecutive chunks of one ligand atom at once: per pair the operations
+ * of gd_pair_terms, the sums in chunk order, so the same bits as two calls.
+ * One pair is a chain of about 40 dependent operations among 54; the two
+ * chains are written side by side so that each fills the other's waits. */
+__device__ __forceinline__ void gd_pair_terms2(const float (&d2)[2], const float (&ele)[2],
+                                               const gd_pair_param (&pp)[2],
+                                               const gd_pair_scalars &sc, bool is_c2,
+                                               const float (&psp)[2], bool hdb_row,
+                                               int near_any, gd_pair_acc &acc,
+                                               int (&contact)[2])
+{
+  float r1[2], d[2], p1[2], p2[2], p4[2], q1[2], rr[2], dm[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    r1[i] = gd_rsqrt(d2[i]);
+    d[i] = d2[i] * r1[i];
+    const float r2 = r1[i] * r1[i];
+    const float r3 = r2 * r1[i];
+    const float r6 = r3 * r3;
+    const float r9 = r6 * r3;
+    p1[i] = pp[i].p1a * r9;
+    p2[i] = pp[i].p2a * r6;
+    p4[i] = gd_fma(p1[i], gd_fma(sc.lj01, d2[i], sc.lj0), 1.0f);
+  }
+  if (near_any) {
+    GD_KEEP_BRANCH();
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const float gn = gd_fma(d2[i], gd_fma(d[i], sc.eb1, sc.ea1), sc.el01);
+      acc.ele = gd_fma(ele[i], d2[i] < sc.dcut2 ? gn : r1[i], acc.ele);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      acc.ele = gd_fma(ele[i], r1[i], acc.ele);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    dm[i] = d[i] - pp[i].pmf0;
+    float es;
+    const float ep = gd_exp_hot_split(gd_fma(-0.5f, d[i], 6.0f) * dm[i], &es);
+    q1[i] = gd_fma(ep, es, 1.0f);
+    rr[i] = gd_rcp(p4[i] * q1[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    acc.vdw = gd_fma((p1[i] - p2[i]) * q1[i], rr[i], acc.vdw);
+    acc.pmf = gd_fma(pp[i].pmf1 * p4[i], rr[i], acc.pmf);
+    if (is_c2)
+      acc.psp += (dm[i] <= 0.0f) ? psp[i] : 0.0f;
+    contact[i] = dm[i] <= 0.0f;
+  }
+  if (hdb_row && (pp[0].hdb0 > 0.1f || pp[1].hdb0 > 0.1f)) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const float h = (d[i] - pp[i].hdb0) * pp[i].hdb1;
+      const float v = gd_fma(pp[i].hdb1, gd_exp_hot((-0.5f * h) * h), acc.hdb);
+      acc.hdb = pp[i].hdb0 > 0.1f ? v : acc.hdb;
+    }
+  }
+}
+
 /* Pair loop + hydrophobic restraint (calcenergy_d.cu:56-149) over ligand
  * atoms [l0, l1): lane partials from +0 into blk, the block's restraint sum
  * (uniform) into *ehpc_b, MCC confusion counts (uniform) added to tp/fp/fn.
  * The PSP rows come from HBM, the pocket from LDS or HBM as staged. */
+template <bool PAIRED>
 __device__ __forceinline__ void gd_atoms_block(
-    const gd_pack &P, const char *smem, int prt, float ax0, float ay0, float az0, float ax1,
+    const gd_hot &H, const char *smem, float ax0, float ay0, float az0, float ax1,
     float ay1, float az1, int l0, int l1, gd_blk &blk, float *ehpc_b, int &tp, int &fp,
     int &fn)
 {
-  const gd_pair_param *__restrict__ s_tab = (const gd_pair_param *) (smem + P.off_tab);
+  const gd_pair_param *__restrict__ s_tab = (const gd_pair_param *) (smem + H.off_tab);
   const int lane = threadIdx.x & (GD_WAVE - 1);
-  const int lna = P.lna;
-  const int nchunk = P.pnp_pad / GD_WAVE;   /* padding points add exact zeros */
-  const int n_rows = P.n_rows;
-  const gd_pair_scalars sc = P.sc;
+  const int nchunk = H.nchunk;
   /* the near-field coefficients and lj0 sit beside other scalars in one
    * fma (one scalar operand per instruction): held in vector registers, the
    * loop needs no copy per pair */
-  gd_pair_scalars sc_v = sc;
+  gd_pair_scalars sc_v;
+  sc_v.ea1 = H.ea1;
+  sc_v.eb1 = H.eb1;
+  sc_v.lj0 = H.lj0;
+  sc_v.lj01 = H.lj01;
+  sc_v.el01 = H.el01;
+  sc_v.dcut2 = H.dcut2;
   asm volatile("" : "+v"(sc_v.ea1), "+v"(sc_v.eb1), "+v"(sc_v.lj0));
+  /* no load may be in flight when the loops begin: the wait for one that an
+   * earlier item left unread (the KDE rounds' last prefetch) would stand
+   * inside the pair loop and catch its own PSP reads */
+  __builtin_amdgcn_s_waitcnt(0x0f70);   /* vmcnt(0) */
 
   gd_pair_acc acc;
   acc.vdw = 0.0f; acc.ele = 0.0f; acc.pmf = 0.0f; acc.psp = 0.0f; acc.hdb = 0.0f;
@@ -173,17 +300,23 @@ __device__ __forceinline__ void gd_atoms_block(
   /* MCC confusion counts (wave-uniform): contacts now vs reference, from one
    * ballot per chunk against the reference mask, read through scalar loads */
   typedef const __attribute__((address_space(4))) unsigned long long *mask_ptr;
-  const mask_ptr mref =
-      P.mcc_ref ? (mask_ptr) (P.mcc_ref + (size_t) prt * lna * nchunk) : nullptr;
+  const mask_ptr mref = (mask_ptr) H.mref;
   typedef const __attribute__((address_space(1))) float *gfloat_ptr;
-  const gfloat_ptr psp_prt = (gfloat_ptr) (P.psp_pt + (size_t) prt * n_rows * P.pnp_pad);
-  const int kp = gd_uload(P.chunk_bounds + 2 * prt + 1);
+  const gfloat_ptr psp_prt = (gfloat_ptr) H.psp;
+  /* Two chunks at a time from GD_PAIR_CHUNKS chunks on: a cycle of 592
+   * replicas of 61 atoms x 17 chunks 757 -> 698 us, of 4,096 of 128 x 63 26.6
+   * -> 25.0 ms; of 128 of 32 x 10 107 -> 108 us, of 64 of 24 x 5 64.7 -> 67.9:
+   * few chunks leave a rest as long as the pairs. */
+  const bool pairs = PAIRED && nchunk >= GD_PAIR_CHUNKS;
+  int kp = H.kp;
+  if (pairs)   /* whole pairs: the chunk past the bound adds exact zeros */
+    kp = min((kp + 1) & ~1, nchunk);
   const unsigned ulane = (unsigned) lane;
-  const int pocket_lds = P.pocket_in_lds;
+  const int pocket_lds = H.pocket_in_lds;
   const __amdgpu_buffer_rsrc_t pos_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      (void *) (P.pt_pos + (size_t) prt * P.pnp_pad), 0, P.pnp_pad * 16, GD_BUFFER_DWORD3);
+      (void *) H.pos, 0, H.pnp_pad * 16, GD_BUFFER_DWORD3);
   const __amdgpu_buffer_rsrc_t eh_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      (void *) (P.pt_eh + (size_t) prt * P.pnp_pad), 0, P.pnp_pad * 8, GD_BUFFER_DWORD3);
+      (void *) H.eh, 0, H.pnp_pad * 8, GD_BUFFER_DWORD3);
 
   /* the atom loops, for one way of reading the pocket: the choice is made
    * once per call, not per atom */
@@ -201,13 +334,13 @@ __device__ __forceinline__ void gd_atoms_block(
         const float lx = gd_bcast(gx, src);
         const float ly = gd_bcast(gy, src);
         const float lz = gd_bcast(gz, src);
-        const gd_atom_rec ar = gd_load_atom(P.atom + l);
+        const gd_atom_rec ar = gd_load_atom(H.atom + l);
         const int row = ar.row;
         const float lq = ar.q;
         const gd_pair_param *trow = s_tab + row * GD_ROW_STRIDE;
         /* the PSP row as a buffer: lane offset fixed, chunk offset scalar */
         const __amdgpu_buffer_rsrc_t psp_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-            (void *) (psp_prt + (size_t) row * P.pnp_pad), 0, P.pnp_pad * 4, GD_BUFFER_DWORD3);
+            (void *) (psp_prt + (size_t) row * H.pnp_pad), 0, H.pnp_pad * 4, GD_BUFFER_DWORD3);
         float hacc = 0.0f;
         acc.ele = 0.0f;
         /* chunks [0, kh) hold the hydrophobic-class points (the canonical order
@@ -215,7 +348,43 @@ __device__ __forceinline__ void gd_atoms_block(
          * every hydrophobic weight and every PSP value is 0, whose terms would
          * add exact zeros, so that loop leaves the terms (and the PSP read) out */
         auto chunks = [&](auto read, auto hpc_tag, auto hdb_tag, auto psp_tag, int k0, int k1) {
-          for (int k = k0; k < k1; ++k) {
+          int k = k0;
+          if (PAIRED)
+            for (; pairs && k + 1 < k1; k += 2) {
+              float4 q[2];
+              float2 eh[2];
+              float pv[2] = {0.0f, 0.0f}, d2[2];
+              gd_pair_param pp[2];
+#pragma unroll
+              for (int i = 0; i < 2; ++i) {
+                read(k + i, q[i], eh[i]);
+                if (decltype(psp_tag)::value)
+                  pv[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                      psp_rsrc, ulane * 4u, (k + i) * GD_WAVE * 4, 0));
+              }
+#pragma unroll
+              for (int i = 0; i < 2; ++i) {
+                pp[i] = *(const gd_pair_param *) ((const char *) trow + __float_as_uint(q[i].w));
+                d2[i] = gd_dist2(lx - q[i].x, ly - q[i].y, lz - q[i].z);
+                if (decltype(hpc_tag)::value)
+                  hacc = gd_hpc_acc2(d2[i], eh[i].y, hacc);
+              }
+              const int near_any = __ballot(fminf(d2[0], d2[1]) < sc_v.dcut2) != 0;
+              const float ele[2] = {eh[0].x, eh[1].x};
+              int contact[2];
+              gd_pair_terms2(d2, ele, pp, sc_v, decltype(psp_tag)::value, pv,
+                             decltype(hdb_tag)::value, near_any, acc, contact);
+              if (mref)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                  const unsigned long long now = __ballot(contact[i]);
+                  const unsigned long long ref = mref[(size_t) l * nchunk + k + i];
+                  tp += __popcll(now & ref);
+                  fp += __popcll(now & ~ref);
+                  fn += __popcll(~now & ref);
+                }
+            }
+          for (; k < k1; ++k) {
             float4 q;
             float2 eh;
             read(k, q, eh);
@@ -302,17 +471,15 @@ __device__ __forceinline__ void gd_atoms_block(
  * of weight 0 after the segments, so they add exact zeros (the sums are
  * never -0) and every lane keeps its sum.  Returns this lane's sum over
  * rounds [r0, r1) from +0. */
-__device__ __forceinline__ float gd_kde_rounds(const gd_pack &P, const char *smem, float ax0,
+__device__ __forceinline__ float gd_kde_rounds(const gd_hot &H, const char *smem, float ax0,
                                                float ay0, float az0, float ax1, float ay1,
                                                float az1, int r0, int r1)
 {
   const unsigned ulane = threadIdx.x & (GD_WAVE - 1);
-  const float kde2 = P.kde2;
-  const int n_lo = P.kde_n_lo, n_hi = P.kde_n_hi;
-  const int rounds_lo = (n_lo + GD_WAVE - 1) / GD_WAVE;
-  const int n_all = (rounds_lo + (n_hi + GD_WAVE - 1) / GD_WAVE) * GD_WAVE;
+  const float kde2 = H.kde2;
+  const int rounds_lo = H.rounds_lo;
   const __amdgpu_buffer_rsrc_t pairs_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      (void *) P.kde_pairs, 0, n_all * 4, GD_BUFFER_DWORD3);
+      (void *) H.kde_pairs, 0, H.n_rounds * GD_WAVE * 4, GD_BUFFER_DWORD3);
   float lane_sum = 0.0f;
   auto rounds = [&](auto read) {
     /* rounds [ra, rb) of one group, whose atoms lanes hold in (gx, gy, gz);
@@ -343,16 +510,16 @@ __device__ __forceinline__ float gd_kde_rounds(const gd_pack &P, const char *sme
     group(r0, r1 < rounds_lo ? r1 : rounds_lo, ax0, ay0, az0);
     group(r0 > rounds_lo ? r0 : rounds_lo, r1, ax1, ay1, az1);
   };
-  if (P.kde_in_lds) {
+  if (H.kde_in_lds) {
     const __attribute__((address_space(3))) char *pts =
-        (const __attribute__((address_space(3))) char *) (smem + P.off_kde);
+        (const __attribute__((address_space(3))) char *) (smem + H.off_kde);
     rounds([&](uint32_t off) {
       return *(const __attribute__((address_space(3))) gd_f4 *) (pts + off);
     });
   } else {
     /* from HBM as a raw buffer */
     const __amdgpu_buffer_rsrc_t kde_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        (void *) P.kde, 0, (P.pnk + 1) * 16, GD_BUFFER_DWORD3);
+        (void *) H.kde, 0, (H.pnk + 1) * 16, GD_BUFFER_DWORD3);
     rounds([&](uint32_t off) {
       return __builtin_bit_cast(gd_f4, __builtin_amdgcn_raw_buffer_load_b128(kde_rsrc, off, 0,
                                                                              0));
@@ -361,38 +528,28 @@ __device__ __forceinline__ float gd_kde_rounds(const gd_pack &P, const char *sme
   return lane_sum;
 }
 
-/* KDE rounds of the pose: (rounds_lo + rounds_hi). */
-__device__ __forceinline__ int gd_kde_round_count(const gd_pack &P)
-{
-  return (P.kde_n_lo + GD_WAVE - 1) / GD_WAVE + (P.kde_n_hi + GD_WAVE - 1) / GD_WAVE;
-}
-
 /* Position restraint m (calcenergy_d.cu:240-258): tcc_m sqrt(mean squared
  * distance of the atoms it names), 0 when it names none (uniform). */
-__device__ __forceinline__ float gd_lhm_one(const gd_pack &P, float ax0, float ay0, float az0,
+__device__ __forceinline__ float gd_lhm_one(const gd_hot &H, float ax0, float ay0, float az0,
                                             float ax1, float ay1, float az1, int m)
 {
   const int lane = threadIdx.x & (GD_WAVE - 1);
-  const int lna = P.lna;
-  float s = 0.0f, c = 0.0f;
-  const float4 *tm = P.mcs + (size_t) m * lna;
-  if (lane < lna) {
-    const float4 t = tm[lane];
-    if (t.w != 0.0f) {
-      s += gd_dist2(ax0 - t.x, ay0 - t.y, az0 - t.z);
-      c += 1.0f;
-    }
-  }
-  if (lane + GD_WAVE < lna) {
-    const float4 t = tm[lane + GD_WAVE];
-    if (t.w != 0.0f) {
-      s += gd_dist2(ax1 - t.x, ay1 - t.y, az1 - t.z);
-      c += 1.0f;
-    }
-  }
+  const int lna = H.lna;
+  float s = 0.0f;
+  int c = 0;   /* atoms it names */
+  const float4 *tm = H.mcs + (size_t) m * lna;
+  float4 t0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), t1 = t0;
+  if (lane < lna)
+    t0 = tm[lane];
+  if (lane + GD_WAVE < lna)
+    t1 = tm[lane + GD_WAVE];
+  if (t0.w != 0.0f)
+    s += gd_dist2(ax0 - t0.x, ay0 - t0.y, az0 - t0.z);
+  if (t1.w != 0.0f)
+    s += gd_dist2(ax1 - t1.x, ay1 - t1.y, az1 - t1.z);
+  c = __popcll(__ballot(t0.w != 0.0f)) + __popcll(__ballot(t1.w != 0.0f));
   s = gd_wave_sum(s);
-  c = gd_wave_sum(c);
-  return c > 0.0f ? gd_uload(P.mcs_tcc + m) * gd_sqrt(s / c) : 0.0f;
+  return c > 0 ? gd_uload(H.mcs_tcc + m) * gd_sqrt(s / (float) c) : 0.0f;
 }
 
 /* From the summed terms to the energies: KDE normalisation, the restraint
@@ -400,10 +557,9 @@ __device__ __forceinline__ float gd_lhm_one(const gd_pack &P, float ax0, float a
  * (calcenergy_d.cu:276-371); out[] (slot order) and *cmcc uniform.  vdw ..
  * kde are the wave sums of the lane totals. */
 /* distance of the placed centre to the pocket centre (calcenergy_d.cu:276-283) */
-__device__ __forceinline__ float gd_edst(const gd_pack &P, const float cen[3])
+__device__ __forceinline__ float gd_edst(const float pc[3], const float cen[3])
 {
-  return gd_sqrt(gd_dist2(cen[0] - P.pocket_center[0], cen[1] - P.pocket_center[1],
-                          cen[2] - P.pocket_center[2]));
+  return gd_sqrt(gd_dist2(cen[0] - pc[0], cen[1] - pc[1], cen[2] - pc[2]));
 }
 
 __device__ __forceinline__ void gd_energy_final_d(const gd_pack &P, float vdw, float ele,
@@ -440,7 +596,7 @@ __device__ __forceinline__ void gd_energy_final(const gd_pack &P, float vdw, flo
                                                 float *cmcc)
 {
   gd_energy_final_d(P, vdw, ele, pmf, hdb, psp, ehpc, kde, elhm_sum, tp, fp, fn,
-                    gd_edst(P, cen), out, cmcc);
+                    gd_edst(P.pocket_center, cen), out, cmcc);
 }
 
 /* The same from the lane totals: their wave sums first. */
@@ -458,19 +614,19 @@ __device__ __forceinline__ void gd_energy_tail(const gd_pack &P, const gd_blk &t
  * order) and *cmcc (MCC against the reference contacts, CalcMcc_d
  * calcmcc_d.cu:148-213, or 0) are identical in every lane. */
 __device__ __forceinline__ void gd_energy_wave(
-    const gd_pack &P, const char *smem, int prt, float ax0, float ay0, float az0, float ax1,
+    const gd_pack &P, const gd_hot &H, const char *smem, float ax0, float ay0, float az0, float ax1,
     float ay1, float az1, const float cen[3], float out[GD_E_N], float *cmcc)
 {
   gd_blk tot;
   tot.vdw = 0.0f; tot.pmf = 0.0f; tot.psp = 0.0f; tot.hdb = 0.0f; tot.ele = 0.0f;
   float ehpc = 0.0f;
   int tp = 0, fp = 0, fn = 0;
-  const int lna = P.lna;
+  const int lna = H.lna;
   const int bs = gd_block_size(lna);
   for (int l0 = 0; l0 < lna; l0 += bs) {
     gd_blk blk;
     float eb;
-    gd_atoms_block(P, smem, prt, ax0, ay0, az0, ax1, ay1, az1, l0, min(l0 + bs, lna),
+    gd_atoms_block<false>(H, smem, ax0, ay0, az0, ax1, ay1, az1, l0, min(l0 + bs, lna),
                           blk, &eb, tp, fp, fn);
     tot.vdw += blk.vdw;
     tot.pmf += blk.pmf;
@@ -479,15 +635,15 @@ __device__ __forceinline__ void gd_energy_wave(
     tot.ele += blk.ele;
     ehpc += eb;
   }
-  const int n_rounds = gd_kde_round_count(P);
+  const int n_rounds = H.n_rounds;
   const int kbs = gd_block_size(n_rounds > 0 ? n_rounds : 1);
   float kde_lane = 0.0f;
   for (int r0 = 0; r0 < n_rounds; r0 += kbs)
-    kde_lane += gd_kde_rounds(P, smem, ax0, ay0, az0, ax1, ay1, az1, r0,
+    kde_lane += gd_kde_rounds(H, smem, ax0, ay0, az0, ax1, ay1, az1, r0,
                                      min(r0 + kbs, n_rounds));
   float elhm = 0.0f;
   for (int m = 0; m < P.pos; ++m)
-    elhm += gd_lhm_one(P, ax0, ay0, az0, ax1, ay1, az1, m);
+    elhm += gd_lhm_one(H, ax0, ay0, az0, ax1, ay1, az1, m);
   gd_energy_tail(P, tot, ehpc, kde_lane, elhm, tp, fp, fn, cen, out, cmcc);
 }
 
@@ -510,21 +666,27 @@ __device__ __forceinline__ void gd_place(const gd_pack &P, const float m[6],
 }
 
 /* Centroid-relative conformer coordinates, two atoms per lane. */
+__device__ __forceinline__ void gd_load_conformer_at(const float4 *cx, int lna, float *bx0,
+                                                     float *by0, float *bz0, float *bx1,
+                                                     float *by1, float *bz1)
+{
+  const int lane = threadIdx.x & (GD_WAVE - 1);
+  *bx0 = *by0 = *bz0 = *bx1 = *by1 = *bz1 = 0.0f;
+  if (lane < lna) {
+    const float4 v = cx[lane];
+    *bx0 = v.x; *by0 = v.y; *bz0 = v.z;
+  }
+  if (lane + GD_WAVE < lna) {
+    const float4 v = cx[lane + GD_WAVE];
+    *bx1 = v.x; *by1 = v.y; *bz1 = v.z;
+  }
+}
+
 __device__ __forceinline__ void gd_load_conformer(const gd_pack &P, int conf, float *bx0,
                                                   float *by0, float *bz0, float *bx1,
                                                   float *by1, float *bz1)
 {
-  const int lane = threadIdx.x & (GD_WAVE - 1);
-  const float4 *cx = P.lig_xyz + (size_t) conf * P.lna;
-  *bx0 = *by0 = *bz0 = *bx1 = *by1 = *bz1 = 0.0f;
-  if (lane < P.lna) {
-    const float4 v = cx[lane];
-    *bx0 = v.x; *by0 = v.y; *bz0 = v.z;
-  }
-  if (lane + GD_WAVE < P.lna) {
-    const float4 v = cx[lane + GD_WAVE];
-    *bx1 = v.x; *by1 = v.y; *bz1 = v.z;
-  }
+  gd_load_conformer_at(P.lig_xyz + (size_t) conf * P.lna, P.lna, bx0, by0, bz0, bx1, by1, bz1);
 }
 
 /* Steps of this cycle for a complex: spe while steps are left (steps_run is
@@ -538,7 +700,8 @@ __device__ __forceinline__ int gd_cycle_steps(const gd_pack &P, int s0)
 /* ------------------------------------------------------------------------ */
 /* One replica, one wavefront.                                               */
 /* ------------------------------------------------------------------------ */
-__device__ __forceinline__ void gd_replica_init(const gd_pack &P, const char *smem, int r)
+__device__ __forceinline__ void gd_replica_init(const gd_pack &P, const gd_hot &H, const char *smem,
+                                                int r)
 {
   const int lane = threadIdx.x & (GD_WAVE - 1);
   const gd_state S = P.S;
@@ -555,7 +718,7 @@ __device__ __forceinline__ void gd_replica_init(const gd_pack &P, const char *sm
   }
   float ax0, ay0, az0, ax1, ay1, az1, cen[3], e[GD_E_N], cm;
   gd_place(P, m, bx0, by0, bz0, bx1, by1, bz1, &ax0, &ay0, &az0, &ax1, &ay1, &az1, cen);
-  gd_energy_wave(P, smem, gd_uload(P.rep_prt + r), ax0, ay0, az0, ax1, ay1, az1, cen, e, &cm);
+  gd_energy_wave(P, H, smem, ax0, ay0, az0, ax1, ay1, az1, cen, e, &cm);
   if (lane == 0) {
     S.cmcc[r] = cm;
     S.cmcc_best[r] = cm;
@@ -574,84 +737,114 @@ __device__ __forceinline__ void gd_replica_init(const gd_pack &P, const char *sm
 }
 
 /* ------------------------------------------------------------------------ */
-/* One replica on SPLIT wavefronts.  Its area in LDS (floats): lane partials */
-/* of every atom block (5 terms x 64 lanes) and of every block of KDE rounds */
-/* (64 lanes); per atom block the restraint sum and the MCC counts; per      */
-/* position restraint its value; three pose buffers (placed atoms, their   */
-/* movematrix and centre); the summed terms; an item counter and the index  */
-/* of the pose being evaluated.  The wavefronts take items (atom blocks,     */
-/* then KDE blocks, then  */
-/* restraints) from the counter until none is left, so one that finishes    */
+/* Replicas split over the wavefronts of a workgroup.  Each replica has an   */
+/* area in LDS (GD_SA_ offsets).  The wavefronts take items -- atom blocks,  */
+/* blocks of KDE rounds, position restraints, of any of the workgroup's      */
+/* replicas -- from one counter until none is left, so one that finishes     */
 /* early takes more.  Each item writes its own slots and the sums read them  */
 /* in block order -- the order one wavefront keeps alone -- so the energies  */
 /* have the same bits whichever wavefront evaluated which item.              */
 /* ------------------------------------------------------------------------ */
-#define GD_SA_PART 0
-#define GD_SA_KPART (GD_MAX_BLOCKS * 5 * GD_WAVE)
-#define GD_SA_EHPC (GD_SA_KPART + GD_MAX_BLOCKS * GD_WAVE)
-#define GD_SA_MCC (GD_SA_EHPC + GD_MAX_BLOCKS)
-#define GD_SA_LHM (GD_SA_MCC + GD_MAX_BLOCKS * 3)
-/* pose buffer i: atoms k * 64 + lane (x0 y0 z0 x1 y1 z1), movematrix at
- * GD_PB_M, centre at GD_PB_CEN */
-#define GD_PB_M (6 * GD_WAVE)
-#define GD_PB_CEN (GD_PB_M + 6)
-#define GD_PB_FLOATS (6 * GD_WAVE + 16)
-#define GD_SA_POSE (GD_SA_LHM + GD_SPLIT_MAX_POS)
-#define GD_SA_CONF (GD_SA_POSE + 3 * GD_PB_FLOATS)  /* the conformer, by lane */
-#define GD_SA_SUMS (GD_SA_CONF + 6 * GD_WAVE)       /* the summed terms */
-#define GD_SA_SEL (GD_SA_SUMS + 14)               /* the pose buffer of this step (int) */
-#define GD_SA_CTR (GD_SA_SUMS + 15)               /* the item counter (int) */
-#define GD_SA_FLOATS (GD_SA_SUMS + 16)
-static_assert(GD_SA_FLOATS * 4 == GD_SPLIT_AREA_BYTES, "split area size");
-
 typedef __attribute__((address_space(3))) int gd_lds_i32;
 
-/* Item counts of a complex, read once per cycle (not after every barrier). */
-struct gd_split_sizes {
-  int bs, nb;          /* atom block size and count */
-  int n_rounds, kbs, nbk;   /* KDE rounds, rounds per block, blocks */
-  int pos, n_items;
-  int mcc;             /* 1: MCC counts are kept */
+/* What the steps need besides, read once per cycle as well: lane k < 10 holds
+ * a_para[k] and b_para[k]. */
+struct gd_split_consts {
+  gd_hot H;
+  int bs, nb;               /* atom block size and count */
+  int kbs, nbk;             /* KDE rounds per block, blocks */
+  int pos;
+  int share, share_inv;     /* replicas of the workgroup; 65536 / share, rounded up */
+  int term_order, combine, fixed_draws, reverse, mcc_pairs;
+  float a_l, b_l;
+  float lna_f, inv_el1, kde3;
+  float center[3], pocket_center[3];
 };
 
-__device__ __forceinline__ gd_split_sizes gd_split_sizes_of(const gd_pack &P)
+__device__ __forceinline__ gd_split_consts gd_split_consts_of(const gd_pack &P, int prt,
+                                                              int share)
 {
-  gd_split_sizes z;
-  z.bs = gd_block_size(P.lna);
-  z.nb = (P.lna + z.bs - 1) / z.bs;
-  z.n_rounds = gd_kde_round_count(P);
-  z.kbs = gd_block_size(z.n_rounds > 0 ? z.n_rounds : 1);
-  z.nbk = (z.n_rounds + z.kbs - 1) / z.kbs;
+  const int lane = threadIdx.x & (GD_WAVE - 1);
+  gd_split_consts z;
+  z.H = gd_hot_of(P, prt);
+  z.bs = gd_block_size(z.H.lna);
+  z.nb = (z.H.lna + z.bs - 1) / z.bs;
+  z.kbs = gd_block_size(z.H.n_rounds > 0 ? z.H.n_rounds : 1);
+  z.nbk = (z.H.n_rounds + z.kbs - 1) / z.kbs;
   z.pos = P.pos;
-  z.n_items = z.nb + z.nbk + z.pos;
-  z.mcc = P.mcc_ref != nullptr;
+  z.share = share;
+  z.share_inv = (65535 + share) / share;
+  z.term_order = P.term_order;
+  z.combine = P.combine;
+  z.fixed_draws = P.fixed_draws;
+  z.reverse = P.reverse;
+  z.mcc_pairs = z.H.lna * P.pnp;   /* padding points are never contacts */
+  z.a_l = lane < 10 ? P.a_para[lane] : 0.0f;
+  z.b_l = lane < 10 ? P.b_para[lane] : 0.0f;
+  z.lna_f = (float) z.H.lna;
+  z.inv_el1 = P.sc.inv_el1;
+  z.kde3 = P.kde3;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    z.center[k] = P.center[k];
+    z.pocket_center[k] = P.pocket_center[k];
+  }
   return z;
 }
 
-__device__ __forceinline__ void gd_energy_items(
-    const gd_pack &P, const char *smem, gd_lds_f32 *A, int prt, const gd_split_sizes &Z,
-    float ax0, float ay0, float az0, float ax1, float ay1, float az1)
+/* Takes items until none is left: `item` first, then by the counter.  Lane j
+ * of sel_l names the pose buffer of replica j.  Item i: block i / share of
+ * replica i % share, so that every replica's atom blocks (the longest items)
+ * come first.  place() runs once: before the first item is worked on, or with
+ * place_late before the second, at the latest when no item is left. */
+template <class F>
+__device__ __forceinline__ void gd_split_items(const char *smem, gd_lds_f32 *areas,
+                                               gd_lds_i32 *ctr, const gd_split_consts &Z,
+                                               int sel_l, int item, bool place_late,
+                                               F place)
 {
   const int lane = threadIdx.x & (GD_WAVE - 1);
-  const int lna = P.lna;
-  const int bs = Z.bs, nb = Z.nb, n_rounds = Z.n_rounds, kbs = Z.kbs, nbk = Z.nbk;
-  const int n_items = Z.n_items;
-  gd_lds_i32 *ctr = (gd_lds_i32 *) (A + GD_SA_CTR);
-  for (;;) {
-    /* every lane adds 1 (one LDS atomic of 64 for the wavefront) and the
-     * first lane's old value / 64 is the item: no lane-divergent branch
-     * feeds the loop */
-    const int got = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_WORKGROUP);
-    const int i = __builtin_amdgcn_readfirstlane(got) >> 6;
-    if (i >= n_items)
+  const int lna = Z.H.lna;
+  const int n_items = (Z.nb + Z.nbk + Z.pos) * Z.share;
+  int j_held = -1;
+  float xyz[6];
+#pragma unroll
+  for (int k = 0; k < 6; ++k)
+    xyz[k] = 0.0f;
+  bool placed = false;
+  for (bool first = true;; first = false) {
+    if (item < 0) {
+      /* every lane adds 1 (one LDS atomic of 64 for the wavefront) and the
+       * first lane's old value / 64 is the item: no lane-divergent branch
+       * feeds the loop */
+      const int got = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_WORKGROUP);
+      item = __builtin_amdgcn_readfirstlane(got) >> 6;
+    }
+    if (!placed && (!first || !place_late || item >= n_items)) {
+      place();
+      placed = true;
+    }
+    if (item >= n_items)
       break;
-    if (i < nb) {
+    /* exact: item < 4 (16 + 16 + 64), share <= 4 */
+    const int i = (item * Z.share_inv) >> 16;
+    const int j = item - i * Z.share;
+    gd_lds_f32 *A = areas + j * GD_SA_FLOATS;
+    if (j != j_held) {
+      const gd_lds_f32 *pb =
+          A + GD_SA_POSE + __builtin_amdgcn_readlane(sel_l, j) * GD_PB_FLOATS + lane;
+#pragma unroll
+      for (int k = 0; k < 6; ++k)
+        xyz[k] = pb[k * GD_WAVE];
+      j_held = j;
+    }
+    if (i < Z.nb) {
       gd_blk blk;
       float eb;
       int tp = 0, fp = 0, fn = 0;
-      gd_atoms_block(P, smem, prt, ax0, ay0, az0, ax1, ay1, az1, i * bs,
-                         min(i * bs + bs, lna), blk, &eb, tp, fp, fn);
+      gd_atoms_block<true>(Z.H, smem, xyz[0], xyz[1], xyz[2], xyz[3], xyz[4], xyz[5],
+                           i * Z.bs, min(i * Z.bs + Z.bs, lna), blk, &eb, tp, fp, fn);
       gd_lds_f32 *pb = A + GD_SA_PART + i * 5 * GD_WAVE + lane;
       pb[0 * GD_WAVE] = blk.vdw;
       pb[1 * GD_WAVE] = blk.pmf;
@@ -664,181 +857,165 @@ __device__ __forceinline__ void gd_energy_items(
         A[GD_SA_MCC + 3 * i + 1] = __int_as_float(fp);
         A[GD_SA_MCC + 3 * i + 2] = __int_as_float(fn);
       }
-    } else if (i < nb + nbk) {
-      const int kb = i - nb;
+    } else if (i < Z.nb + Z.nbk) {
+      const int kb = i - Z.nb;
       A[GD_SA_KPART + kb * GD_WAVE + lane] =
-          gd_kde_rounds(P, smem, ax0, ay0, az0, ax1, ay1, az1, kb * kbs,
-                            min(kb * kbs + kbs, n_rounds));
+          gd_kde_rounds(Z.H, smem, xyz[0], xyz[1], xyz[2], xyz[3], xyz[4], xyz[5], kb * Z.kbs,
+                        min(kb * Z.kbs + Z.kbs, Z.H.n_rounds));
     } else {
-      const int m = i - nb - nbk;
-      const float v = gd_lhm_one(P, ax0, ay0, az0, ax1, ay1, az1, m);
+      const int m = i - Z.nb - Z.nbk;
+      const float v = gd_lhm_one(Z.H, xyz[0], xyz[1], xyz[2], xyz[3], xyz[4], xyz[5], m);
       if (lane == 0)
         A[GD_SA_LHM + m] = v;
     }
+    item = -1;
   }
 }
 
-/* t + src[0] + src[stride] + ... + src[(n - 1) stride], in that order, for
- * n <= GD_MAX_BLOCKS: the values are read eight at a time before they are
- * added, so the LDS loads overlap. */
-__device__ __forceinline__ float gd_ordered_sum(const gd_lds_f32 *src, int stride, int n)
+/* src[0] + src[stride] + ... over the GD_MAX_BLOCKS slots, in order.  Slots
+ * past the last block hold +0, which leaves the sum's bits unchanged (a sum
+ * that starts at +0 is never -0), so no test stands between the adds. */
+__device__ __forceinline__ float gd_ordered_sum(const gd_lds_f32 *src, int stride)
 {
+  float v[GD_MAX_BLOCKS];
+#pragma unroll
+  for (int b = 0; b < GD_MAX_BLOCKS; ++b)
+    v[b] = src[b * stride];
   float t = 0.0f;
 #pragma unroll
-  for (int b0 = 0; b0 < GD_MAX_BLOCKS; b0 += 8) {
-    if (b0 >= n)
-      break;
-    float v[8];
-#pragma unroll
-    for (int b = 0; b < 8; ++b)
-      v[b] = src[(b0 + b) * stride];
-#pragma unroll
-    for (int b = 0; b < 8; ++b)
-      if (b0 + b < n)
-        t += v[b];
-  }
+  for (int b = 0; b < GD_MAX_BLOCKS; ++b)
+    t += v[b];
   return t;
 }
 
-/* After the items: the partials added in block order, spread over the
- * wavefronts -- job j on wavefront j % split: jobs 0-4 the vdw, pmf, psp,
- * hdb, ele lane totals over the atom blocks and their wave sums, job 5 the
- * KDE lane total and its wave sum, job 6 the restraint sum and the MCC
- * counts, job 7 the position-restraint sum -- into the sums area.  Every
- * job reads all its slots before adding (the area has GD_MAX_BLOCKS of
- * each; the adds use the first nb / nbk in order). */
-__device__ __forceinline__ void gd_energy_sums(gd_lds_f32 *A, int role, int split,
-                                               const gd_split_sizes &Z)
+/* file-order term <-> slot, 4 bits each: slot i holds file term s2f[i] */
+#define GD_S2F 0x587346210ull
+#define GD_F2S 0x763845210ull
+
+/* Normalised value of file-order term f (raw: the term as gd_finalize takes
+ * it) into the terms of one step, by the index of the parameter that applies
+ * to it: gd_finalize's operations. */
+__device__ __forceinline__ void gd_term_put(const gd_split_consts &Z,
+                                            gd_lds_f32 *term, int f, float raw)
 {
   const int lane = threadIdx.x & (GD_WAVE - 1);
-  const int nb = Z.nb, nbk = Z.nbk;
-  for (int j = role; j < 8; j += split) {
-    if (j < 6) {
-      const float t = gd_wave_sum(
-          j < 5 ? gd_ordered_sum(A + GD_SA_PART + j * GD_WAVE + lane, 5 * GD_WAVE, nb)
-                : gd_ordered_sum(A + GD_SA_KPART + lane, GD_WAVE, nbk));
-      if (lane == 0)
-        A[GD_SA_SUMS + j] = t;
-    } else if (j == 6) {
-      const float ehpc = gd_ordered_sum(A + GD_SA_EHPC, 1, nb);
+  const int k = Z.term_order ? (int) ((GD_F2S >> (4 * f)) & 0xfu) : f;
+  const float v = gd_fma(gd_bcast(Z.a_l, k), raw, gd_bcast(Z.b_l, k));
+  if (lane == 0)
+    term[k] = v;
+}
+
+/* After the items: the partials added in block order and reduced, each term
+ * normalised, spread over the wavefronts -- job q of a replica: 0-4 the vdw,
+ * pmf, psp, hdb, ele lane totals over the atom blocks and their wave sums, 5
+ * the KDE lane total and its wave sum, 6 the restraint sum and the MCC
+ * counts, 7 the position-restraint sum.  The divisions and the logarithm are done here, by eight
+ * wavefronts at once, not by the one that decides. */
+__device__ __forceinline__ void gd_split_sums(gd_lds_f32 *areas, int role, int split,
+                                              const gd_split_consts &Z)
+{
+  const int lane = threadIdx.x & (GD_WAVE - 1);
+  const int nb = Z.nb;
+  const float lna_f = Z.lna_f;
+  for (int job = role; job < 8 * Z.share; job += split) {
+    const int q = job & 7;
+    gd_lds_f32 *A = areas + (job >> 3) * GD_SA_FLOATS;
+    gd_lds_f32 *term = A + GD_SA_TERM;
+    if (q < 6) {
+      float x = gd_wave_sum(
+          q < 5 ? gd_ordered_sum(A + GD_SA_PART + q * GD_WAVE + lane, 5 * GD_WAVE)
+                : gd_ordered_sum(A + GD_SA_KPART + lane, GD_WAVE));
+      /* file-order term of each job */
+      const int f = (int) ((0x714620u >> (4 * q)) & 0xfu);
+      if (f == GD_F_ELE)
+        x = x * Z.inv_el1;   /* the pair loop sums el1 g */
+      if (f == GD_F_KDE)
+        x = x / Z.kde3;
+      float y = x / lna_f;
+      if (f == GD_F_HDB)
+        y = y / 0x1.40d932p+1f * -1.0f;   /* sqrt(2 pi) */
+      gd_term_put(Z, term, f, y);
+    } else if (q == 6) {
+      gd_term_put(Z, term, GD_F_HPC, gd_ordered_sum(A + GD_SA_EHPC, 1) / lna_f);
       /* the MCC counts are integers: any order */
-      int tp = 0, fp = 0, fn = 0;
-      if (Z.mcc) {
+      if (Z.H.mref) {
         const bool in_b = lane < nb;
-        tp = in_b ? __float_as_int(A[GD_SA_MCC + 3 * lane + 0]) : 0;
-        fp = in_b ? __float_as_int(A[GD_SA_MCC + 3 * lane + 1]) : 0;
-        fn = in_b ? __float_as_int(A[GD_SA_MCC + 3 * lane + 2]) : 0;
+        int tp = in_b ? __float_as_int(A[GD_SA_MCC + 3 * lane + 0]) : 0;
+        int fp = in_b ? __float_as_int(A[GD_SA_MCC + 3 * lane + 1]) : 0;
+        int fn = in_b ? __float_as_int(A[GD_SA_MCC + 3 * lane + 2]) : 0;
 #pragma unroll
         for (int off = 1; off < GD_MAX_BLOCKS; off <<= 1) {
           tp += __shfl_xor(tp, off, GD_WAVE);
           fp += __shfl_xor(fp, off, GD_WAVE);
           fn += __shfl_xor(fn, off, GD_WAVE);
         }
-      }
-      if (lane == 0) {
-        A[GD_SA_SUMS + 6] = ehpc;
-        A[GD_SA_SUMS + 8] = __int_as_float(tp);
-        A[GD_SA_SUMS + 9] = __int_as_float(fp);
-        A[GD_SA_SUMS + 10] = __int_as_float(fn);
+        if (lane == 0) {
+          A[GD_SA_CNT + 0] = __int_as_float(tp);
+          A[GD_SA_CNT + 1] = __int_as_float(fp);
+          A[GD_SA_CNT + 2] = __int_as_float(fn);
+        }
       }
     } else {
-      /* position restraints in order, value m in lane m */
+      /* position restraints in order; the slots past the last hold +0 */
       const int pos = Z.pos;
       float elhm = 0.0f;
       if (pos > 0) {
-        const float lv = lane < pos ? A[GD_SA_LHM + lane] : 0.0f;
-        for (int m = 0; m < pos; ++m)
-          elhm += gd_bcast(lv, m);
+        for (int m0 = 0; m0 < pos; m0 += 8) {
+          float v[8];
+#pragma unroll
+          for (int m = 0; m < 8; ++m)
+            v[m] = A[GD_SA_LHM + m0 + m];
+#pragma unroll
+          for (int m = 0; m < 8; ++m)
+            elhm += v[m];
+        }
+        elhm = gd_log(elhm / (float) pos);
       }
-      if (lane == 0)
-        A[GD_SA_SUMS + 7] = elhm;
+      gd_term_put(Z, term, GD_F_LHM, elhm);
     }
   }
 }
 
-/* What the energies need of a complex, read once per cycle: lane k < 10
- * holds a_para[k] and b_para[k]; the weights are uniform. */
-struct gd_final_consts {
-  float a_l, b_l;
-  float w[GD_F_NTERM];   /* uniform */
-  float lna_f, kde3, inv_el1;
-  int pos, term_order, combine;
-};
-
-__device__ __forceinline__ gd_final_consts gd_final_consts_of(const gd_pack &P)
+/* The Bayesian total of the terms of one step (uniform). */
+__device__ __forceinline__ float gd_split_bayes(const gd_split_consts &Z, const gd_lds_f32 *term)
 {
-  const int lane = threadIdx.x & (GD_WAVE - 1);
-  gd_final_consts F;
-  F.a_l = lane < 10 ? P.a_para[lane] : 0.0f;
-  F.b_l = lane < 10 ? P.b_para[lane] : 0.0f;
+  float nf[GD_F_NTERM];
 #pragma unroll
-  for (int k = 0; k < GD_F_NTERM; ++k)
-    F.w[k] = P.w[k];
-  F.lna_f = (float) P.lna;
-  F.kde3 = P.kde3;
-  F.inv_el1 = P.sc.inv_el1;
-  F.pos = P.pos;
-  F.term_order = P.term_order;
-  F.combine = P.combine;
-  return F;
+  for (int f = 0; f < GD_F_NTERM; ++f)
+    nf[f] = term[Z.term_order ? (int) ((GD_F2S >> (4 * f)) & 0xfu) : f];
+  return gd_bayes_total(nf);
 }
 
-/* Wavefront 0, after the sums: the energies (edst: the distance term of the
- * placed centre).  The weighted-sum total (combine 0) with one term per
- * lane: lane L takes parameter L and the term it applies to -- file-order
- * term L (term_order 0) or the term of slot L (term_order 1) -- and forms
- * it with the operations of gd_energy_final_d / gd_finalize (one division
- * sequence serves every term); the total adds w x value over the lanes in
- * parameter order, as gd_finalize does.  Bitwise equal to
- * gd_energy_final_d, which the Bayesian total still uses. */
-__device__ __forceinline__ void gd_energy_combine(const gd_pack &P, const gd_lds_f32 *A,
-                                                  const gd_final_consts &F, float edst,
-                                                  float out[GD_E_N], float *cmcc)
+/* The weighted sum of the terms of one step, in parameter order. */
+__device__ __forceinline__ float gd_split_total(const gd_lds_f32 *term, const float *w)
 {
-  const gd_lds_f32 *S = A + GD_SA_SUMS;
-  if (F.combine != 0) {
-    gd_energy_final_d(P, S[0], S[4], S[1], S[3], S[2], S[6], S[5], S[7],
-                      __float_as_int(S[8]), __float_as_int(S[9]), __float_as_int(S[10]), edst,
-                      out, cmcc);
-    return;
-  }
-  const int lane = threadIdx.x & (GD_WAVE - 1);
-  const int L = lane < GD_F_NTERM ? lane : 0;
-  /* file-order term of each slot (slot i holds file term s2f[i]), 4 bits each */
-  const unsigned long long s2f = 0x587346210ull;
-  /* the sums-area word of each file-order term (term 5 is edst) */
-  const unsigned long long fword = 0x752036140ull;
-  const int f = F.term_order ? (int) ((s2f >> (4 * L)) & 0xfu) : L;
-  float x = S[(int) ((fword >> (4 * f)) & 0xfu)];
-  if (f == GD_F_ELE)
-    x = x * F.inv_el1;   /* the pair loop sums el1 g */
-  if (f == GD_F_KDE)
-    x = x / F.kde3;
-  float y = x / F.lna_f;
-  if (f == GD_F_HDB)
-    y = y / 0x1.40d932p+1f * -1.0f;   /* sqrt(2 pi) */
-  if (f == GD_F_DST)
-    y = edst;
-  if (f == GD_F_LHM)
-    y = F.pos > 0 ? gd_log(x / (float) F.pos) : 0.0f;
-  const float v = gd_fma(F.a_l, y, F.b_l);
   float total = 0.0f;
 #pragma unroll
   for (int k = 0; k < GD_F_NTERM; ++k)
-    total = gd_fma(F.w[k], gd_bcast(v, k), total);
-#pragma unroll
-  for (int i = 0; i < GD_F_NTERM; ++i) {
-    /* the lane that formed slot i */
-    const int src = F.term_order ? i : (int) ((s2f >> (4 * i)) & 0xfu);
-    out[i] = gd_bcast(v, src);
-  }
-  out[GD_E_TOTAL] = total;
-  *cmcc = 0.0f;
-  if (P.mcc_ref) {
-    const int tp = __float_as_int(S[8]), fp = __float_as_int(S[9]), fn = __float_as_int(S[10]);
-    const int tn = P.lna * P.pnp - tp - fp - fn;
-    *cmcc = gd_mcc((float) tp, (float) fn, (float) fp, (float) tn);
-  }
+    total = gd_fma(w[k], term[k], total);
+  return total;
+}
+
+/* Lane i < GD_E_N: the energy of slot i. */
+__device__ __forceinline__ float gd_split_energy(const gd_split_consts &Z, const gd_lds_f32 *term,
+                                                 float total)
+{
+  const int lane = threadIdx.x & (GD_WAVE - 1);
+  const int i = lane < GD_F_NTERM ? lane : 0;
+  const int k = Z.term_order ? i : (int) ((GD_S2F >> (4 * i)) & 0xfu);
+  const float v = term[k];
+  return lane == GD_E_TOTAL ? total : v;
+}
+
+/* MCC from the counts of the step's sums (uniform; 0 without MCC). */
+__device__ __forceinline__ float gd_split_mcc(const gd_split_consts &Z, const gd_lds_f32 *A)
+{
+  if (!Z.H.mref)
+    return 0.0f;
+  const int tp = __float_as_int(A[GD_SA_CNT + 0]), fp = __float_as_int(A[GD_SA_CNT + 1]);
+  const int fn = __float_as_int(A[GD_SA_CNT + 2]);
+  const int tn = Z.mcc_pairs - tp - fp - fn;
+  return gd_mcc((float) tp, (float) fn, (float) fp, (float) tn);
 }
 
 /* The draws of step s of replica r (move_d.cu:73-84, accept_d.cu:20-27): the
@@ -955,9 +1132,9 @@ __device__ __forceinline__ void gd_slot_store(const gd_pack &P, const gd_lds_f32
 /* n_steps MC steps from step s0 of replica r on one wavefront.  The
  * movematrices and energies live in the replica's LDS slot
  * ws[GD_WSLOT_FLOATS]; only totals stay in registers. */
-__device__ __forceinline__ void gd_replica_cycle(const gd_pack &P, const char *smem,
-                                                 gd_lds_f32 *ws, int r, int prt, int s0,
-                                                 int n_steps)
+__device__ __forceinline__ void gd_replica_cycle(const gd_pack &P, const gd_hot &H,
+                                                 const char *smem, gd_lds_f32 *ws, int r,
+                                                 int s0, int n_steps)
 {
   const int lane = threadIdx.x & (GD_WAVE - 1);
   const gd_state S = P.S;
@@ -993,167 +1170,211 @@ __device__ __forceinline__ void gd_replica_cycle(const gd_pack &P, const char *s
       for (int k = 0; k < 6; ++k)
         ws[GD_WS_MNEW + k] = m_new[k];
     }
-    gd_energy_wave(P, smem, prt, ax0, ay0, az0, ax1, ay1, az1, cen, e_new, &cm_new);
+    gd_energy_wave(P, H, smem, ax0, ay0, az0, ax1, ay1, az1, cen, e_new, &cm_new);
     acs += gd_accept(P, ws, r, s, u_acc, mb, e_new, cm_new, &e_old_total, &best_total);
     __builtin_amdgcn_wave_barrier();
   }
   gd_slot_store(P, ws, r, acs);
 }
 
-/* Wavefront 0: pose buffer pb from movematrix m and the conformer staged
- * at conf (lane-wise atoms; the movematrix and centre by lane 0). */
-__device__ __forceinline__ void gd_pose_put(const gd_pack &P, gd_lds_f32 *pb, const float m[6],
-                                            const gd_lds_f32 *conf)
+/* Pose buffer pb from the movematrix that lanes 0-5 hold (m_l) and ligand
+ * conformer conf: one sine-cosine sequence serves the three angles. */
+__device__ __forceinline__ void gd_pose_put(const gd_split_consts &Z, gd_lds_f32 *pb,
+                                            float m_l, const float4 *conf)
 {
   const int lane = threadIdx.x & (GD_WAVE - 1);
-  const float bx0 = conf[0 * GD_WAVE + lane], by0 = conf[1 * GD_WAVE + lane];
-  const float bz0 = conf[2 * GD_WAVE + lane], bx1 = conf[3 * GD_WAVE + lane];
-  const float by1 = conf[4 * GD_WAVE + lane], bz1 = conf[5 * GD_WAVE + lane];
-  float ax0, ay0, az0, ax1, ay1, az1, cen[3];
-  gd_place(P, m, bx0, by0, bz0, bx1, by1, bz1, &ax0, &ay0, &az0, &ax1, &ay1, &az1, cen);
+  float bx0, by0, bz0, bx1, by1, bz1;
+  gd_load_conformer_at(conf, Z.H.lna, &bx0, &by0, &bz0, &bx1, &by1, &bz1);
+  float s_l, c_l;
+  gd_sincos(m_l, &s_l, &c_l);
+  float rot[9];
+  gd_rotation_sc(gd_bcast(s_l, 3), gd_bcast(c_l, 3), gd_bcast(s_l, 4), gd_bcast(c_l, 4),
+                 gd_bcast(s_l, 5), gd_bcast(c_l, 5), rot);
+  const float m[6] = {gd_bcast(m_l, 0), gd_bcast(m_l, 1), gd_bcast(m_l, 2), 0.0f, 0.0f, 0.0f};
+  const float c[3] = {Z.center[0], Z.center[1], Z.center[2]};
+  float ax0, ay0, az0, ax1, ay1, az1;
+  gd_transform(rot, m, c, bx0, by0, bz0, &ax0, &ay0, &az0);
+  gd_transform(rot, m, c, bx1, by1, bz1, &ax1, &ay1, &az1);
   pb[0 * GD_WAVE + lane] = ax0;
   pb[1 * GD_WAVE + lane] = ay0;
   pb[2 * GD_WAVE + lane] = az0;
   pb[3 * GD_WAVE + lane] = ax1;
   pb[4 * GD_WAVE + lane] = ay1;
   pb[5 * GD_WAVE + lane] = az1;
+  if (lane < 6)
+    pb[GD_PB_M + lane] = m_l;
   if (lane == 0) {
 #pragma unroll
-    for (int k = 0; k < 6; ++k)
-      pb[GD_PB_M + k] = m[k];
-#pragma unroll
     for (int k = 0; k < 3; ++k)
-      pb[GD_PB_CEN + k] = cen[k];
+      pb[GD_PB_CEN + k] = c[k] + m[k];
   }
 }
 
-/* Items of the pose in buffer pb. */
-__device__ __forceinline__ void gd_pose_items(const gd_pack &P, const char *smem,
-                                              gd_lds_f32 *A, const gd_lds_f32 *pb, int prt,
-                                              const gd_split_sizes &Z)
+/* The distance term of the pose in buffer pb. */
+__device__ __forceinline__ float gd_pose_edst(const gd_split_consts &Z, const gd_lds_f32 *pb)
 {
-  const int lane = threadIdx.x & (GD_WAVE - 1);
-  float xyz[6];
-#pragma unroll
-  for (int k = 0; k < 6; ++k)
-    xyz[k] = pb[k * GD_WAVE + lane];
-  gd_energy_items(P, smem, A, prt, Z, xyz[0], xyz[1], xyz[2], xyz[3], xyz[4], xyz[5]);
+  const float cen[3] = {pb[GD_PB_CEN + 0], pb[GD_PB_CEN + 1], pb[GD_PB_CEN + 2]};
+  return gd_edst(Z.pocket_center, cen);
 }
 
-/* n_steps MC steps from step s0 of replica r on the SPLIT wavefronts of the
- * workgroup, `role` = this wavefront's index.  Per step: wavefront 0 names
- * the pose buffer of the step and clears the item counter; barrier; every
- * wavefront takes items -- wavefront 0 only after placing, in the two other
- * buffers, both poses step s + 1 may start from (the move from the current
- * pose if this one is rejected, from the proposed one if it is accepted:
- * the same draws and arithmetic as placing it after the decision); barrier;
- * the sums; barrier; wavefront 0 adds the terms up, decides, and takes the
- * buffer that the decision selects.  Wavefront 0 keeps the state, the
- * decisions and the records.  One code path for every role (the item and
- * sum code is shared, not repeated per role). */
-template <int SPLIT>
-__device__ __forceinline__ void gd_replica_cycle_split(const gd_pack &P, const char *smem,
-                                                       gd_lds_f32 *ws, gd_lds_f32 *A,
-                                                       int role, int r, int prt, int s0,
-                                                       int n_steps)
+/* The draws of n <= GD_SPLIT_DRAWS steps from step s0 of replica r (gd_draws),
+ * one Philox sequence for all: lane 2 i + h takes call h of step s0 + i. */
+__device__ __forceinline__ void gd_split_draws(const gd_pack &P, gd_lds_f32 *out, int r, int s0)
 {
   const int lane = threadIdx.x & (GD_WAVE - 1);
-  gd_lds_f32 *pose = A + GD_SA_POSE;
-  const gd_split_sizes Z = gd_split_sizes_of(P);
-  const bool lead = role == 0;
+  const int h = lane & 1;
+  const gd_u32x4 u = gd_philox4x32_10((uint32_t) r, (uint32_t) (s0 + (lane >> 1)),
+                                      h ? GD_CTR_MOVE_B : GD_CTR_MOVE_A, 0u, P.seed, P.cid);
+  const int fx = P.fixed_draws;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const float sc = h ? P.move_scale[k < 2 ? 4 + k : 0] : P.move_scale[k];
+    const float d = sc * gd_perturbation(fx, u.v[k]);
+    out[lane * 4 + k] = h && k >= 2 ? gd_u01(u.v[k]) : d;
+  }
+}
+static_assert(GD_SPLIT_DRAWS * 2 == GD_WAVE, "one lane per draw call");
 
+/* n_steps MC steps from step s0 of the Z.share replicas r0, r0 + 1, .. on the
+ * SPLIT wavefronts of the workgroup, `role` = this wavefront's index.
+ * Two wavefronts lead replica j, and the first of them keeps its state.  Per step: the wavefronts take items; barrier; the
+ * sums; barrier; the keepers take the decisions; barrier.  The move of step s + 1 never waits for
+ * the decision: among their items the two leaders place both poses that step
+ * may start from, in the replica's two other buffers (the move from the
+ * current pose if this one is rejected, from the proposed one if it is
+ * accepted: the same draws and arithmetic as placing it after the decision),
+ * and the decision only selects the buffer; the state, the best pose and the
+ * records follow behind the barrier, while the others already take items. */
+template <int SPLIT>
+__device__ __forceinline__ void gd_replica_cycle_split(const gd_pack &P, const char *smem,
+                                                       gd_lds_f32 *areas, gd_lds_i32 *ctr,
+                                                       int role, int r0, int s0, int n_steps,
+                                                       const gd_split_consts &Z)
+{
+  const int lane = threadIdx.x & (GD_WAVE - 1);
   const gd_state S = P.S;
-  float e_old_total = 0.0f, best_total = 0.0f, mb = 0.0f;
-  int itmp = 0, acs = 0, cur = 0;
-  gd_lds_f32 *conf = A + GD_SA_CONF;
-  float d[6], u_acc[2] = {0.0f, 0.0f};
-  gd_final_consts F;
-  const uint32_t seed = P.seed, cid = P.cid;
-  if (lead) {
+  const int share = Z.share;
+  /* Each wavefront begins with the item of its own index, unasked.  Where the
+   * others cover the atom blocks, the leaders place their poses first and are
+   * the last wavefronts, since a SIMD issues its oldest first and the blocks
+   * last longest; else they are the oldest, take a block like the others and
+   * place the poses behind it. */
+  const bool place_late = Z.nb * share > SPLIT - 2 * share;
+  const int q = place_late ? role : SPLIT - 1 - role;
+  const int j_lead = q >> 1;
+  const bool lead = j_lead < share;
+  const bool keeper = lead && (q & 1) == 0;
+  const int n_first = place_late ? SPLIT : SPLIT - 2 * share;
+  gd_lds_f32 *A = areas + (lead ? j_lead : 0) * GD_SA_FLOATS;
+  gd_lds_f32 *ws = A;
+  gd_lds_f32 *pose = A + GD_SA_POSE;
+  const int r = r0 + (lead ? j_lead : 0);
+  const float4 *conf = P.lig_xyz + (size_t) gd_uload(P.rep_lig + r) * Z.H.lna;
+  float e_old = 0.0f, best_total = 0.0f, mb = 0.0f;
+  int acs = 0, itmp = 0;
+  float w[GD_F_NTERM];
+#pragma unroll
+  for (int k = 0; k < GD_F_NTERM; ++k)
+    w[k] = P.w[k];
+  if (keeper) {
     gd_slot_load(P, ws, r);
-    __builtin_amdgcn_wave_barrier();
-    e_old_total = S.e[r * 10 + GD_E_TOTAL];
+    e_old = S.e[r * 10 + GD_E_TOTAL];
     best_total = S.e_best[r * 10 + GD_E_TOTAL];
     itmp = S.idx_tmp[r];
     mb = P.minus_beta[itmp];
-    F = gd_final_consts_of(P);
-    {
-      float bx0, by0, bz0, bx1, by1, bz1;
-      gd_load_conformer(P, gd_uload(P.rep_lig + r), &bx0, &by0, &bz0, &bx1, &by1, &bz1);
-      conf[0 * GD_WAVE + lane] = bx0;
-      conf[1 * GD_WAVE + lane] = by0;
-      conf[2 * GD_WAVE + lane] = bz0;
-      conf[3 * GD_WAVE + lane] = bx1;
-      conf[4 * GD_WAVE + lane] = by1;
-      conf[5 * GD_WAVE + lane] = bz1;
-    }
-    /* the pose of the first step, in buffer 0 */
-    float m[6];
-    gd_draws(P, r, s0, seed, cid, d, u_acc);
-#pragma unroll
-    for (int k = 0; k < 6; ++k)
-      m[k] = d[k] + ws[GD_WS_MOLD + k];
-    gd_pose_put(P, pose, m, conf);
-    __builtin_amdgcn_wave_barrier();
   }
+  /* slots that no item writes count as +0 in the sums */
+  for (int j = 0; j < share; ++j)
+    for (int i = GD_SA_PART + (int) threadIdx.x; i < GD_SA_POSE; i += GD_WAVE * SPLIT)
+      areas[j * GD_SA_FLOATS + i] = 0.0f;
 
-  for (int s = s0; s < s0 + n_steps; ++s) {
-    if (lead) {
-      const gd_lds_f32 *pc = pose + cur * GD_PB_FLOATS;
-      if (P.rec != nullptr && s % P.rec_stride == 0)
-        gd_record(P, ws, r, itmp, s);
-      if (lane == 0) {
-        *(gd_lds_i32 *) (A + GD_SA_CTR) = 0;
-        *(gd_lds_i32 *) (A + GD_SA_SEL) = cur;
-#pragma unroll
-        for (int k = 0; k < 6; ++k)
-          ws[GD_WS_MNEW + k] = pc[GD_PB_M + k];
-      }
-    }
-    __syncthreads();
-    const int sel = __builtin_amdgcn_readfirstlane(*(const gd_lds_i32 *) (A + GD_SA_SEL));
-    const gd_lds_f32 *pc = pose + sel * GD_PB_FLOATS;
-
-    /* wavefront 0: both poses of step s + 1, buffer ia if this move is
-     * rejected, ib if it is accepted */
-    const int ia = sel == 2 ? 0 : sel + 1;
-    const int ib = ia == 2 ? 0 : ia + 1;
-    float u_next[2] = {0.0f, 0.0f}, edst = 0.0f;
-    if (lead) {
-      if (s + 1 < s0 + n_steps) {
-        gd_draws(P, r, s + 1, seed, cid, d, u_next);
-        float ma[6], mbv[6];
-#pragma unroll
-        for (int k = 0; k < 6; ++k) {
-          ma[k] = d[k] + ws[GD_WS_MOLD + k];
-          mbv[k] = d[k] + pc[GD_PB_M + k];
-        }
-        gd_pose_put(P, pose + ia * GD_PB_FLOATS, ma, conf);
-        gd_pose_put(P, pose + ib * GD_PB_FLOATS, mbv, conf);
-      }
-      float cen[3];
-#pragma unroll
-      for (int k = 0; k < 3; ++k)
-        cen[k] = pc[GD_PB_CEN + k];
-      edst = gd_edst(P, cen);
-    }
-    gd_pose_items(P, smem, A, pc, prt, Z);
-    __syncthreads();
-    gd_energy_sums(A, role, SPLIT, Z);
-    __syncthreads();
-    if (lead) {
-      float e_new[GD_E_N], cm_new;
-      gd_energy_combine(P, A, F, edst, e_new, &cm_new);
-      const int took = gd_accept(P, ws, r, s, u_acc, mb, e_new, cm_new, &e_old_total,
-                                 &best_total);
-      acs += took;
-      cur = took ? ib : ia;
-      u_acc[0] = u_next[0];
-      u_acc[1] = u_next[1];
+  for (int c0 = s0; c0 < s0 + n_steps; c0 += GD_SPLIT_DRAWS) {
+    const int c1 = min(c0 + GD_SPLIT_DRAWS, s0 + n_steps);
+    /* the draws of these steps and the pose of the first, in buffer 0 */
+    if (keeper) {
+      gd_split_draws(P, A + GD_SA_DRAW, r, c0);
       __builtin_amdgcn_wave_barrier();
+      const int k = lane < 6 ? lane : 0;
+      gd_pose_put(Z, pose, A[GD_SA_DRAW + k] + ws[GD_WS_MOLD + k], conf);
+    }
+    if (role == 0 && lane == 0) {
+      ctr[0] = n_first * GD_WAVE;
+      ctr[1] = n_first * GD_WAVE;
+    }
+    int sel_l = 0;   /* lane j: the pose buffer of replica j */
+    __syncthreads();
+
+    for (int s = c0; s < c1; ++s) {
+      const int par = (s - c0) & 1;
+      const int k = lane < 6 ? lane : 0;
+      const int sel = __builtin_amdgcn_readlane(sel_l, lead ? j_lead : 0);
+      const gd_lds_f32 *pc = pose + sel * GD_PB_FLOATS;
+      float m_l = 0.0f;   /* keeper: the movematrix being evaluated */
+      gd_split_items(smem, areas, ctr + par, Z, sel_l, lead && !place_late ? -1 : role,
+                     place_late, [&]() {
+                       if (!lead)
+                         return;
+                       const int ia = sel == 2 ? 0 : sel + 1;
+                       const int ib = ia == 2 ? 0 : ia + 1;
+                       m_l = pc[GD_PB_M + k];
+                       if (keeper) {
+                         if (P.rec != nullptr && s % P.rec_stride == 0)
+                           gd_record(P, ws, r, itmp, s);
+                         gd_term_put(Z, A + GD_SA_TERM, GD_F_DST, gd_pose_edst(Z, pc));
+                       }
+                       if (s + 1 < c1)
+                         gd_pose_put(Z, pose + (keeper ? ia : ib) * GD_PB_FLOATS,
+                                     A[GD_SA_DRAW + (s + 1 - c0) * 8 + k] +
+                                         (keeper ? ws[GD_WS_MOLD + k] : m_l),
+                                     conf);
+                     });
+      __syncthreads();
+      gd_split_sums(areas, role, SPLIT, Z);
+      if (role == 0 && lane == 0)
+        ctr[par ^ 1] = n_first * GD_WAVE;   /* last used before the barrier above */
+      __syncthreads();
+      int took = 0;
+      float total = 0.0f;
+      if (keeper) {
+        const gd_lds_f32 *term = A + GD_SA_TERM;
+        const gd_lds_f32 *u = A + GD_SA_DRAW + (s - c0) * 8 + 6;
+        total = Z.combine ? gd_split_bayes(Z, term) : gd_split_total(term, w);
+        took = gd_metropolis(total, e_old, mb, u[0], u[1], Z.fixed_draws, Z.reverse);
+        int next = sel + (took ? 2 : 1);
+        next = next >= 3 ? next - 3 : next;
+        *(gd_lds_i32 *) (A + GD_SA_SEL) = next;
+      }
+      __syncthreads();
+      sel_l = *(const gd_lds_i32 *) (areas + (lane < share ? lane : 0) * GD_SA_FLOATS +
+                                     GD_SA_SEL);
+      if (took) {   /* (the terms and counts are next written behind two barriers
+                       that this wavefront takes part in) */
+        ++acs;
+        e_old = total;
+        const float e_l = gd_split_energy(Z, A + GD_SA_TERM, total);
+        const float cm = gd_split_mcc(Z, A);
+        if (lane < GD_E_N)
+          ws[GD_WS_EOLD + lane] = e_l;
+        if (lane < 6)
+          ws[GD_WS_MOLD + lane] = m_l;
+        if (lane == 0)
+          ws[GD_WS_CMCC] = cm;
+        if (total < best_total) {
+          best_total = total;
+          if (lane < 6)
+            S.mv_best[r * 8 + lane] = m_l;
+          if (lane < GD_E_N)
+            S.e_best[r * 10 + lane] = e_l;
+          if (lane == 0) {
+            S.cmcc_best[r] = cm;
+            S.step_best[r] = s;
+          }
+        }
+        __builtin_amdgcn_wave_barrier();
+      }
     }
   }
-  if (lead)
+  if (keeper)
     gd_slot_store(P, ws, r, acs);
 }
 
@@ -1356,7 +1577,7 @@ gd_mc_kernel(const gd_pack *__restrict__ packs, const gd_task *__restrict__ task
     const gd_pack &P = packs[task.cx];
     int s0 = 0, n_steps = 0;
     if (mode == 0) {
-      s0 = P.step[0];
+      s0 = __builtin_amdgcn_readfirstlane(P.step[0]);
       n_steps = gd_cycle_steps(P, s0);
     }
     if (mode != 0 || n_steps > 0) {
@@ -1369,10 +1590,11 @@ gd_mc_kernel(const gd_pack *__restrict__ packs, const gd_task *__restrict__ task
       }
       if (w < task.r_count) {
         const int r = task.r_begin + w;
+        const gd_hot H = gd_hot_of(P, task.prt);
         if (mode == 0)
-          gd_replica_cycle(P, smem, ws, r, task.prt, s0, n_steps);
+          gd_replica_cycle(P, H, smem, ws, r, s0, n_steps);
         else
-          gd_replica_init(P, smem, r);
+          gd_replica_init(P, H, smem, r);
       }
     }
     if (!queue)
@@ -1380,22 +1602,22 @@ gd_mc_kernel(const gd_pack *__restrict__ packs, const gd_task *__restrict__ task
   }
 }
 
-/* MC cycle with SPLIT wavefronts per replica and one replica per workgroup
- * (tasks of one replica), grid form or persistent as gd_mc_kernel: for
- * launches with fewer replicas than the device has SIMDs, where one
- * wavefront per replica leaves most of the device idle and every step
- * waits on its own latency. */
+/* MC cycle with SPLIT wavefronts per workgroup and the task's one to four
+ * replicas sharing them, grid form or persistent as gd_mc_kernel: for launches
+ * with too few replicas to give every SIMD several, where one wavefront per
+ * replica leaves most of the device idle and every step waits on its own
+ * latency. */
 template <int SPLIT>
 __global__ void __launch_bounds__(GD_WAVE *SPLIT)
 gd_mc_split_kernel(const gd_pack *__restrict__ packs, const gd_task *__restrict__ tasks,
-                   int n_tasks, int *queue, int wslot_off, int prio)
+                   int n_tasks, int *queue, int area_off, int prio)
 {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   gd_set_prio(prio);
   __shared__ int s_task;
+  __shared__ int s_ctr[2];
   const int role = __builtin_amdgcn_readfirstlane(threadIdx.x / GD_WAVE);
-  gd_lds_f32 *ws = (gd_lds_f32 *) (smem + wslot_off);
-  gd_lds_f32 *A = ws + GD_WSLOT_FLOATS;
+  gd_lds_f32 *areas = (gd_lds_f32 *) (smem + area_off);
   int staged_cx = -1, staged_prt = -1;
   int t = queue ? -1 : (int) blockIdx.x;
 
@@ -1413,18 +1635,19 @@ gd_mc_split_kernel(const gd_pack *__restrict__ packs, const gd_task *__restrict_
       break;
     const gd_task task = tasks[t];
     const gd_pack &P = packs[task.cx];
-    const int s0 = P.step[0];
+    const int s0 = __builtin_amdgcn_readfirstlane(P.step[0]);
     const int n_steps = gd_cycle_steps(P, s0);
     if (n_steps > 0) {
       if (task.cx != staged_cx || task.prt != staged_prt) {
         __syncthreads();
         gd_stage(P, task.prt, smem);
-        __syncthreads();
         staged_cx = task.cx;
         staged_prt = task.prt;
       }
-      gd_replica_cycle_split<SPLIT>(P, smem, ws, A, role, task.r_begin, task.prt, s0,
-                                        n_steps);
+      /* (the cycle's first barrier covers the staging) */
+      gd_replica_cycle_split<SPLIT>(P, smem, areas, (gd_lds_i32 *) s_ctr, role, task.r_begin,
+                                    s0, n_steps,
+                                    gd_split_consts_of(P, task.prt, task.r_count));
     }
     if (!queue)
       t = -2;
@@ -1459,7 +1682,7 @@ gd_score_kernel(const gd_pack *__restrict__ packs, const gd_task *__restrict__ t
   float ax0, ay0, az0, ax1, ay1, az1, cen[3], e[GD_E_N];
   gd_place(P, m, bx0, by0, bz0, bx1, by1, bz1, &ax0, &ay0, &az0, &ax1, &ay1, &az1, cen);
   float cm;
-  gd_energy_wave(P, smem, task.prt, ax0, ay0, az0, ax1, ay1, az1, cen, e, &cm);
+  gd_energy_wave(P, gd_hot_of(P, task.prt), smem, ax0, ay0, az0, ax1, ay1, az1, cen, e, &cm);
   if (lane == 0) {
 #pragma unroll
     for (int k = 0; k < GD_E_N; ++k)
@@ -1504,7 +1727,7 @@ static hipError_t launch_split(const gd_launch_cfg &C, const gd_pack *packs,
                                const gd_task *tasks, int n_tasks, int *queue, int grid,
                                hipStream_t st)
 {
-  const int lds = C.stage_bytes + GD_SPLIT_LDS_BYTES - 64;
+  const int lds = C.stage_bytes + GD_SPLIT_LDS_BYTES(C.share) - GD_SPLIT_ROOM;
   hipLaunchKernelGGL(gd_mc_split_kernel<SPLIT>, dim3(grid), dim3(GD_WAVE * SPLIT), lds, st,
                      packs, tasks, n_tasks, queue, C.stage_bytes, C.prio);
   return hipGetLastError();
@@ -1586,7 +1809,7 @@ static hipError_t set_attr_wpg(int bytes)
 template <int SPLIT>
 static hipError_t set_attr_split(int bytes)
 {
-  /* at most the device's LDS, less the 64 bytes of room: a complex whose
+  /* at most the device's LDS, less the room: a complex whose
    * staging and split area exceed it does not run split (the engine checks
    * the same sum), but others in the engine may */
   int dev = 0, max_lds = 0;
@@ -1595,10 +1818,10 @@ static hipError_t set_attr_split(int bytes)
     e = hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
   if (e != hipSuccess)
     return e;
-  const int want = bytes + GD_SPLIT_LDS_BYTES;
+  const int want = bytes + GD_SPLIT_LDS_BYTES(GD_SPLIT_MAX_SHARE);
   return hipFuncSetAttribute((const void *) gd_mc_split_kernel<SPLIT>,
                              hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (want < max_lds ? want : max_lds) - 64);
+                             (want < max_lds ? want : max_lds) - GD_SPLIT_ROOM);
 }
 
 hipError_t gd_set_kernel_attrs(int stage_bytes)
@@ -1633,19 +1856,19 @@ static hipError_t occ_wpg(int occ, int stage_bytes, int *blocks)
 }
 
 template <int SPLIT>
-static hipError_t occ_split(int stage_bytes, int *blocks)
+static hipError_t occ_split(int share, int stage_bytes, int *blocks)
 {
   return hipOccupancyMaxActiveBlocksPerMultiprocessor(
       blocks, gd_mc_split_kernel<SPLIT>, GD_WAVE * SPLIT,
-      stage_bytes + GD_SPLIT_LDS_BYTES - 64);
+      stage_bytes + GD_SPLIT_LDS_BYTES(share) - GD_SPLIT_ROOM);
 }
 
 hipError_t gd_mc_occupancy(const gd_launch_cfg &C, int stage_bytes, int *blocks_per_cu)
 {
   switch (C.split) {
-  case 4: return occ_split<4>(stage_bytes, blocks_per_cu);
-  case 8: return occ_split<8>(stage_bytes, blocks_per_cu);
-  case 16: return occ_split<16>(stage_bytes, blocks_per_cu);
+  case 4: return occ_split<4>(C.share, stage_bytes, blocks_per_cu);
+  case 8: return occ_split<8>(C.share, stage_bytes, blocks_per_cu);
+  case 16: return occ_split<16>(C.share, stage_bytes, blocks_per_cu);
   default: break;
   }
   switch (C.wpg) {

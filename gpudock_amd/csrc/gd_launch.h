@@ -13,8 +13,9 @@ typedef struct gd_launch_cfg {
   int stage_bytes;  /* dynamic LDS for staging: max over resident complexes */
   int persistent;   /* 1: grid of resident workgroups pulling from a queue */
   int occ;          /* register budget for waves per SIMD: 0 (compiler), 6 or 8 */
-  int split;        /* wavefronts per replica in MC cycles: 1, or 4, 8, 16 with one
-                       replica per workgroup (tasks of one replica) */
+  int split;        /* MC cycles: 1 = one wavefront per replica, or wavefronts (4, 8,
+                       16) of a workgroup that its task's replicas share */
+  int share;        /* most replicas of a split task (<= split / 2, <= 4) */
   int prio;         /* issue priority of the MC launches' wavefronts in their SIMD
                        against other launches' (s_setprio 0-3) */
 } gd_launch_cfg;

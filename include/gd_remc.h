@@ -397,11 +397,13 @@ typedef struct gd_engine_config {
   int occ;             /* MC kernel register budget: 0 (compiler's choice),
                           6 or 8 waves per SIMD */
   int split;           /* wavefronts per replica in the MC cycles: 0 = chosen
-                          for each resident complex (16 or 8 where one
+                          for each resident complex (several where one
                           wavefront per replica would leave a SIMD fewer than
                           four: few replicas, or tables that fill a CU's
-                          LDS), 1 = one, or 4, 8, 16 (one replica per
-                          workgroup); the energies are the same bits for
+                          LDS), 1 = one, or 4, 8, 16: workgroups of 16
+                          wavefronts that 16 / split replicas share, or where
+                          their LDS areas do not fit, of `split` with one; the
+                          energies are the same bits for
                           every choice.  A complex with more than 64 position
                           restraints, or whose staged tables leave no room in
                           LDS for the split area, has one wavefront per
@@ -434,7 +436,8 @@ typedef struct gd_engine_layout_info {
   int n_classes;       /* MC launches per cycle (occupancy classes) */
   int kde_global;      /* 1: KDE points read from HBM for every complex */
   int occ;             /* MC kernel register budget (waves per SIMD, 0 = default) */
-  int split;           /* most wavefronts per replica of a resident complex */
+  int split;           /* most wavefronts per replica of a resident complex (16
+                          for one to four replicas: 16, 8, 5, 4) */
 } gd_engine_layout_info;
 
 int gd_engine_create(const gd_engine_config *cfg, gd_engine **out);
