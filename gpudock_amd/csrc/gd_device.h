@@ -192,6 +192,8 @@ typedef struct gd_chain {
  * position restraints than GD_SPLIT_MAX_POS run one wavefront per replica. */
 #define GD_SPLIT_MAX_POS 64
 #define GD_SPLIT_DRAWS 32
+/* wavefronts of a workgroup that evaluates single poses */
+#define GD_POSE_SPLIT 16
 /* most replicas that share a split workgroup */
 #define GD_SPLIT_MAX_SHARE 4
 #define GD_SA_PART GD_WSLOT_FLOATS

@@ -217,15 +217,36 @@ int gd_engine::stage_of(const GdImage &I) const
   return std::max(16, kde_global && I.P.kde_in_lds ? I.P.off_kde : I.P.lds_bytes);
 }
 
-int gd_engine::max_share(const GdImage &I) const
+/* Most replicas whose areas fit beside `stage` bytes of tables. */
+static int max_share(const GdImage &I, int stage, int max_lds)
 {
   if (I.P.pos > GD_SPLIT_MAX_POS)
     return 0;
-  const int room = max_lds - stage_of(I) - GD_SPLIT_LDS_BYTES(0);
+  const int room = max_lds - stage - GD_SPLIT_LDS_BYTES(0);
   return std::max(0, std::min(GD_SPLIT_MAX_SHARE, room / GD_SPLIT_AREA_BYTES));
 }
 
-bool gd_engine::can_split(const GdImage &I) const { return max_share(I) > 0; }
+/* How many of n replicas share a workgroup, at most `most`: the fewest
+ * rounds x (share + 1) (split_of). */
+static int pick_share(long long n, int most, int n_cu)
+{
+  int best = 1;
+  long long best_cost = 0;
+  for (int share = 1; share <= most; ++share) {
+    const long long per_round = (long long) share * n_cu;
+    const long long cost = (n + per_round - 1) / per_round * (share + 1);
+    if (share == 1 || cost < best_cost) {
+      best_cost = cost;
+      best = share;
+    }
+  }
+  return best;
+}
+
+bool gd_engine::can_split(const GdImage &I) const
+{
+  return max_share(I, stage_of(I), max_lds) > 0;
+}
 
 /* The workgroups of one of the resident complexes, n_rep replicas in all.
  * A wavefront alone issues an instruction every 6-8 cycles and a SIMD one
@@ -243,7 +264,8 @@ bool gd_engine::can_split(const GdImage &I) const { return max_share(I) > 0; }
  * wavefronts a SIMD) 2.2 ms, split 2.3 ms. */
 gd_engine::Split gd_engine::split_of(const GdImage &I, long long n_rep) const
 {
-  const int most = max_share(I);
+  const int stage = stage_of(I);
+  const int most = max_share(I, stage, max_lds);
   if (most < 1 || lc.split == 1)
     return {1, 1};
   if (lc.split > 1) {
@@ -252,22 +274,11 @@ gd_engine::Split gd_engine::split_of(const GdImage &I, long long n_rep) const
     const int share = 16 / lc.split;
     return share <= most ? Split{16, share} : Split{lc.split, 1};
   }
-  const int stage = stage_of(I);
   const int groups = std::min(max_lds / (stage + lc.wpg * GD_WSLOT_FLOATS * 4), 20 / lc.wpg);
   const long long waves = std::min<long long>(std::max(groups, 1) * lc.wpg, n_rep / n_cu);
   if (waves >= 14)
     return {1, 1};
-  Split best{16, 1};
-  long long best_cost = 0;
-  for (int share = 1; share <= most; ++share) {
-    const long long per_round = (long long) share * n_cu;
-    const long long cost = (n_rep + per_round - 1) / per_round * (share + 1);
-    if (share == 1 || cost < best_cost) {
-      best_cost = cost;
-      best.share = share;
-    }
-  }
-  return best;
+  return {16, pick_share(n_rep, most, n_cu)};
 }
 
 long long gd_engine::replicas() const
@@ -405,40 +416,61 @@ int gd_engine::rebuild()
   n_tasks = (int) sorted.size();
   n_chain = (int) chains.size();
   /* initial energies of newly admitted complexes (MonteCarlo_Init_d,
-   * montecarlo_d.cu:12-55): one grid launch over their tasks, queued before
-   * the first cycle that includes them */
-  std::vector<gd_task> init_tasks;
-  int init_stage = 16;
+   * montecarlo_d.cu:12-55): a grid launch over the tasks of those whose
+   * replicas run whole and one over those that are split, queued before the
+   * first cycle that includes them */
+  std::vector<gd_task> init_tasks, init_split;
+  int init_stage = 16, init_split_stage = 16, init_share = 1;
   for (int h : pending_init) {
     GdSlot *s = find(h);
     if (!s)
       continue;
-    gd_complex_tasks(*s->img, s->cx_index, lc.wpg, init_tasks);
-    init_stage = std::max(init_stage, packs[s->cx_index].lds_bytes);
+    const Split sp = split_of(*s->img, n_rep);
+    const int stage = packs[s->cx_index].lds_bytes;
+    if (sp.waves > 1 && max_share(*s->img, std::max(stage, init_split_stage), max_lds) >=
+                            std::max(sp.share, init_share)) {
+      gd_complex_tasks(*s->img, s->cx_index, sp.share, init_split);
+      init_split_stage = std::max(init_split_stage, stage);
+      init_share = std::max(init_share, sp.share);
+    } else {
+      gd_complex_tasks(*s->img, s->cx_index, lc.wpg, init_tasks);
+      init_stage = std::max(init_stage, stage);
+    }
   }
   pending_init.clear();
   lc.stage_bytes = max_stage;
-  GD_HIP_TRY(gd_set_kernel_attrs(std::max(max_stage, init_stage)));
-  if (!init_tasks.empty()) {
-    const size_t tb = GdArena::round(vbytes(init_tasks));
+  GD_HIP_TRY(gd_set_kernel_attrs(std::max({max_stage, init_stage, init_split_stage})));
+  auto start = [&](const std::vector<gd_task> &list, bool split) -> int {
+    if (list.empty())
+      return GD_OK;
+    const size_t tb = GdArena::round(vbytes(list));
     const size_t toff = arena_take(*this, tb, true);
     if (toff == (size_t) -1)
       return gd_fail(GD_ERR_NOMEM, "arena too small for the initial-energy tasks");
-    rc = upload(arena.base() + toff, init_tasks.data(), vbytes(init_tasks));
-    gd_launch_cfg ic = lc;
-    ic.persistent = 0;
-    ic.split = 1;
-    ic.stage_bytes = init_stage;
-    hipError_t he = rc ? hipSuccess
-                       : gd_launch_mc(ic, (const gd_pack *) (arena.base() + packs_off),
-                                      (const gd_task *) (arena.base() + toff),
-                                      (int) init_tasks.size(), nullptr,
-                                      (int) init_tasks.size(), 1, stream);
+    int rc2 = upload(arena.base() + toff, list.data(), vbytes(list));
+    const gd_pack *pd = (const gd_pack *) (arena.base() + packs_off);
+    const gd_task *td = (const gd_task *) (arena.base() + toff);
+    hipError_t he = hipSuccess;
+    if (!rc2 && split) {
+      he = gd_launch_init_split(pd, td, (int) list.size(), init_split_stage, init_share, stream);
+    } else if (!rc2) {
+      gd_launch_cfg ic = lc;
+      ic.persistent = 0;
+      ic.split = 1;
+      ic.stage_bytes = init_stage;
+      he = gd_launch_mc(ic, pd, td, (int) list.size(), nullptr, (int) list.size(), 1, 1, stream);
+    }
     defer(toff, tb);
-    if (rc)
-      return rc;
+    if (rc2)
+      return rc2;
     GD_HIP_TRY(he);
-  }
+    return GD_OK;
+  };
+  rc = start(init_tasks, false);
+  if (!rc)
+    rc = start(init_split, true);
+  if (rc)
+    return rc;
   dirty = false;
   ++n_rebuilds;
   return GD_OK;
@@ -468,8 +500,8 @@ int gd_engine::resident() const
   return r;
 }
 
-/* MC launches of one cycle, one per occupancy class */
-static hipError_t launch_classes(gd_engine &E, int *queue_base)
+/* MC launches of n_cyc cycles, one per occupancy class */
+static hipError_t launch_classes(gd_engine &E, int *queue_base, int n_cyc = 1)
 {
   const gd_pack *packs = (const gd_pack *) (E.arena.base() + E.packs_off);
   const gd_task *tasks = (const gd_task *) (E.arena.base() + E.tasks_off);
@@ -480,7 +512,7 @@ static hipError_t launch_classes(gd_engine &E, int *queue_base)
     C.share = c.share;
     C.stage_bytes = c.stage;
     hipError_t e = gd_launch_mc(C, packs, tasks + c.off, c.n,
-                                E.lc.persistent ? queue_base + i : nullptr, c.grid, 0,
+                                E.lc.persistent ? queue_base + i : nullptr, c.grid, 0, n_cyc,
                                 E.stream);
     if (e != hipSuccess)
       return e;
@@ -614,6 +646,27 @@ int gd_engine::enqueue_cycle()
   return GD_OK;
 }
 
+/* Cycles that one launch may run of n: all of them, within bounds, while no
+ * resident complex has temperatures to swap between cycles: 100 cycles of 63
+ * replicas of 34 atoms x 344 points at one temperature take 8.1 ms in one
+ * launch, and 9.8 in one a cycle with its staging, advance and gaps.  A launch stays within
+ * 1,000 steps and about 50 ms (4e10 pairs), so that other streams get their
+ * turn. */
+int gd_engine::merged_cycles(int n) const
+{
+  double pairs = 0.0;   /* of one cycle */
+  int spe = 1;
+  for (auto *s : slots) {
+    const gd_pack &P = s->img->P;
+    if (P.exchange && P.n_tmp >= 2)
+      return 1;
+    pairs += (double) P.n_rep * P.lna * P.pnp_pad * P.spe;
+    spe = std::max(spe, P.spe);
+  }
+  const double most = std::min(1000.0 / spe, 4e10 / std::max(pairs, 1.0));
+  return std::max(1, std::min(n, (int) most));
+}
+
 int gd_engine::cycles(int n)
 {
   if (n < 0)
@@ -624,7 +677,8 @@ int gd_engine::cycles(int n)
   if (n_tasks == 0)
     return GD_OK;
   GD_HIP_TRY(hipSetDevice(conf.device));
-  for (int c = 0; c < n; ++c) {
+  for (int c = 0, m = 1; c < n; c += m) {
+    m = timing ? 1 : merged_cycles(n - c);
     if (timing) {
       hipEvent_t a, b, x0, x1;
       GD_HIP_TRY(hipEventCreate(&a));
@@ -641,6 +695,10 @@ int gd_engine::cycles(int n)
       ev_mc.push_back(b);
       ev_x.push_back(x0);
       ev_x.push_back(x1);
+    } else if (m > 1) {
+      GD_HIP_TRY(launch_classes(*this, queue_ptr(), m));
+      GD_HIP_TRY(gd_launch_advance((const gd_pack *) (arena.base() + packs_off), n_cx,
+                                   queue_ptr(), (int) classes.size(), m, stream));
     } else if (conf.use_graph) {
       if (!gexec) {
         GD_HIP_TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
@@ -662,13 +720,13 @@ int gd_engine::cycles(int n)
       if (rc2)
         return rc2;
     }
-    ++n_cycles;
+    n_cycles += m;
     for (auto *s : slots) {
       const int left = s->total_steps - s->steps_done;
-      const int k = left < s->spe ? left : s->spe;
+      const int k = std::min(left, s->spe * m);
       if (k > 0) {
         s->steps_done += k;
-        s->cycles_done += 1;
+        s->cycles_done += k / s->spe;
       }
     }
   }
@@ -681,7 +739,7 @@ int gd_engine::trial_cycle()
 {
   const gd_pack *packs = (const gd_pack *) (arena.base() + packs_off);
   GD_HIP_TRY(launch_classes(*this, queue_ptr()));
-  GD_HIP_TRY(gd_launch_advance(packs, 0, queue_ptr(), (int) classes.size(), stream));
+  GD_HIP_TRY(gd_launch_advance(packs, 0, queue_ptr(), (int) classes.size(), 1, stream));
   return GD_OK;
 }
 
@@ -1581,7 +1639,9 @@ namespace {
 struct ScoreJob {
   GdImage I;
   std::vector<int> order;
-  std::vector<gd_task> tasks;          /* FP32: up to 8 poses each */
+  std::vector<gd_task> tasks;          /* FP32: up to 8 poses, or `share`, each */
+  int share = 0;                       /* > 0: poses split over wavefronts */
+  size_t tasks8 = 0;                   /* tasks of up to 8 poses */
   std::vector<gd_r64_task> tasks64;    /* FP64: up to 8 / split64 poses each */
   int split64 = 1, lds64 = 0, max_lds = 65536;
 };
@@ -1618,10 +1678,11 @@ ScoreLayout score_layout(const ScoreJob &J, int n_pose)
  * and 156 bytes a pose (conformers, order, move, both energies).  The
  * workspace holds GD_SCRATCH_SLACK more than that limit for the FP64 tasks:
  * at most 20 bytes a conformer of at least 1.8 KB of image, and 2.5 a pose
- * against the 4 counted for its protein conformer. */
+ * against the 4 counted for its protein conformer, and for the 16 bytes a
+ * pose of split FP32 tasks, of which there are less than 14 a CU. */
 size_t score_counted(const ScoreJob &J, int n_pose)
 {
-  size_t b = GdArena::round(gd_image_footprint(J.I)) + GdArena::round(vbytes(J.tasks));
+  size_t b = GdArena::round(gd_image_footprint(J.I)) + GdArena::round(J.tasks8 * sizeof(gd_task));
   for (int per : {4, 4, 4, 24, 40, 80})
     b += GdArena::round((size_t) n_pose * per);
   return b;
@@ -1681,8 +1742,14 @@ int score_prepare(const gd_ligand *lig, const gd_protein *prt, const gd_psp *psp
       i = j;
     }
   };
+  J.tasks8 = 0;
+  runs(8, [&](int, int, int) { ++J.tasks8; });
+  /* as split_of: split below 14 wavefronts a CU */
+  const int most = max_share(J.I, J.I.P.lds_bytes, J.max_lds);
+  J.share = most > 0 && n_pose / n_cu < 14 ? pick_share(n_pose, most, n_cu) : 0;
   J.tasks.clear();
-  runs(8, [&](int p, int i, int n) { J.tasks.push_back(gd_task{0, p, i, n}); });
+  runs(J.share ? J.share : 8,
+       [&](int p, int i, int n) { J.tasks.push_back(gd_task{0, p, i, n}); });
   J.tasks64.clear();
   if (energy_fp64 && n_pose > 0) {
     J.split64 = gd_rescore64_split(n_pose, n_cu);
@@ -1719,7 +1786,8 @@ int score_run(char *B, const ScoreLayout &L, ScoreJob &J, int n_pose, const int 
     if (he == hipSuccess)
       he = gd_launch_score(pack_dev, (const gd_task *) (B + L.tasks), (int) J.tasks.size(),
                            (const int *) (B + L.order), (const int *) (B + L.lc),
-                           (const float *) (B + L.mv), J.I.P.lds_bytes, (float *) (B + L.e), st);
+                           (const float *) (B + L.mv), std::max(16, J.I.P.lds_bytes), J.share,
+                           (float *) (B + L.e), st);
   }
   if (he == hipSuccess && energy_fp64)
     he = gd_launch_rescore64(pack_dev, (const gd_r64_task *) (B + L.tasks64),

@@ -184,6 +184,7 @@ private:
   int upload(char *dev, const void *src, size_t bytes);
   int upload_image(GdImage &I, size_t off, GdBlock &b);
   int enqueue_cycle();
+  int merged_cycles(int n) const;
   int trial_cycle();
   /* LDS staging bytes of a complex */
   int stage_of(const GdImage &I) const;
@@ -195,7 +196,6 @@ private:
     int waves, share;
     int per_replica() const { return waves / share; }
   };
-  int max_share(const GdImage &I) const;
   Split split_of(const GdImage &I, long long n_rep) const;
   int choose_split() const;
 };

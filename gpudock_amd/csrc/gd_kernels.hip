@@ -14,6 +14,8 @@
  *   gd_advance_kernel  advances each complex's device step counter after a
  *                      cycle and re-arms the work queue.
  *   gd_score_kernel    energies of caller-given poses (FP32).
+ *   gd_pose_split_kernel the same and the initial energies, each pose split
+ *                      over a workgroup's wavefronts (few poses).
  * (FP64 energies: gd_rescore.hip.)
  *
  * Execution model: a workgroup takes a task -- up to WPG replicas of one
@@ -689,12 +691,12 @@ __device__ __forceinline__ void gd_load_conformer(const gd_pack &P, int conf, fl
   gd_load_conformer_at(P.lig_xyz + (size_t) conf * P.lna, P.lna, bx0, by0, bz0, bx1, by1, bz1);
 }
 
-/* Steps of this cycle for a complex: spe while steps are left (steps_run is
- * a whole number of cycles), else 0. */
-__device__ __forceinline__ int gd_cycle_steps(const gd_pack &P, int s0)
+/* Steps of a launch of n_cyc cycles for a complex: spe a cycle while steps
+ * are left (steps_run is a whole number of cycles). */
+__device__ __forceinline__ int gd_launch_steps(const gd_pack &P, int s0, int n_cyc)
 {
-  const int left = P.steps_run - s0;
-  return left < P.spe ? left : P.spe;
+  const int left = P.steps_run - s0, want = P.spe * n_cyc;
+  return left < want ? left : want;
 }
 
 /* ------------------------------------------------------------------------ */
@@ -1395,7 +1397,7 @@ __device__ __forceinline__ void gd_replica_cycle_split(const gd_pack &P, const c
 #define GD_X_WORDS (2 * GD_MAXTMP_DEV)
 
 __device__ __forceinline__ void gd_advance_all(const gd_pack *__restrict__ packs, int n_cx,
-                                               int *queue, int n_queue)
+                                               int *queue, int n_queue, int n_cyc)
 {
   const int n = n_cx > n_queue ? n_cx : n_queue;
   for (int i = threadIdx.x; i < n; i += blockDim.x) {
@@ -1404,10 +1406,10 @@ __device__ __forceinline__ void gd_advance_all(const gd_pack *__restrict__ packs
     if (i < n_cx) {
       const gd_pack &P = packs[i];
       const int s0 = P.step[0];
-      const int k = gd_cycle_steps(P, s0);
+      const int k = gd_launch_steps(P, s0, n_cyc);
       if (k > 0) {
         P.step[0] = s0 + k;
-        P.step[1] = P.step[1] + 1;
+        P.step[1] = P.step[1] + k / P.spe;
       }
     }
   }
@@ -1429,7 +1431,7 @@ __device__ __forceinline__ void gd_exchange_wave(const gd_pack *__restrict__ pac
     const gd_chain ch = chains[g];
     P = &packs[ch.cx];
     n_tmp = P->n_tmp;
-    active = P->exchange && n_tmp >= 2 && gd_cycle_steps(*P, P->step[0]) > 0;
+    active = P->exchange && n_tmp >= 2 && gd_launch_steps(*P, P->step[0], 1) > 0;
     if (active) {
       x = P->step[1];
       c = ch.c;
@@ -1486,7 +1488,7 @@ gd_exchange1_kernel(const gd_pack *__restrict__ packs, const gd_chain *__restric
   const int wv = threadIdx.x / GD_WAVE;
   for (int g0 = 0; g0 < n_chain; g0 += nw)
     gd_exchange_wave(packs, chains, n_chain, g0 + wv, s_x + wv * GD_X_WORDS);
-  gd_advance_all(packs, n_cx, queue, n_queue);
+  gd_advance_all(packs, n_cx, queue, n_queue, 1);
 }
 
 /* Exchange of chains GD_XWAVES per workgroup; the last workgroup to finish
@@ -1505,20 +1507,21 @@ gd_exchange_kernel(const gd_pack *__restrict__ packs, const gd_chain *__restrict
     s_last = atomicAdd(done, 1) == (int) gridDim.x - 1;
   __syncthreads();
   if (s_last) {
-    gd_advance_all(packs, n_cx, queue, n_queue);
+    gd_advance_all(packs, n_cx, queue, n_queue, 1);
     if (threadIdx.x == 0)
       atomicExch(done, 0);
   }
 }
 
-/* After MC (no temperature chains to exchange): step[0] += steps of this
- * cycle, step[1] += 1; threads 0 .. n_queue-1 re-arm the persistent work
+/* After MC (no temperature chains to exchange): step[0] += steps of the
+ * launch, step[1] += its cycles; threads 0 .. n_queue-1 re-arm the persistent work
  * queues. */
 __global__ void __launch_bounds__(256)
-gd_advance_kernel(const gd_pack *__restrict__ packs, int n_cx, int *queue, int n_queue)
+gd_advance_kernel(const gd_pack *__restrict__ packs, int n_cx, int *queue, int n_queue,
+                  int n_cyc)
 {
   if (blockIdx.x == 0)
-    gd_advance_all(packs, n_cx, queue, n_queue);
+    gd_advance_all(packs, n_cx, queue, n_queue, n_cyc);
 }
 
 /* Issue priority of this wavefront in its SIMD (s_setprio takes an
@@ -1537,7 +1540,7 @@ __device__ __forceinline__ void gd_set_prio(int p)
 
 /* ------------------------------------------------------------------------ */
 /* MC kernel                                                                 */
-/* mode 0: one cycle (steps from each complex's device counter)              */
+/* mode 0: n_cyc cycles (steps from each complex's device counter)           */
 /* mode 1: initial energies (44.5 * move_scale displacement if P.away)       */
 /* queue != nullptr: persistent -- tasks are taken from *queue until it      */
 /* passes n_tasks (every workgroup exits once the list is drained).          */
@@ -1549,7 +1552,7 @@ __device__ __forceinline__ void gd_set_prio(int p)
 template <int WPG, int MINW>
 __global__ void __launch_bounds__(GD_WAVE *WPG) __attribute__((amdgpu_waves_per_eu(MINW, 8)))
 gd_mc_kernel(const gd_pack *__restrict__ packs, const gd_task *__restrict__ tasks,
-             int n_tasks, int *queue, int mode, int wslot_off, int prio)
+             int n_tasks, int *queue, int mode, int n_cyc, int wslot_off, int prio)
 {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   gd_set_prio(prio);
@@ -1578,7 +1581,7 @@ gd_mc_kernel(const gd_pack *__restrict__ packs, const gd_task *__restrict__ task
     int s0 = 0, n_steps = 0;
     if (mode == 0) {
       s0 = __builtin_amdgcn_readfirstlane(P.step[0]);
-      n_steps = gd_cycle_steps(P, s0);
+      n_steps = gd_launch_steps(P, s0, n_cyc);
     }
     if (mode != 0 || n_steps > 0) {
       if (task.cx != staged_cx || task.prt != staged_prt) {
@@ -1610,7 +1613,7 @@ gd_mc_kernel(const gd_pack *__restrict__ packs, const gd_task *__restrict__ task
 template <int SPLIT>
 __global__ void __launch_bounds__(GD_WAVE *SPLIT)
 gd_mc_split_kernel(const gd_pack *__restrict__ packs, const gd_task *__restrict__ tasks,
-                   int n_tasks, int *queue, int area_off, int prio)
+                   int n_tasks, int *queue, int n_cyc, int area_off, int prio)
 {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   gd_set_prio(prio);
@@ -1636,7 +1639,7 @@ gd_mc_split_kernel(const gd_pack *__restrict__ packs, const gd_task *__restrict_
     const gd_task task = tasks[t];
     const gd_pack &P = packs[task.cx];
     const int s0 = __builtin_amdgcn_readfirstlane(P.step[0]);
-    const int n_steps = gd_cycle_steps(P, s0);
+    const int n_steps = gd_launch_steps(P, s0, n_cyc);
     if (n_steps > 0) {
       if (task.cx != staged_cx || task.prt != staged_prt) {
         __syncthreads();
@@ -1690,66 +1693,162 @@ gd_score_kernel(const gd_pack *__restrict__ packs, const gd_task *__restrict__ t
   }
 }
 
+/* The energies of one to four poses a workgroup, each split over its 16
+ * wavefronts as the MC steps are: with energy, of the given poses of the task
+ * (as gd_score_kernel); else the initial energies of its replicas (as
+ * gd_mc_kernel's mode 1).  A wavefront alone waits on its own latency: one
+ * pose of 24 atoms x 300 points 60 us whole | 14 split, 189 of 34 x 344
+ * 99 | 18, 592 replicas of 61 x 1,037 352 | 79. */
+__global__ void __launch_bounds__(GD_WAVE *GD_POSE_SPLIT)
+gd_pose_split_kernel(const gd_pack *__restrict__ packs, const gd_task *__restrict__ tasks,
+                     const int *__restrict__ pose_ids, const int *__restrict__ lig_conf,
+                     const float *__restrict__ move, float *__restrict__ energy, int area_off)
+{
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  __shared__ int s_ctr;
+  const gd_task task = tasks[blockIdx.x];
+  const gd_pack &P = packs[task.cx];
+  const int role = __builtin_amdgcn_readfirstlane(threadIdx.x / GD_WAVE);
+  const int lane = threadIdx.x & (GD_WAVE - 1);
+  gd_lds_f32 *areas = (gd_lds_f32 *) (smem + area_off);
+  const gd_split_consts Z = gd_split_consts_of(P, task.prt, task.r_count);
+  gd_stage(P, task.prt, smem);
+  /* slots that no item writes count as +0 in the sums */
+  for (int j = 0; j < Z.share; ++j)
+    for (int i = GD_SA_PART + (int) threadIdx.x; i < GD_SA_POSE; i += GD_WAVE * GD_POSE_SPLIT)
+      areas[j * GD_SA_FLOATS + i] = 0.0f;
+  if (threadIdx.x == 0)
+    s_ctr = GD_POSE_SPLIT * GD_WAVE;   /* every wavefront begins with its own item */
+
+  /* wavefront j: pose j of the task */
+  const bool lead = role < Z.share;
+  gd_lds_f32 *A = areas + (lead ? role : 0) * GD_SA_FLOATS;
+  const int at = task.r_begin + (lead ? role : 0);
+  const int i = energy ? gd_uload(pose_ids + at) : at;
+  const int k = lane < 6 ? lane : 0;
+  float m_l = 0.0f;
+  if (lead) {
+    if (energy) {
+      m_l = move[i * 6 + k];
+    } else {
+      m_l = P.S.mv[i * 8 + k];
+      if (P.away)
+        m_l = P.move_scale[k] * 44.5f + m_l;
+    }
+    const int conf = gd_uload((energy ? lig_conf : P.rep_lig) + i);
+    gd_pose_put(Z, A + GD_SA_POSE, m_l, P.lig_xyz + (size_t) conf * Z.H.lna);
+    __builtin_amdgcn_wave_barrier();
+    gd_term_put(Z, A + GD_SA_TERM, GD_F_DST, gd_pose_edst(Z, A + GD_SA_POSE));
+  }
+  __syncthreads();
+  gd_split_items(smem, areas, (gd_lds_i32 *) &s_ctr, Z, 0, role, false, []() {});
+  __syncthreads();
+  gd_split_sums(areas, role, GD_POSE_SPLIT, Z);
+  __syncthreads();
+  if (!lead)
+    return;
+  float w[GD_F_NTERM];
+#pragma unroll
+  for (int t = 0; t < GD_F_NTERM; ++t)
+    w[t] = P.w[t];
+  const gd_lds_f32 *term = A + GD_SA_TERM;
+  const float total = Z.combine ? gd_split_bayes(Z, term) : gd_split_total(term, w);
+  const float e_l = gd_split_energy(Z, term, total);
+  if (energy) {
+    if (lane < GD_E_N)
+      energy[i * GD_E_N + lane] = e_l;
+    return;
+  }
+  const gd_state S = P.S;
+  const float cm = gd_split_mcc(Z, A);
+  if (lane < 6) {
+    S.mv[i * 8 + lane] = m_l;
+    S.mv_best[i * 8 + lane] = m_l;
+  }
+  if (lane < GD_E_N) {
+    S.e[i * 10 + lane] = e_l;
+    S.e_best[i * 10 + lane] = e_l;
+  }
+  if (lane == 0) {
+    S.cmcc[i] = cm;
+    S.cmcc_best[i] = cm;
+    S.step_best[i] = -1;
+  }
+}
+
 /* ------------------------------------------------------------------------ */
 /* host-callable launch wrappers                                             */
 /* ------------------------------------------------------------------------ */
 template <int WPG, int MINW>
 static hipError_t launch_mc_var(const gd_pack *packs, const gd_task *tasks, int n_tasks,
-                                int *queue, int grid, int mode, int stage_bytes, int prio,
-                                hipStream_t st)
+                                int *queue, int grid, int mode, int n_cyc, int stage_bytes,
+                                int prio, hipStream_t st)
 {
   const int lds = stage_bytes + WPG * GD_WSLOT_FLOATS * 4;
   hipLaunchKernelGGL((gd_mc_kernel<WPG, MINW>), dim3(grid), dim3(GD_WAVE * WPG), lds, st,
-                     packs, tasks, n_tasks, queue, mode, stage_bytes, prio);
+                     packs, tasks, n_tasks, queue, mode, n_cyc, stage_bytes, prio);
   return hipGetLastError();
 }
 
 template <int WPG>
 static hipError_t launch_mc_wpg(const gd_launch_cfg &C, const gd_pack *packs,
                                 const gd_task *tasks, int n_tasks, int *queue, int grid,
-                                int mode, hipStream_t st)
+                                int mode, int n_cyc, hipStream_t st)
 {
   switch (C.occ) {
   case 6:
-    return launch_mc_var<WPG, 6>(packs, tasks, n_tasks, queue, grid, mode, C.stage_bytes,
-                                 C.prio, st);
+    return launch_mc_var<WPG, 6>(packs, tasks, n_tasks, queue, grid, mode, n_cyc,
+                                 C.stage_bytes, C.prio, st);
   case 8:
-    return launch_mc_var<WPG, 8>(packs, tasks, n_tasks, queue, grid, mode, C.stage_bytes,
-                                 C.prio, st);
+    return launch_mc_var<WPG, 8>(packs, tasks, n_tasks, queue, grid, mode, n_cyc,
+                                 C.stage_bytes, C.prio, st);
   default:
-    return launch_mc_var<WPG, 1>(packs, tasks, n_tasks, queue, grid, mode, C.stage_bytes,
-                                 C.prio, st);
+    return launch_mc_var<WPG, 1>(packs, tasks, n_tasks, queue, grid, mode, n_cyc,
+                                 C.stage_bytes, C.prio, st);
   }
 }
 
 template <int SPLIT>
 static hipError_t launch_split(const gd_launch_cfg &C, const gd_pack *packs,
                                const gd_task *tasks, int n_tasks, int *queue, int grid,
-                               hipStream_t st)
+                               int n_cyc, hipStream_t st)
 {
   const int lds = C.stage_bytes + GD_SPLIT_LDS_BYTES(C.share) - GD_SPLIT_ROOM;
   hipLaunchKernelGGL(gd_mc_split_kernel<SPLIT>, dim3(grid), dim3(GD_WAVE * SPLIT), lds, st,
-                     packs, tasks, n_tasks, queue, C.stage_bytes, C.prio);
+                     packs, tasks, n_tasks, queue, n_cyc, C.stage_bytes, C.prio);
+  return hipGetLastError();
+}
+
+static hipError_t launch_pose_split(const gd_pack *packs, const gd_task *tasks, int n_tasks,
+                                    const int *pose_ids, const int *lig_conf,
+                                    const float *move, int stage_bytes, int share,
+                                    float *energy, hipStream_t st)
+{
+  if (n_tasks <= 0)
+    return hipSuccess;
+  hipLaunchKernelGGL(gd_pose_split_kernel, dim3(n_tasks), dim3(GD_WAVE * GD_POSE_SPLIT),
+                     stage_bytes + GD_SPLIT_LDS_BYTES(share) - GD_SPLIT_ROOM, st, packs, tasks,
+                     pose_ids, lig_conf, move, energy, stage_bytes);
   return hipGetLastError();
 }
 
 hipError_t gd_launch_mc(const gd_launch_cfg &C, const gd_pack *packs, const gd_task *tasks,
-                        int n_tasks, int *queue, int grid, int mode, hipStream_t st)
+                        int n_tasks, int *queue, int grid, int mode, int n_cyc, hipStream_t st)
 {
   if (n_tasks <= 0 || grid <= 0)
     return hipSuccess;
   if (mode == 0 && C.split > 1) {
     switch (C.split) {
-    case 4: return launch_split<4>(C, packs, tasks, n_tasks, queue, grid, st);
-    case 8: return launch_split<8>(C, packs, tasks, n_tasks, queue, grid, st);
-    case 16: return launch_split<16>(C, packs, tasks, n_tasks, queue, grid, st);
+    case 4: return launch_split<4>(C, packs, tasks, n_tasks, queue, grid, n_cyc, st);
+    case 8: return launch_split<8>(C, packs, tasks, n_tasks, queue, grid, n_cyc, st);
+    case 16: return launch_split<16>(C, packs, tasks, n_tasks, queue, grid, n_cyc, st);
     default: return hipErrorInvalidValue;
     }
   }
   switch (C.wpg) {
-  case 4: return launch_mc_wpg<4>(C, packs, tasks, n_tasks, queue, grid, mode, st);
-  case 16: return launch_mc_wpg<16>(C, packs, tasks, n_tasks, queue, grid, mode, st);
-  default: return launch_mc_wpg<8>(C, packs, tasks, n_tasks, queue, grid, mode, st);
+  case 4: return launch_mc_wpg<4>(C, packs, tasks, n_tasks, queue, grid, mode, n_cyc, st);
+  case 16: return launch_mc_wpg<16>(C, packs, tasks, n_tasks, queue, grid, mode, n_cyc, st);
+  default: return launch_mc_wpg<8>(C, packs, tasks, n_tasks, queue, grid, mode, n_cyc, st);
   }
 }
 
@@ -1757,7 +1856,7 @@ hipError_t gd_launch_exchange(const gd_pack *packs, const gd_chain *chains, int 
                               int n_cx, int *queue, int n_queue, int *done, hipStream_t st)
 {
   if (n_chain <= 0)
-    return gd_launch_advance(packs, n_cx, queue, n_queue, st);
+    return gd_launch_advance(packs, n_cx, queue, n_queue, 1, st);
   if (n_chain <= GD_X1_MAX_CHAINS) {
     const int nw = n_chain < GD_X1_WAVES ? n_chain : GD_X1_WAVES;
     hipLaunchKernelGGL(gd_exchange1_kernel, dim3(1), dim3(GD_WAVE * nw), 0, st, packs, chains,
@@ -1771,22 +1870,32 @@ hipError_t gd_launch_exchange(const gd_pack *packs, const gd_chain *chains, int 
 }
 
 hipError_t gd_launch_advance(const gd_pack *packs, int n_cx, int *queue, int n_queue,
-                             hipStream_t st)
+                             int n_cyc, hipStream_t st)
 {
   hipLaunchKernelGGL(gd_advance_kernel, dim3(1), dim3(256), 0, st, packs, n_cx, queue,
-                     n_queue);
+                     n_queue, n_cyc);
   return hipGetLastError();
 }
 
 hipError_t gd_launch_score(const gd_pack *packs, const gd_task *tasks, int n_tasks,
                            const int *pose_ids, const int *lig_conf, const float *move,
-                           int stage_bytes, float *energy, hipStream_t st)
+                           int stage_bytes, int share, float *energy, hipStream_t st)
 {
   if (n_tasks <= 0)
     return hipSuccess;
+  if (share > 0)
+    return launch_pose_split(packs, tasks, n_tasks, pose_ids, lig_conf, move, stage_bytes,
+                             share, energy, st);
   hipLaunchKernelGGL(gd_score_kernel, dim3(n_tasks), dim3(GD_WAVE * 8), stage_bytes, st,
                      packs, tasks, pose_ids, lig_conf, move, energy);
   return hipGetLastError();
+}
+
+hipError_t gd_launch_init_split(const gd_pack *packs, const gd_task *tasks, int n_tasks,
+                                int stage_bytes, int share, hipStream_t st)
+{
+  return launch_pose_split(packs, tasks, n_tasks, nullptr, nullptr, nullptr, stage_bytes,
+                           share, nullptr, st);
 }
 
 template <int WPG, int MINW>
@@ -1806,8 +1915,7 @@ static hipError_t set_attr_wpg(int bytes)
   return e;
 }
 
-template <int SPLIT>
-static hipError_t set_attr_split(int bytes)
+static hipError_t set_attr_split(const void *kernel, int bytes)
 {
   /* at most the device's LDS, less the room: a complex whose
    * staging and split area exceed it does not run split (the engine checks
@@ -1819,16 +1927,16 @@ static hipError_t set_attr_split(int bytes)
   if (e != hipSuccess)
     return e;
   const int want = bytes + GD_SPLIT_LDS_BYTES(GD_SPLIT_MAX_SHARE);
-  return hipFuncSetAttribute((const void *) gd_mc_split_kernel<SPLIT>,
-                             hipFuncAttributeMaxDynamicSharedMemorySize,
+  return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                              (want < max_lds ? want : max_lds) - GD_SPLIT_ROOM);
 }
 
 hipError_t gd_set_kernel_attrs(int stage_bytes)
 {
-  hipError_t e = set_attr_split<4>(stage_bytes);
-  if (e == hipSuccess) e = set_attr_split<8>(stage_bytes);
-  if (e == hipSuccess) e = set_attr_split<16>(stage_bytes);
+  hipError_t e = set_attr_split((const void *) gd_pose_split_kernel, stage_bytes);
+  if (e == hipSuccess) e = set_attr_split((const void *) gd_mc_split_kernel<4>, stage_bytes);
+  if (e == hipSuccess) e = set_attr_split((const void *) gd_mc_split_kernel<8>, stage_bytes);
+  if (e == hipSuccess) e = set_attr_split((const void *) gd_mc_split_kernel<16>, stage_bytes);
   if (e == hipSuccess) e = set_attr_wpg<4>(stage_bytes);
   if (e == hipSuccess) e = set_attr_wpg<8>(stage_bytes);
   if (e == hipSuccess) e = set_attr_wpg<16>(stage_bytes);

@@ -20,20 +20,29 @@ typedef struct gd_launch_cfg {
                        against other launches' (s_setprio 0-3) */
 } gd_launch_cfg;
 
+/* mode 0: n_cyc cycles of MC steps without exchange between them; 1: initial
+ * energies */
 hipError_t gd_launch_mc(const gd_launch_cfg &C, const gd_pack *packs, const gd_task *tasks,
-                        int n_tasks, int *queue, int grid, int mode, hipStream_t st);
+                        int n_tasks, int *queue, int grid, int mode, int n_cyc,
+                        hipStream_t st);
 /* exchange over chains[0 .. n_chain), then the advance of
  * gd_launch_advance: by one workgroup for few chains, else by the last
  * workgroup to finish (*done: a zeroed counter the launch leaves zeroed).
  * With no chains, the advance alone. */
 hipError_t gd_launch_exchange(const gd_pack *packs, const gd_chain *chains, int n_chain,
                               int n_cx, int *queue, int n_queue, int *done, hipStream_t st);
-/* advances the step counters of packs[0 .. n_cx) and zeroes queue[0 .. n_queue) */
+/* advances the step counters of packs[0 .. n_cx) by n_cyc cycles and zeroes
+ * queue[0 .. n_queue) */
 hipError_t gd_launch_advance(const gd_pack *packs, int n_cx, int *queue, int n_queue,
-                             hipStream_t st);
+                             int n_cyc, hipStream_t st);
 hipError_t gd_launch_score(const gd_pack *packs, const gd_task *tasks, int n_tasks,
                            const int *pose_ids, const int *lig_conf, const float *move,
-                           int stage_bytes, float *energy, hipStream_t st);
+                           int stage_bytes, int share, float *energy, hipStream_t st);
+/* initial energies of the tasks' replicas, at most `share` a task, split over
+ * workgroups of GD_POSE_SPLIT wavefronts (gd_launch_score with share > 0: the
+ * same for given poses) */
+hipError_t gd_launch_init_split(const gd_pack *packs, const gd_task *tasks, int n_tasks,
+                                int stage_bytes, int share, hipStream_t st);
 /* blocks x 256 lanes, each 128 x iters FMAs; out holds blocks x 256 floats */
 hipError_t gd_launch_valu_probe(float *out, int blocks, int iters, hipStream_t st);
 /* one kind of gd_valu_probe_kinds (0 .. GD_VALU_KINDS - 1) */
