@@ -11,16 +11,19 @@
  * so a pose's energies have the same bits however many wavefronts share it.
  *
  * What bounds it: FP64 VALU issue (a wavefront instruction takes four
- * cycles of its SIMD).  One pair needs d, 1/d^6, 1/d^9, two quotients and an
- * exponential: from one v_rsq_f64 and one v_rcp_f64, each refined by one
- * third-order step, and a degree-11 exponential, in place of a library sqrt,
- * five divisions and exp.  Two atoms of a slice run through the point loop
- * together: they share the point's LDS reads and conversions, and each hides
- * the other's latency.  Against one wavefront per pose with library math and
- * the tables read through the caches: 16,384 poses of 48 atoms x 800 points
- * 6.12 -> 2.04 ms, 4,096 of 128 x 4,000 18.8 -> 7.7 ms, 592 of 61 x 1,037
- * 662 -> 280 us, one pose of 24 x 300 114 -> 18 us.  The error against
- * 80-bit arithmetic is as before or smaller (1e-16 of the energies' norm).
+ * cycles of its SIMD; about 105 a 64-pair chunk now, 70 % of the issue slots).
+ * One pair needs d, 1/d^6, 1/d^9, two quotients and an exponential: from one
+ * v_rsq_f64 and one v_rcp_f64, each refined by one third-order step, and a
+ * degree-11 exponential, in place of a library sqrt, five divisions and exp.
+ * Two atoms of a slice run through the point loop together: they share the
+ * point's LDS reads and conversions and the loop's branches, and each hides
+ * the other's latency.  One wavefront per pose with library math and the
+ * tables read through the caches | this split, an atom at a time between the
+ * branches, literal coefficients | as it is: 16,384 poses of 48 atoms x 800
+ * points 6.12 | 2.07 | 1.96 ms, 4,096 of them - | 674 | 621 us, 4,096 of 128 x
+ * 4,000 18.8 | 7.71 | 6.89 ms, 592 of 61 x 1,037 662 | 166 | 155 us, one pose of
+ * 24 x 300 114 | 18 | 18 us.  The error against 80-bit arithmetic is as before
+ * or smaller (1e-16 of the energies' norm).
  */
 #include <hip/hip_runtime.h>
 #include "gd_device.h"
@@ -55,23 +58,35 @@ __device__ __forceinline__ double gd_rcp64(double x)
  * is then the low word), r = x - n ln2 in two steps, e^r = 1 + r + r^2 q(r)
  * with q of degree 9 interpolated here at the Chebyshev nodes of
  * |r| <= ln2 / 2 (truncation below 1e-17), scaled by v_ldexp_f64.  Clamped at
- * -700 (1e-304: no sum can tell it from 0). */
-__device__ __forceinline__ double gd_exp64(double x)
+ * -700 (1e-304: no sum can tell it from 0).  The coefficients of r^11 .. r^3
+ * come in scalar registers (gd_exp64_coeffs): as literals each is copied into
+ * the accumulator of its fma first, a fifth of the pair loop's instructions. */
+struct gd_exp64_c {
+  double c[9];
+};
+
+__device__ __forceinline__ gd_exp64_c gd_exp64_coeffs()
+{
+  gd_exp64_c K = {{0x1.af389ecfc4b9cp-26, 0x1.28917c89a43a7p-22, 0x1.71de0db2f6b19p-19,
+                   0x1.a019b9149a41cp-16, 0x1.a01a01a7c2efep-13, 0x1.6c16c17889ef1p-10,
+                   0x1.11111111109b5p-7, 0x1.5555555553d68p-5, 0x1.5555555555556p-3}};
+#pragma unroll
+  for (int k = 0; k < 9; ++k)
+    asm volatile("" : "+s"(K.c[k]));
+  return K;
+}
+
+__device__ __forceinline__ double gd_exp64(double x, const gd_exp64_c &K)
 {
   const double xc = __builtin_fmax(x, -700.0);
   const double t = __builtin_fma(xc, 0x1.71547652b82fep+0, 0x1.8p+52);
   const double n = t - 0x1.8p+52;
   double r = __builtin_fma(-n, 0x1.62e42fefa39efp-1, xc);
   r = __builtin_fma(-n, 0x1.abc9e3b39803fp-56, r);
-  double p = 0x1.af389ecfc4b9cp-26;
-  p = __builtin_fma(p, r, 0x1.28917c89a43a7p-22);
-  p = __builtin_fma(p, r, 0x1.71de0db2f6b19p-19);
-  p = __builtin_fma(p, r, 0x1.a019b9149a41cp-16);
-  p = __builtin_fma(p, r, 0x1.a01a01a7c2efep-13);
-  p = __builtin_fma(p, r, 0x1.6c16c17889ef1p-10);
-  p = __builtin_fma(p, r, 0x1.11111111109b5p-7);
-  p = __builtin_fma(p, r, 0x1.5555555553d68p-5);
-  p = __builtin_fma(p, r, 0x1.5555555555556p-3);
+  double p = K.c[0];
+#pragma unroll
+  for (int k = 1; k < 9; ++k)
+    p = __builtin_fma(p, r, K.c[k]);
   p = __builtin_fma(p, r, 0.5);
   p = __builtin_fma(p, r, 1.0);
   p = __builtin_fma(p, r, 1.0);
@@ -158,6 +173,7 @@ struct gd_r64_consts {
   double el0, a1, b1, el1;     /* g(s) = el0 + a1 s^2 + b1 s^3 below s = el1 d = 1 */
   double inv_el1;
   unsigned near_hi, far_hi;    /* high words of dcut^2 (just above) and of infinity */
+  gd_exp64_c K;
 };
 
 struct gd_r64_acc {
@@ -176,7 +192,7 @@ __device__ __forceinline__ void gd_r64_atoms(const gd_pack &P, const char *smem,
 {
   const int lane = threadIdx.x & (GD_WAVE - 1);
   const int nchunk = P.pnp_pad / GD_WAVE;
-  const int kp = P.chunk_bounds[2 * prt + 1];
+  const int kp = __builtin_amdgcn_readfirstlane(P.chunk_bounds[2 * prt + 1]);
   const float4 *g_pos = P.pt_pos + (size_t) prt * P.pnp_pad;
   const float2 *g_eh = P.pt_eh + (size_t) prt * P.pnp_pad;
   const float *g_psp = P.psp_pt + (size_t) prt * P.n_rows * P.pnp_pad;
@@ -188,6 +204,7 @@ __device__ __forceinline__ void gd_r64_atoms(const gd_pack &P, const char *smem,
     hacc[i] = 0.0;
     any_hdb |= ar[i].hdb;
   }
+  any_hdb = __builtin_amdgcn_readfirstlane(any_hdb);
   for (int k = 0; k < nchunk; ++k) {
     float4 q;
     float2 eh;
@@ -207,57 +224,83 @@ __device__ __forceinline__ void gd_r64_atoms(const gd_pack &P, const char *smem,
       pv[i] = lead ? g_psp[(size_t) ar[i].row * P.pnp_pad + k * GD_WAVE + lane] : 0.0f;
     const double qx = q.x, qy = q.y, qz = q.z, qe = eh.x, qh = eh.y;
     const unsigned bits = __float_as_uint(q.w);
+    /* the atoms side by side, branches shared: the one's chain of dependent
+     * operations fills the other's waits */
+    const char *row[M];
+    float4 tp[M];
+    double d2[M], r1[M], d[M], dl[M], g[M], dm[M];
+    bool out = false;
 #pragma unroll
     for (int i = 0; i < M; ++i) {
-      const char *row = smem + off_tab + ar[i].row * (GD_ROW_STRIDE * (int) sizeof(gd_pair_param));
-      const float4 tp = *(const float4 *) (row + bits);   /* p1a p2a pmf0 pmf1 */
+      row[i] = smem + off_tab + ar[i].row * (GD_ROW_STRIDE * (int) sizeof(gd_pair_param)) + bits;
+      tp[i] = *(const float4 *) row[i];   /* p1a p2a pmf0 pmf1 */
       const double dx = xyz[i][0] - qx, dy = xyz[i][1] - qy, dz = xyz[i][2] - qz;
-      const double d2 = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
-      double r1 = gd_rsqrt64(d2);
-      double d = d2 * r1;
-      double dl = d2;                     /* d^2 of the soft-LJ denominator */
-      double g = r1 * C.inv_el1;
-      /* pairs inside the short range, and the degenerate distances 0 and
-       * infinity, in a branch that a wavefront seldom takes (one unsigned
-       * compare of the high word finds both) */
-      if (__ballot((unsigned) __double2hiint(d2) - C.near_hi >= C.far_hi - C.near_hi)) {
-        asm volatile("");
-        if (d2 == 0.0 || d2 == HUGE_VAL) {
+      d2[i] = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
+      r1[i] = gd_rsqrt64(d2[i]);
+      d[i] = d2[i] * r1[i];
+      dl[i] = d2[i];                      /* d^2 of the soft-LJ denominator */
+      g[i] = r1[i] * C.inv_el1;
+      out |= (unsigned) __double2hiint(d2[i]) - C.near_hi >= C.far_hi - C.near_hi;
+    }
+    /* pairs inside the short range, and the degenerate distances 0 and
+     * infinity, in a branch that a wavefront seldom takes (one unsigned
+     * compare of the high word finds both) */
+    if (__ballot(out)) {
+      asm volatile("");
+#pragma unroll
+      for (int i = 0; i < M; ++i) {
+        if (d2[i] == 0.0 || d2[i] == HUGE_VAL) {
           /* the soft-LJ quotient is inf - inf or 0 inf there; the others
            * are finite */
-          r1 = 0.0;
-          d = d2;
-          dl = 0.0;
-          g = 0.0;
+          r1[i] = 0.0;
+          d[i] = d2[i];
+          dl[i] = 0.0;
+          g[i] = 0.0;
           acc.vdw += __builtin_nan("");
         }
-        const double s = C.el1 * d;
+        const double s = C.el1 * d[i];
         if (s < 1.0)
-          g = __builtin_fma(s * s, __builtin_fma(C.b1, s, C.a1), C.el0);
+          g[i] = __builtin_fma(s * s, __builtin_fma(C.b1, s, C.a1), C.el0);
       }
-      const double r2 = r1 * r1;
-      const double r3 = r2 * r1;
+    }
+#pragma unroll
+    for (int i = 0; i < M; ++i) {
+      const double r2 = r1[i] * r1[i];
+      const double r3 = r2 * r1[i];
       const double r6 = r3 * r3;
-      const double p1 = (double) tp.x * (r6 * r3);
-      const double p2 = (double) tp.y * r6;
-      const double p4 = __builtin_fma(p1, __builtin_fma(C.lj01, dl, C.lj0), 1.0);
-      ele[i] = __builtin_fma(qe, g, ele[i]);
-      const double dm = d - (double) tp.z;
-      const double q1 = 1.0 + gd_exp64(__builtin_fma(-0.5, d, 6.0) * dm);
+      const double p1 = (double) tp[i].x * (r6 * r3);
+      const double p2 = (double) tp[i].y * r6;
+      const double p4 = __builtin_fma(p1, __builtin_fma(C.lj01, dl[i], C.lj0), 1.0);
+      ele[i] = __builtin_fma(qe, g[i], ele[i]);
+      dm[i] = d[i] - (double) tp[i].z;
+      const double q1 = 1.0 + gd_exp64(__builtin_fma(-0.5, d[i], 6.0) * dm[i], C.K);
       const double rr = gd_rcp64(p4 * q1);   /* serves both quotients */
       acc.vdw = __builtin_fma((p1 - p2) * q1, rr, acc.vdw);
-      acc.pmf = __builtin_fma((double) tp.w * p4, rr, acc.pmf);
-      if (lead) {
-        acc.psp += dm <= 0.0 ? (double) pv[i] : 0.0;
+      acc.pmf = __builtin_fma((double) tp[i].w * p4, rr, acc.pmf);
+    }
+    if (lead) {
+#pragma unroll
+      for (int i = 0; i < M; ++i) {
+        acc.psp += dm[i] <= 0.0 ? (double) pv[i] : 0.0;
         /* (1 - u)^3 (1 - u/2) = w^3 (1 + w) / 2, u = d^2 / 81, w = 1 - u */
-        const double w = __builtin_fmax(__builtin_fma(d2, -1.0 / 81.0, 1.0), 0.0);
+        const double w = __builtin_fmax(__builtin_fma(d2[i], -1.0 / 81.0, 1.0), 0.0);
         hacc[i] = __builtin_fma((w * w) * w, __builtin_fma(w, qh, qh), hacc[i]);
       }
-      if (any_hdb) {
-        const float2 hb = *(const float2 *) (row + bits + 16);   /* hdb0 hdb1 */
-        if (hb.x > 0.1f) {
-          const double h = (d - (double) hb.x) * (double) hb.y;
-          acc.hdb = __builtin_fma((double) hb.y, gd_exp64((-0.5 * h) * h), acc.hdb);
+    }
+    if (any_hdb) {
+      float2 hb[M];
+      bool on = false;
+#pragma unroll
+      for (int i = 0; i < M; ++i) {
+        hb[i] = *(const float2 *) (row[i] + 16);   /* hdb0 hdb1 */
+        on |= hb[i].x > 0.1f;
+      }
+      if (on) {
+#pragma unroll
+        for (int i = 0; i < M; ++i) {
+          const double h = (d[i] - (double) hb[i].x) * (double) hb[i].y;
+          const double v = __builtin_fma((double) hb[i].y, gd_exp64((-0.5 * h) * h, C.K), acc.hdb);
+          acc.hdb = hb[i].x > 0.1f ? v : acc.hdb;
         }
       }
     }
@@ -360,6 +403,7 @@ gd_rescore64_kernel(const gd_pack *__restrict__ packs, const gd_r64_task *__rest
 
   if (active) {
     gd_r64_consts C;
+    C.K = gd_exp64_coeffs();
     {
       const double lj0 = P.sc.lj0, el0 = P.sc.el0, el1 = P.sc.el1;
       C.lj0 = lj0;
@@ -410,7 +454,7 @@ gd_rescore64_kernel(const gd_pack *__restrict__ packs, const gd_r64_task *__rest
         const double ex = ax[a] - q.x, ey = ay[a] - q.y, ez = az[a] - q.z;
         const double d2 = __builtin_fma(ez, ez, __builtin_fma(ey, ey, ex * ex));
         /* the pairs that pad a round name a point of weight 0 */
-        kde += q.w != 0.0f ? aw[a] * gd_exp64((double) P.kde2 * d2) : 0.0;
+        kde += q.w != 0.0f ? aw[a] * gd_exp64((double) P.kde2 * d2, C.K) : 0.0;
       }
       double lhm = 0.0;
       for (int mm = sl; mm < P.pos; mm += GD_R64_SLICES) {
