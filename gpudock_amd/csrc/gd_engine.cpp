@@ -1108,6 +1108,58 @@ int gd_engine::results(int handle, gd_mclog *mclog, gd_replica_result *results)
   return GD_OK;
 }
 
+int gd_engine::results_all(const int *handles, int n, gd_mclog *mclogs,
+                           gd_replica_result **res)
+{
+  std::vector<GdCollect> cs(n);
+  size_t bytes = 0, scratch = 0;
+  for (int i = 0; i < n; ++i) {
+    cs[i].handle = handles[i];
+    cs[i].host_bytes = GdArena::round(collect_bytes(handles[i]));
+    bytes += cs[i].host_bytes;
+    GdSlot *s = find(handles[i]);
+    if (s)   /* an energy row and at most one task a replica */
+      scratch += (size_t) s->img->P.n_rep * (10 * sizeof(double) + sizeof(gd_r64_task));
+  }
+  auto one_by_one = [&]() -> int {
+    for (int i = 0; i < n; ++i) {
+      const int rc = results(handles[i], mclogs ? &mclogs[i] : nullptr,
+                             res ? res[i] : nullptr);
+      if (rc)
+        return rc;
+    }
+    return GD_OK;
+  };
+  if (n < 2 || scratch > arena.size() - arena.used())
+    return one_by_one();
+  std::unique_ptr<char[]> host(new char[bytes]);
+  size_t off = 0;
+  for (GdCollect &c : cs) {
+    c.host = host.get() + off;
+    off += c.host_bytes;
+  }
+  hipEvent_t done = nullptr;
+  const int rc = collect_async(cs.data(), n, &done);
+  const hipError_t he = hipStreamSynchronize(stream);
+  if (done)
+    (void) hipEventDestroy(done);
+  if (rc == GD_ERR_NOMEM)
+    return one_by_one();   /* no single block is left for it */
+  if (rc)
+    return rc;
+  if (he != hipSuccess)
+    return gd_fail(GD_ERR_HIP, "read-back: %s", hipGetErrorString(he));
+  drain_timing();
+  reap();
+  for (int i = 0; i < n; ++i) {
+    GdSlot *s = find(handles[i]);
+    gd_parse_state(*s->img, s->blk, cs[i].host,
+                   (const double *) (cs[i].host + GdArena::round(s->state_bytes())),
+                   mclogs ? &mclogs[i] : nullptr, res ? res[i] : nullptr);
+  }
+  return GD_OK;
+}
+
 /* ------------------------------------------------------------------------ */
 /* C ABI: engine                                                             */
 /* ------------------------------------------------------------------------ */
@@ -1609,11 +1661,12 @@ extern "C" int gd_batch_run(int n_jobs, const gd_job *jobs, const gd_batch_confi
   if (rc)
     return rc;
   auto t3 = std::chrono::steady_clock::now();
-  for (int i = 0; i < n_jobs; ++i) {
-    rc = eng.results(handles[i], mclogs ? &mclogs[i] : nullptr, results ? results[i] : nullptr);
-    if (rc)
-      return rc;
-  }
+  /* every job's FP64 re-score in one launch and one wait where the arena has
+   * room for its scratch, else job by job (24 uneven jobs of 100 steps: 67 us of
+   * kernel and a wait for each, 62.5 ms a batch | 61.1) */
+  rc = eng.results_all(handles.data(), n_jobs, mclogs, results);
+  if (rc)
+    return rc;
   auto t4 = std::chrono::steady_clock::now();
   if (report) {
     report->admit_s = std::chrono::duration<double>(t1 - t0).count();

@@ -158,6 +158,9 @@ struct gd_engine {
   int sync();
   /* synchronous results of one complex */
   int results(int handle, gd_mclog *mclog, gd_replica_result *results);
+  /* the same for n complexes in one launch and one wait, where the arena has
+   * room */
+  int results_all(const int *handles, int n, gd_mclog *mclogs, gd_replica_result **res);
   /* queue, for complexes cs[0..n), one FP64 re-score launch of all their
    * replicas' best poses and the read-back of each into cs[i].host
    * (cs[i].host_bytes >= collect_bytes()); *done (created here) is recorded
