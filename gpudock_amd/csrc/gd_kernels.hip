@@ -934,8 +934,10 @@ __device__ __forceinline__ void gd_split_sums(gd_lds_f32 *areas, int role, int s
       if (f == GD_F_KDE)
         x = x / Z.kde3;
       float y = x / lna_f;
-      if (f == GD_F_HDB)
+      if (f == GD_F_HDB) {
+        GD_KEEP_BRANCH();
         y = y / 0x1.40d932p+1f * -1.0f;   /* sqrt(2 pi) */
+      }
       gd_term_put(Z, term, f, y);
     } else if (q == 6) {
       gd_term_put(Z, term, GD_F_HPC, gd_ordered_sum(A + GD_SA_EHPC, 1) / lna_f);
@@ -1007,6 +1009,38 @@ __device__ __forceinline__ float gd_split_energy(const gd_split_consts &Z, const
   const int k = Z.term_order ? i : (int) ((GD_S2F >> (4 * i)) & 0xfu);
   const float v = term[k];
   return lane == GD_E_TOTAL ? total : v;
+}
+
+/* gd_exp without a branch: the general form at the clamped argument, then the
+ * special cases selected.  The same bits; three branches on a vector compare
+ * cost the deciding wavefront, which all others wait for, more than they save. */
+__device__ __forceinline__ float gd_exp_select(float x)
+{
+  const float xc = __builtin_fminf(__builtin_fmaxf(x, -86.0f), 88.0f);
+  const float n = gd_rint(xc * 0x1.715476p+0f);
+  float r = gd_fma(-n, 0x1.62e430p-1f, xc);
+  r = gd_fma(-n, -0x1.05c610p-29f, r);
+  float p = 0x1.a01a02p-13f;
+  p = gd_fma(p, r, 0x1.6c16c2p-10f);
+  p = gd_fma(p, r, 0x1.111112p-7f);
+  p = gd_fma(p, r, 0x1.555556p-5f);
+  p = gd_fma(p, r, 0x1.555556p-3f);
+  p = gd_fma(p, r, 0.5f);
+  p = gd_fma(p, r, 1.0f);
+  p = gd_fma(p, r, 1.0f);
+  float v = p * gd_as_float((uint32_t) ((int) n + 127) << 23);
+  v = x > 88.0f ? gd_as_float(GD_INF_BITS) : v;
+  v = x < -86.0f ? 0.0f : v;
+  return x != x ? x : v;
+}
+
+/* gd_metropolis with it. */
+__device__ __forceinline__ int gd_split_decide(float e_new, float e_old, float mb, float u,
+                                               float u2, int fixed_draws, int reverse)
+{
+  const float d = e_new - e_old;
+  const float p = gd_exp_select((reverse ? -d : d) * mb);
+  return fixed_draws || (reverse ? u2 : u) < p;
 }
 
 /* MCC from the counts of the step's sums (uniform; 0 without MCC). */
@@ -1341,7 +1375,7 @@ __device__ __forceinline__ void gd_replica_cycle_split(const gd_pack &P, const c
         const gd_lds_f32 *term = A + GD_SA_TERM;
         const gd_lds_f32 *u = A + GD_SA_DRAW + (s - c0) * 8 + 6;
         total = Z.combine ? gd_split_bayes(Z, term) : gd_split_total(term, w);
-        took = gd_metropolis(total, e_old, mb, u[0], u[1], Z.fixed_draws, Z.reverse);
+        took = gd_split_decide(total, e_old, mb, u[0], u[1], Z.fixed_draws, Z.reverse);
         int next = sel + (took ? 2 : 1);
         next = next >= 3 ? next - 3 : next;
         *(gd_lds_i32 *) (A + GD_SA_SEL) = next;
