@@ -1949,28 +1949,27 @@ static hipError_t set_attr_wpg(int bytes)
   return e;
 }
 
-static hipError_t set_attr_split(const void *kernel, int bytes)
+static hipError_t set_attr_split(const void *kernel)
 {
-  /* at most the device's LDS, less the room: a complex whose
-   * staging and split area exceed it does not run split (the engine checks
-   * the same sum), but others in the engine may */
+  /* the device's LDS less the room, whatever this launch needs: launches of
+   * other threads set the same value, and a complex whose staging and area
+   * exceed it does not run split (the engine checks the same sum) */
   int dev = 0, max_lds = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e == hipSuccess)
     e = hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
   if (e != hipSuccess)
     return e;
-  const int want = bytes + GD_SPLIT_LDS_BYTES(GD_SPLIT_MAX_SHARE);
   return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (want < max_lds ? want : max_lds) - GD_SPLIT_ROOM);
+                             max_lds - GD_SPLIT_ROOM);
 }
 
 hipError_t gd_set_kernel_attrs(int stage_bytes)
 {
-  hipError_t e = set_attr_split((const void *) gd_pose_split_kernel, stage_bytes);
-  if (e == hipSuccess) e = set_attr_split((const void *) gd_mc_split_kernel<4>, stage_bytes);
-  if (e == hipSuccess) e = set_attr_split((const void *) gd_mc_split_kernel<8>, stage_bytes);
-  if (e == hipSuccess) e = set_attr_split((const void *) gd_mc_split_kernel<16>, stage_bytes);
+  hipError_t e = set_attr_split((const void *) gd_pose_split_kernel);
+  if (e == hipSuccess) e = set_attr_split((const void *) gd_mc_split_kernel<4>);
+  if (e == hipSuccess) e = set_attr_split((const void *) gd_mc_split_kernel<8>);
+  if (e == hipSuccess) e = set_attr_split((const void *) gd_mc_split_kernel<16>);
   if (e == hipSuccess) e = set_attr_wpg<4>(stage_bytes);
   if (e == hipSuccess) e = set_attr_wpg<8>(stage_bytes);
   if (e == hipSuccess) e = set_attr_wpg<16>(stage_bytes);
