@@ -269,10 +269,12 @@ gd_engine::Split gd_engine::split_of(const GdImage &I, long long n_rep) const
   if (most < 1 || lc.split == 1)
     return {1, 1};
   if (lc.split > 1) {
-    /* asked for: workgroups of 16 where the areas of 16 / split replicas
-     * fit, else of `split` wavefronts with one */
+    /* asked for: with more replicas than CUs, workgroups of 16 where the areas
+     * of 16 / split replicas fit, else of `split` wavefronts with one (64
+     * replicas of 24 x 300 eight to a replica 88 us a cycle, shared 105) */
     const int share = 16 / lc.split;
-    return share <= most ? Split{16, share} : Split{lc.split, 1};
+    const int whole = lc.split == 5 ? 4 : lc.split;   /* 5: the tuner's three a workgroup */
+    return share <= most && n_rep > n_cu ? Split{16, share} : Split{whole, 1};
   }
   const int groups = std::min(max_lds / (stage + lc.wpg * GD_WSLOT_FLOATS * 4), 20 / lc.wpg);
   const long long waves = std::min<long long>(std::max(groups, 1) * lc.wpg, n_rep / n_cu);

@@ -400,9 +400,9 @@ typedef struct gd_engine_config {
                           for each resident complex (several where one
                           wavefront per replica would leave a SIMD fewer than
                           four: few replicas, or tables that fill a CU's
-                          LDS), 1 = one, or 4, 8, 16: workgroups of 16
-                          wavefronts that 16 / split replicas share, or where
-                          their LDS areas do not fit, of `split` with one; the
+                          LDS), 1 = one, or 4, 8, 16: workgroups of `split`
+                          wavefronts with one replica, or with more replicas
+                          than CUs, of 16 that 16 / split replicas share; the
                           energies are the same bits for
                           every choice.  A complex with more than 64 position
                           restraints, or whose staged tables leave no room in
