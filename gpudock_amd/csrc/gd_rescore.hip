@@ -58,7 +58,8 @@ __device__ __forceinline__ double gd_rcp64(double x)
  * is then the low word), r = x - n ln2 in two steps, e^r = 1 + r + r^2 q(r)
  * with q of degree 9 interpolated here at the Chebyshev nodes of
  * |r| <= ln2 / 2 (truncation below 1e-17), scaled by v_ldexp_f64.  Clamped at
- * -700 (1e-304: no sum can tell it from 0).  The coefficients of r^11 .. r^3
+ * -700 (1e-304: no sum can tell it from 0) by a compare, which leaves a NaN a
+ * NaN where a maximum would drop it.  The coefficients of r^11 .. r^3
  * come in scalar registers (gd_exp64_coeffs): as literals each is copied into
  * the accumulator of its fma first, a fifth of the pair loop's instructions. */
 struct gd_exp64_c {
@@ -78,7 +79,7 @@ __device__ __forceinline__ gd_exp64_c gd_exp64_coeffs()
 
 __device__ __forceinline__ double gd_exp64(double x, const gd_exp64_c &K)
 {
-  const double xc = __builtin_fmax(x, -700.0);
+  const double xc = x < -700.0 ? -700.0 : x;
   const double t = __builtin_fma(xc, 0x1.71547652b82fep+0, 0x1.8p+52);
   const double n = t - 0x1.8p+52;
   double r = __builtin_fma(-n, 0x1.62e42fefa39efp-1, xc);

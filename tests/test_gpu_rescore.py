@@ -68,3 +68,27 @@ def test_fp64_degenerate_distances():
     vdw = remc.SLOTS.index("vdw")
     assert np.isnan(r64[:, vdw]).all() and np.isfinite(r64[0, 1:9]).all()
     np.testing.assert_allclose(e64, r64, rtol=TOL, atol=TOL)
+
+
+@pytest.mark.parametrize("lna,pnp,pnk,pos", [(24, 300, 300, 11), (65, 129, 700, 0)])
+def test_fp64_nan_poses_keep_their_nan(lna, pnp, pnk, pos):
+    """A NaN of either sign in the translation or an angle, and an infinite
+    angle: every term that the oracle gives as NaN is NaN, the others have its
+    value, and the poses beside them are untouched."""
+    cx = synth.make_complex(pnp=pnp, radius=None, lna=lna, n_lig=1, n_prt=1, pnk=pnk, pos=pos,
+                            seed=lna)
+    mv = np.zeros((8, 6), np.float32)
+    mv[1, 0] = np.nan
+    mv[2, 2] = -np.float32(np.nan)
+    mv[3, 4] = np.nan
+    mv[4, 3] = np.inf
+    mv[6, :] = np.nan
+    z = np.zeros(len(mv), np.int32)
+    with np.errstate(all="ignore"):
+        r64 = O.pose_ref64(cx, z, z, mv)
+    for name in ("hdb", "kde"):
+        k = remc.SLOTS.index(name)
+        assert np.isnan(r64[[1, 2, 3, 4, 6], k]).all() and np.isfinite(r64[[0, 5, 7], k]).all()
+    for noalloc in (False, True):
+        _, e64 = remc.score_poses(cx, z, z, mv, noalloc=noalloc)
+        np.testing.assert_allclose(e64, r64, rtol=TOL, atol=TOL)
