@@ -1730,11 +1730,19 @@ ScoreLayout score_layout(const ScoreJob &J, int n_pose)
 }
 
 /* What a call counts against the static workspace: the image, one task list
- * and 156 bytes a pose (conformers, order, move, both energies).  The
- * workspace holds GD_SCRATCH_SLACK more than that limit for the FP64 tasks:
- * at most 20 bytes a conformer of at least 1.8 KB of image, and 2.5 a pose
- * against the 4 counted for its protein conformer, and for the 16 bytes a
- * pose of split FP32 tasks, of which there are less than 14 a CU. */
+ * (2 bytes a pose or more) and 156 bytes a pose (conformers, order, move, both
+ * energies).  The layout takes more than that, which is what the workspace
+ * holds GD_SCRATCH_SLACK above the limit for:
+ *   FP64 tasks of two poses: 20 bytes each, 6 a pose more than the 4 counted
+ *   for its protein conformer, and 10 for the odd pose of a conformer, whose
+ *   image takes 1.8 KB or more;
+ *   up to four poses a CU, FP64 tasks of one pose, and below 14 a CU, split
+ *   FP32 tasks of one pose: 36 bytes a pose;
+ *   the rounding of the arrays to 256 bytes. */
+static_assert(GD_SCRATCH_SLACK >= GD_SCRATCH_BYTES / 158 * (sizeof(gd_r64_task) / 2 - 4) +
+                                      14 * 256 * (sizeof(gd_task) + sizeof(gd_r64_task)) +
+                                      9 * 256,
+              "slack of the static workspace");
 size_t score_counted(const ScoreJob &J, int n_pose)
 {
   size_t b = GdArena::round(gd_image_footprint(J.I)) + GdArena::round(J.tasks8 * sizeof(gd_task));
@@ -1928,12 +1936,15 @@ extern "C" int gd_score_poses_noalloc(const gd_ligand *lig, const gd_protein *pr
     return rc;
   const ScoreLayout L = score_layout(J, n_pose);
   const size_t need = score_counted(J, n_pose);
-  if (need > GD_SCRATCH_BYTES || L.total > GD_SCRATCH_BYTES + GD_SCRATCH_SLACK)
+  if (need > GD_SCRATCH_BYTES)
     return gd_fail(GD_ERR_ARG,
                    "gd_score_poses_noalloc: %d poses of this complex need %zu bytes of "
                    "workspace; the static workspace holds %zu (use gd_score_poses, or fewer "
                    "poses per call)",
                    n_pose, need, (size_t) GD_SCRATCH_BYTES);
+  if (L.total > GD_SCRATCH_BYTES + GD_SCRATCH_SLACK)
+    return gd_fail(GD_ERR_ARG, "gd_score_poses_noalloc: %zu bytes of %zu", L.total,
+                   (size_t) (GD_SCRATCH_BYTES + GD_SCRATCH_SLACK));
   if (gd_device_count() < 1)
     return gd_fail(GD_ERR_NODEV, "no HIP device visible");
   if (n_pose == 0)

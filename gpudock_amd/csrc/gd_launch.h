@@ -62,7 +62,7 @@ hipError_t gd_set_kernel_attrs(int stage_bytes);
 /* Bytes of the static per-GPU workspace of gd_score_poses_noalloc. */
 #define GD_SCRATCH_BYTES ((size_t) 64 << 20)
 /* room in it beyond what a call is counted for (score_counted) */
-#define GD_SCRATCH_SLACK ((size_t) 1 << 20)
+#define GD_SCRATCH_SLACK ((size_t) 3 << 20)
 /* Device address of that workspace on `device`, which must be the current
  * device; resolved once per device (hipGetSymbolAddress) and kept. */
 hipError_t gd_scratch_region(int device, char **ptr);
