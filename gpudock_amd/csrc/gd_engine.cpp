@@ -441,7 +441,7 @@ int gd_engine::rebuild()
   }
   pending_init.clear();
   lc.stage_bytes = max_stage;
-  GD_HIP_TRY(gd_set_kernel_attrs(std::max({max_stage, init_stage, init_split_stage})));
+  GD_HIP_TRY(gd_set_kernel_attrs());
   auto start = [&](const std::vector<gd_task> &list, bool split) -> int {
     if (list.empty())
       return GD_OK;
@@ -1856,7 +1856,7 @@ int score_run(char *B, const ScoreLayout &L, ScoreJob &J, int n_pose, const int 
   put(move, (size_t) n_pose * 24, L.mv);
   put(host.get(), one_up ? L.mv + (size_t) n_pose * 24 : img, L.img);
   if (he == hipSuccess && energy) {
-    he = gd_set_kernel_attrs(J.I.P.lds_bytes);
+    he = gd_set_kernel_attrs();
     if (he == hipSuccess)
       he = gd_launch_score(pack_dev, (const gd_task *) (B + L.tasks), (int) J.tasks.size(),
                            (const int *) (B + L.order), (const int *) (B + L.lc),

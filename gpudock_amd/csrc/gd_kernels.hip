@@ -1932,50 +1932,30 @@ hipError_t gd_launch_init_split(const gd_pack *packs, const gd_task *tasks, int 
                            share, nullptr, st);
 }
 
-template <int WPG, int MINW>
-static hipError_t set_attr_var(int bytes)
+/* The dynamic LDS limit of every MC and scoring kernel: the device's LDS less
+ * the room for static LDS, whatever a launch needs.  The limit belongs to the
+ * process, so launches of other threads and engines must set the same value;
+ * one that set its own smaller need would lower it between another's setting
+ * and launch.  (No complex runs that needs more: the image and the engine
+ * check the same sums.) */
+hipError_t gd_set_kernel_attrs()
 {
-  return hipFuncSetAttribute((const void *) gd_mc_kernel<WPG, MINW>,
-                             hipFuncAttributeMaxDynamicSharedMemorySize,
-                             bytes + WPG * GD_WSLOT_FLOATS * 4);
-}
-
-template <int WPG>
-static hipError_t set_attr_wpg(int bytes)
-{
-  hipError_t e = set_attr_var<WPG, 1>(bytes);
-  if (e == hipSuccess) e = set_attr_var<WPG, 6>(bytes);
-  if (e == hipSuccess) e = set_attr_var<WPG, 8>(bytes);
-  return e;
-}
-
-static hipError_t set_attr_split(const void *kernel)
-{
-  /* the device's LDS less the room, whatever this launch needs: launches of
-   * other threads set the same value, and a complex whose staging and area
-   * exceed it does not run split (the engine checks the same sum) */
   int dev = 0, max_lds = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e == hipSuccess)
     e = hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
-  if (e != hipSuccess)
-    return e;
-  return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                             max_lds - GD_SPLIT_ROOM);
-}
-
-hipError_t gd_set_kernel_attrs(int stage_bytes)
-{
-  hipError_t e = set_attr_split((const void *) gd_pose_split_kernel);
-  if (e == hipSuccess) e = set_attr_split((const void *) gd_mc_split_kernel<4>);
-  if (e == hipSuccess) e = set_attr_split((const void *) gd_mc_split_kernel<8>);
-  if (e == hipSuccess) e = set_attr_split((const void *) gd_mc_split_kernel<16>);
-  if (e == hipSuccess) e = set_attr_wpg<4>(stage_bytes);
-  if (e == hipSuccess) e = set_attr_wpg<8>(stage_bytes);
-  if (e == hipSuccess) e = set_attr_wpg<16>(stage_bytes);
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void *) gd_score_kernel,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, stage_bytes);
+  const void *kernels[] = {
+      (const void *) gd_pose_split_kernel,   (const void *) gd_mc_split_kernel<4>,
+      (const void *) gd_mc_split_kernel<8>,  (const void *) gd_mc_split_kernel<16>,
+      (const void *) gd_mc_kernel<4, 1>,     (const void *) gd_mc_kernel<4, 6>,
+      (const void *) gd_mc_kernel<4, 8>,     (const void *) gd_mc_kernel<8, 1>,
+      (const void *) gd_mc_kernel<8, 6>,     (const void *) gd_mc_kernel<8, 8>,
+      (const void *) gd_mc_kernel<16, 1>,    (const void *) gd_mc_kernel<16, 6>,
+      (const void *) gd_mc_kernel<16, 8>,    (const void *) gd_score_kernel};
+  for (const void *k : kernels)
+    if (e == hipSuccess)
+      e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              max_lds - GD_SPLIT_ROOM);
   return e;
 }
 

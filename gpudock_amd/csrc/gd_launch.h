@@ -57,7 +57,8 @@ hipError_t gd_launch_rescore64(const gd_pack *packs, const gd_r64_task *tasks, i
                                int split, int max_lna, int lds_bytes, int max_lds,
                                const int *order, const int *lig_conf, const float *move,
                                double *energy, hipStream_t st);
-hipError_t gd_set_kernel_attrs(int stage_bytes);
+/* before the first launch on the current device */
+hipError_t gd_set_kernel_attrs();
 
 /* Bytes of the static per-GPU workspace of gd_score_poses_noalloc. */
 #define GD_SCRATCH_BYTES ((size_t) 64 << 20)
