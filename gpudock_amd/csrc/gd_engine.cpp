@@ -266,7 +266,7 @@ gd_engine::Split gd_engine::split_of(const GdImage &I, long long n_rep) const
 {
   const int stage = stage_of(I);
   const int most = max_share(I, stage, max_lds);
-  if (most < 1 || lc.split == 1)
+  if (most < 1 || lc.split == 1 || whole_lists)
     return {1, 1};
   if (lc.split > 1) {
     /* asked for: with more replicas than CUs, workgroups of 16 where the areas
@@ -304,6 +304,19 @@ int gd_engine::choose_split() const
  * members (fresh blocks: queued launches keep reading the old ones, which
  * are released behind them). */
 int gd_engine::rebuild()
+{
+  whole_lists = false;
+  int rc = build_lists();
+  if (rc == GD_ERR_NOMEM && split_eff > 1) {
+    /* tasks of split replicas hold four at most, of whole ones lc.wpg: an
+     * arena that has no room for the longer list runs them whole */
+    whole_lists = true;
+    rc = build_lists();
+  }
+  return rc;
+}
+
+int gd_engine::build_lists()
 {
   drop_graph();
   split_eff = choose_split();
@@ -399,6 +412,12 @@ int gd_engine::rebuild()
   if (chains_bytes) defer(chains_off, chains_bytes);
   packs_bytes = tasks_bytes = chains_bytes = 0;
   packs_off = tasks_off = chains_off = 0;
+  if (whole_lists) {
+    /* room is short: the old lists go first, so that the new ones leave one
+     * block free, not two */
+    (void) hipStreamSynchronize(stream);
+    reap();
+  }
   auto place = [&](size_t &off, size_t &cap, const void *src, size_t bytes) -> int {
     if (!bytes)
       return GD_OK;
@@ -422,6 +441,7 @@ int gd_engine::rebuild()
    * replicas run whole and one over those that are split, queued before the
    * first cycle that includes them */
   std::vector<gd_task> init_tasks, init_split;
+  std::vector<int> split_handles;
   int init_stage = 16, init_split_stage = 16, init_share = 1;
   for (int h : pending_init) {
     GdSlot *s = find(h);
@@ -434,45 +454,58 @@ int gd_engine::rebuild()
       gd_complex_tasks(*s->img, s->cx_index, sp.share, init_split);
       init_split_stage = std::max(init_split_stage, stage);
       init_share = std::max(init_share, sp.share);
+      split_handles.push_back(h);
     } else {
       gd_complex_tasks(*s->img, s->cx_index, lc.wpg, init_tasks);
       init_stage = std::max(init_stage, stage);
     }
   }
-  pending_init.clear();
   lc.stage_bytes = max_stage;
   GD_HIP_TRY(gd_set_kernel_attrs());
   auto start = [&](const std::vector<gd_task> &list, bool split) -> int {
     if (list.empty())
       return GD_OK;
-    const size_t tb = GdArena::round(vbytes(list));
-    const size_t toff = arena_take(*this, tb, true);
+    /* a split list that the arena has no room for: an eighth of it at a time,
+     * what whole replicas' tasks would take */
+    size_t per = list.size();
+    size_t toff = arena_take(*this, GdArena::round(per * sizeof(gd_task)), true);
+    if (toff == (size_t) -1 && split) {
+      per = std::max<size_t>(1, per / 8);
+      toff = arena_take(*this, GdArena::round(per * sizeof(gd_task)), true);
+    }
     if (toff == (size_t) -1)
       return gd_fail(GD_ERR_NOMEM, "arena too small for the initial-energy tasks");
-    int rc2 = upload(arena.base() + toff, list.data(), vbytes(list));
     const gd_pack *pd = (const gd_pack *) (arena.base() + packs_off);
     const gd_task *td = (const gd_task *) (arena.base() + toff);
+    int rc2 = GD_OK;
     hipError_t he = hipSuccess;
-    if (!rc2 && split) {
-      he = gd_launch_init_split(pd, td, (int) list.size(), init_split_stage, init_share, stream);
-    } else if (!rc2) {
-      gd_launch_cfg ic = lc;
-      ic.persistent = 0;
-      ic.split = 1;
-      ic.stage_bytes = init_stage;
-      he = gd_launch_mc(ic, pd, td, (int) list.size(), nullptr, (int) list.size(), 1, 1, stream);
+    for (size_t k = 0; k < list.size() && !rc2 && he == hipSuccess; k += per) {
+      const int n = (int) std::min(per, list.size() - k);
+      rc2 = upload(arena.base() + toff, list.data() + k, n * sizeof(gd_task));
+      if (!rc2 && split) {
+        he = gd_launch_init_split(pd, td, n, init_split_stage, init_share, stream);
+      } else if (!rc2) {
+        gd_launch_cfg ic = lc;
+        ic.persistent = 0;
+        ic.split = 1;
+        ic.stage_bytes = init_stage;
+        he = gd_launch_mc(ic, pd, td, n, nullptr, n, 1, 1, stream);
+      }
     }
-    defer(toff, tb);
+    defer(toff, GdArena::round(per * sizeof(gd_task)));
     if (rc2)
       return rc2;
     GD_HIP_TRY(he);
     return GD_OK;
   };
   rc = start(init_tasks, false);
-  if (!rc)
-    rc = start(init_split, true);
   if (rc)
     return rc;
+  pending_init = split_handles;   /* (an initial energy is evaluated once) */
+  rc = start(init_split, true);
+  if (rc)
+    return rc;
+  pending_init.clear();
   dirty = false;
   ++n_rebuilds;
   return GD_OK;
@@ -1042,22 +1075,42 @@ int gd_engine::collect_async(GdCollect *cs, int n, hipEvent_t *done)
     row += s->img->P.n_rep;
     lds = std::max(lds, gd_rescore64_lds(s->img->P, split, max_lna, max_lds));
   }
-  const size_t ib = GdArena::round(items.size() * sizeof(gd_r64_task));
+  /* one launch over all tasks, or where the arena has no room for their list,
+   * launches behind one another over as many as 8 bytes a replica hold; with no
+   * room for that either, the task lists of whole replicas make some */
   const size_t eb = GdArena::round(nitem * 10 * sizeof(double));
-  const size_t ioff = arena_take(*this, ib, true);
-  const size_t eoff = ioff == (size_t) -1 ? (size_t) -1 : arena_take(*this, eb, true);
-  if (eoff == (size_t) -1) {
-    if (ioff != (size_t) -1)
+  size_t per = 0, ib = 0, ioff = (size_t) -1, eoff = (size_t) -1;
+  auto take = [&](size_t most) {
+    per = std::max<size_t>(1, std::min(items.size(), most));
+    ib = GdArena::round(per * sizeof(gd_r64_task));
+    ioff = arena_take(*this, ib, true);
+    eoff = ioff == (size_t) -1 ? (size_t) -1 : arena_take(*this, eb, true);
+    if (eoff == (size_t) -1 && ioff != (size_t) -1)
       arena.free(ioff, ib);
-    return gd_fail(GD_ERR_NOMEM, "arena too small for the FP64 re-score");
+    return eoff != (size_t) -1;
+  };
+  const size_t few = nitem * 8 / sizeof(gd_r64_task);
+  bool room = take(items.size()) || take(few);
+  if (!room && split_eff > 1) {
+    whole_lists = true;
+    rc = build_lists();
+    if (rc)
+      return rc;
+    room = take(few);
   }
+  if (!room)
+    return gd_fail(GD_ERR_NOMEM, "arena too small for the FP64 re-score");
   const double *e64 = (const double *) (arena.base() + eoff);
-  rc = upload(arena.base() + ioff, items.data(), vbytes(items));
-  hipError_t he = rc ? hipSuccess
-                     : gd_launch_rescore64((const gd_pack *) (arena.base() + packs_off),
-                                           (const gd_r64_task *) (arena.base() + ioff),
-                                           (int) items.size(), split, max_lna, lds, max_lds,
-                                           nullptr, nullptr, nullptr, (double *) e64, stream);
+  hipError_t he = hipSuccess;
+  for (size_t k = 0; k < items.size() && !rc && he == hipSuccess; k += per) {
+    const size_t m = std::min(per, items.size() - k);
+    rc = upload(arena.base() + ioff, items.data() + k, m * sizeof(gd_r64_task));
+    if (!rc)
+      he = gd_launch_rescore64((const gd_pack *) (arena.base() + packs_off),
+                               (const gd_r64_task *) (arena.base() + ioff), (int) m, split,
+                               max_lna, lds, max_lds, nullptr, nullptr, nullptr, (double *) e64,
+                               stream);
+  }
   size_t first = 0;
   for (int i = 0; i < n && !rc && he == hipSuccess; ++i) {
     GdSlot *s = ss[i];

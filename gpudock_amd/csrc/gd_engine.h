@@ -179,6 +179,8 @@ struct gd_engine {
 
 private:
   int rebuild();
+  int build_lists();
+  bool whole_lists = false;         /* no room for the task lists of split replicas */
   void drop_graph();
   void defer(size_t off, size_t bytes, hipGraph_t g = nullptr, hipGraphExec_t x = nullptr,
              bool host = false);
