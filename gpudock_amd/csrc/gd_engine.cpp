@@ -681,26 +681,46 @@ int gd_engine::enqueue_cycle()
   return GD_OK;
 }
 
+/* Time of one MC step of a workgroup, seconds, some 30 % either way: pairs by
+ * the rate of the wavefronts that share it, restraints, and the serial end.
+ * Measured a workgroup of 16 at 7.7e3 pairs a step 6.7 us, 6.6e4 25, 5.2e5 156;
+ * 8 wavefronts 31 and 4 57 us at 6.6e4; one wavefront per replica 2.7e8 pairs/s
+ * with little beside it, 2e8 on a full device. */
+static double step_seconds(const gd_pack &P, int waves, int replicas)
+{
+  const double pairs = (double) P.lna * P.pnp_pad + P.kde_n_lo + P.kde_n_hi;
+  const double w = waves / (double) replicas;   /* wavefronts of a replica */
+  return 5e-6 + pairs / (2e8 * w) + P.pos * 2e-7 / w;
+}
+
 /* Cycles that one launch may run of n: all of them, within bounds, while no
  * resident complex has temperatures to swap between cycles: 100 cycles of 63
  * replicas of 34 atoms x 344 points at one temperature take 8.1 ms in one
- * launch, and 9.8 in one a cycle with its staging, advance and gaps.  A launch stays within
- * 1,000 steps and about 50 ms (4e10 pairs), so that other streams get their
- * turn. */
+ * launch, and 9.8 in one a cycle with its staging, advance and gaps.  A launch
+ * stays within 1,000 steps and, unless one cycle takes longer, about 50 ms, so
+ * that other work gets its turn: 4e10 pairs on the whole device, and the same
+ * time for the slowest workgroup (one replica of 128 x 7,000 runs 160 steps in
+ * it, not 1,000). */
 int gd_engine::merged_cycles(int n) const
 {
-  double pairs = 0.0;   /* of one cycle */
+  double pairs = 0.0, longest = 1e-6;   /* of one cycle */
   int spe = 1;
+  const long long n_rep = replicas();
   for (auto *s : slots) {
     const gd_pack &P = s->img->P;
     if (P.exchange && P.n_tmp >= 2)
       return 1;
+    const Split sp = split_of(*s->img, n_rep);
     pairs += (double) P.n_rep * P.lna * P.pnp_pad * P.spe;
+    longest = std::max(longest, P.spe * step_seconds(P, sp.waves, sp.share));
     spe = std::max(spe, P.spe);
   }
-  const double most = std::min(1000.0 / spe, 4e10 / std::max(pairs, 1.0));
+  const double most = std::min({1000.0 / spe, 4e10 / std::max(pairs, 1.0), 0.05 / longest});
   return std::max(1, std::min(n, (int) most));
 }
+
+/* the same for the tests */
+extern "C" int gd_engine_merged_cycles(const gd_engine *e, int n) { return e->merged_cycles(n); }
 
 int gd_engine::cycles(int n)
 {

@@ -155,6 +155,8 @@ struct gd_engine {
   int remove(int handle);
   GdSlot *find(int handle);
   int cycles(int n);
+  /* cycles that the next launch would run of n */
+  int merged_cycles(int n) const;
   int sync();
   /* synchronous results of one complex */
   int results(int handle, gd_mclog *mclog, gd_replica_result *results);
@@ -189,7 +191,6 @@ private:
   int upload(char *dev, const void *src, size_t bytes);
   int upload_image(GdImage &I, size_t off, GdBlock &b);
   int enqueue_cycle();
-  int merged_cycles(int n) const;
   int trial_cycle();
   /* LDS staging bytes of a complex */
   int stage_of(const GdImage &I) const;
