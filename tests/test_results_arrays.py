@@ -26,3 +26,17 @@ def test_results_to_numpy(n):
     for a in out.values():
         a[...] = 0   # arrays of their own
     assert bytes(res) == raw.tobytes()
+
+
+def test_results_to_numpy_of_any_sequence():
+    """A slice of a result array, a list and a tuple of picked replicas."""
+    res = (remc.ReplicaResult * 9)()
+    for i, r in enumerate(res):
+        r.step_best, r.move_best[2], r.energy_best_fp64[9] = i, 0.5 * i, -1.0 / (i + 1)
+    for part, ids in ((res[2:7], range(2, 7)), ([res[8], res[0]], (8, 0)),
+                      (tuple(res), range(9)), ([], ())):
+        out = remc.results_to_numpy(part)
+        np.testing.assert_array_equal(out["step_best"], list(ids))
+        np.testing.assert_array_equal(out["move_best"][:, 2], [0.5 * i for i in ids])
+        np.testing.assert_array_equal(out["energy_best_fp64"][:, 9], [-1.0 / (i + 1) for i in ids])
+        assert out["move_best"].shape == (len(ids), 6)
