@@ -142,10 +142,16 @@ __device__ __forceinline__ void gd_stage(const gd_pack &P, int prt, char *smem)
 /* j and j + 64 in (ax0..az0) and (ax1..az1).  prt = the protein conformer   */
 /* staged in smem.                                                           */
 /* ------------------------------------------------------------------------ */
-/* What the energy loops need of a complex and a protein conformer, read once
- * per cycle and kept in scalar registers.  Read where it is used instead, the
- * loads are repeated after every barrier and atomic, six of them one behind
- * the other (some 2,000 cycles) before an atom block's first pair. */
+/* What the energy loops need of a complex and a protein conformer.  The split
+ * steps read it once per cycle and keep it, in scalar registers as far as they
+ * go and in lanes of vector registers beyond: read where it is used instead,
+ * the loads are repeated after every barrier and atomic, six of them one behind
+ * the other (some 2,000 cycles) before an atom block's first pair.  One
+ * wavefront per replica has no barriers and hides such loads behind the other
+ * replicas of its SIMD, so there it is read where it is used: kept over the
+ * cycle instead, it spilled 153 scalar registers for 126 (146 for 123 at 6
+ * waves a SIMD, where 16,384 replicas of 48 x 800 took 8.30 ms a cycle for
+ * 8.19; no difference at the other budgets). */
 struct gd_hot {
   int lna, nchunk, pnp_pad;
   int kp;                           /* chunks that hold a class-2 point */
@@ -616,20 +622,20 @@ __device__ __forceinline__ void gd_energy_tail(const gd_pack &P, const gd_blk &t
  * order) and *cmcc (MCC against the reference contacts, CalcMcc_d
  * calcmcc_d.cu:148-213, or 0) are identical in every lane. */
 __device__ __forceinline__ void gd_energy_wave(
-    const gd_pack &P, const gd_hot &H, const char *smem, float ax0, float ay0, float az0, float ax1,
+    const gd_pack &P, const char *smem, int prt, float ax0, float ay0, float az0, float ax1,
     float ay1, float az1, const float cen[3], float out[GD_E_N], float *cmcc)
 {
   gd_blk tot;
   tot.vdw = 0.0f; tot.pmf = 0.0f; tot.psp = 0.0f; tot.hdb = 0.0f; tot.ele = 0.0f;
   float ehpc = 0.0f;
   int tp = 0, fp = 0, fn = 0;
-  const int lna = H.lna;
+  const int lna = P.lna;
   const int bs = gd_block_size(lna);
   for (int l0 = 0; l0 < lna; l0 += bs) {
     gd_blk blk;
     float eb;
-    gd_atoms_block<false>(H, smem, ax0, ay0, az0, ax1, ay1, az1, l0, min(l0 + bs, lna),
-                          blk, &eb, tp, fp, fn);
+    gd_atoms_block<false>(gd_hot_of(P, prt), smem, ax0, ay0, az0, ax1, ay1, az1, l0,
+                          min(l0 + bs, lna), blk, &eb, tp, fp, fn);
     tot.vdw += blk.vdw;
     tot.pmf += blk.pmf;
     tot.psp += blk.psp;
@@ -637,15 +643,15 @@ __device__ __forceinline__ void gd_energy_wave(
     tot.ele += blk.ele;
     ehpc += eb;
   }
-  const int n_rounds = H.n_rounds;
+  const int n_rounds = gd_hot_of(P, prt).n_rounds;
   const int kbs = gd_block_size(n_rounds > 0 ? n_rounds : 1);
   float kde_lane = 0.0f;
   for (int r0 = 0; r0 < n_rounds; r0 += kbs)
-    kde_lane += gd_kde_rounds(H, smem, ax0, ay0, az0, ax1, ay1, az1, r0,
-                                     min(r0 + kbs, n_rounds));
+    kde_lane += gd_kde_rounds(gd_hot_of(P, prt), smem, ax0, ay0, az0, ax1, ay1, az1, r0,
+                              min(r0 + kbs, n_rounds));
   float elhm = 0.0f;
   for (int m = 0; m < P.pos; ++m)
-    elhm += gd_lhm_one(H, ax0, ay0, az0, ax1, ay1, az1, m);
+    elhm += gd_lhm_one(gd_hot_of(P, prt), ax0, ay0, az0, ax1, ay1, az1, m);
   gd_energy_tail(P, tot, ehpc, kde_lane, elhm, tp, fp, fn, cen, out, cmcc);
 }
 
@@ -702,8 +708,8 @@ __device__ __forceinline__ int gd_launch_steps(const gd_pack &P, int s0, int n_c
 /* ------------------------------------------------------------------------ */
 /* One replica, one wavefront.                                               */
 /* ------------------------------------------------------------------------ */
-__device__ __forceinline__ void gd_replica_init(const gd_pack &P, const gd_hot &H, const char *smem,
-                                                int r)
+__device__ __forceinline__ void gd_replica_init(const gd_pack &P, const char *smem, int r,
+                                                int prt)
 {
   const int lane = threadIdx.x & (GD_WAVE - 1);
   const gd_state S = P.S;
@@ -720,7 +726,7 @@ __device__ __forceinline__ void gd_replica_init(const gd_pack &P, const gd_hot &
   }
   float ax0, ay0, az0, ax1, ay1, az1, cen[3], e[GD_E_N], cm;
   gd_place(P, m, bx0, by0, bz0, bx1, by1, bz1, &ax0, &ay0, &az0, &ax1, &ay1, &az1, cen);
-  gd_energy_wave(P, H, smem, ax0, ay0, az0, ax1, ay1, az1, cen, e, &cm);
+  gd_energy_wave(P, smem, prt, ax0, ay0, az0, ax1, ay1, az1, cen, e, &cm);
   if (lane == 0) {
     S.cmcc[r] = cm;
     S.cmcc_best[r] = cm;
@@ -1168,9 +1174,9 @@ __device__ __forceinline__ void gd_slot_store(const gd_pack &P, const gd_lds_f32
 /* n_steps MC steps from step s0 of replica r on one wavefront.  The
  * movematrices and energies live in the replica's LDS slot
  * ws[GD_WSLOT_FLOATS]; only totals stay in registers. */
-__device__ __forceinline__ void gd_replica_cycle(const gd_pack &P, const gd_hot &H,
-                                                 const char *smem, gd_lds_f32 *ws, int r,
-                                                 int s0, int n_steps)
+__device__ __forceinline__ void gd_replica_cycle(const gd_pack &P, const char *smem,
+                                                 gd_lds_f32 *ws, int r, int prt, int s0,
+                                                 int n_steps)
 {
   const int lane = threadIdx.x & (GD_WAVE - 1);
   const gd_state S = P.S;
@@ -1206,7 +1212,7 @@ __device__ __forceinline__ void gd_replica_cycle(const gd_pack &P, const gd_hot 
       for (int k = 0; k < 6; ++k)
         ws[GD_WS_MNEW + k] = m_new[k];
     }
-    gd_energy_wave(P, H, smem, ax0, ay0, az0, ax1, ay1, az1, cen, e_new, &cm_new);
+    gd_energy_wave(P, smem, prt, ax0, ay0, az0, ax1, ay1, az1, cen, e_new, &cm_new);
     acs += gd_accept(P, ws, r, s, u_acc, mb, e_new, cm_new, &e_old_total, &best_total);
     __builtin_amdgcn_wave_barrier();
   }
@@ -1627,11 +1633,10 @@ gd_mc_kernel(const gd_pack *__restrict__ packs, const gd_task *__restrict__ task
       }
       if (w < task.r_count) {
         const int r = task.r_begin + w;
-        const gd_hot H = gd_hot_of(P, task.prt);
         if (mode == 0)
-          gd_replica_cycle(P, H, smem, ws, r, s0, n_steps);
+          gd_replica_cycle(P, smem, ws, r, task.prt, s0, n_steps);
         else
-          gd_replica_init(P, H, smem, r);
+          gd_replica_init(P, smem, r, task.prt);
       }
     }
     if (!queue)
@@ -1719,7 +1724,7 @@ gd_score_kernel(const gd_pack *__restrict__ packs, const gd_task *__restrict__ t
   float ax0, ay0, az0, ax1, ay1, az1, cen[3], e[GD_E_N];
   gd_place(P, m, bx0, by0, bz0, bx1, by1, bz1, &ax0, &ay0, &az0, &ax1, &ay1, &az1, cen);
   float cm;
-  gd_energy_wave(P, gd_hot_of(P, task.prt), smem, ax0, ay0, az0, ax1, ay1, az1, cen, e, &cm);
+  gd_energy_wave(P, smem, task.prt, ax0, ay0, az0, ax1, ay1, az1, cen, e, &cm);
   if (lane == 0) {
 #pragma unroll
     for (int k = 0; k < GD_E_N; ++k)
