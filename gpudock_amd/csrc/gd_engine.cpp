@@ -271,7 +271,7 @@ gd_engine::Split gd_engine::split_of(const GdImage &I, long long n_rep) const
   if (lc.split > 1) {
     /* asked for: with more replicas than CUs, workgroups of 16 where the areas
      * of 16 / split replicas fit, else of `split` wavefronts with one (64
-     * replicas of 24 x 300 eight to a replica 88 us a cycle, shared 105) */
+     * replicas of 24 x 300 eight to a replica 86 us a cycle, shared 105) */
     const int share = 16 / lc.split;
     const int whole = lc.split == 5 ? 4 : lc.split;   /* 5: the tuner's three a workgroup */
     return share <= most && n_rep > n_cu ? Split{16, share} : Split{whole, 1};

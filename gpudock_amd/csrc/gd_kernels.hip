@@ -1300,8 +1300,11 @@ __device__ __forceinline__ void gd_replica_cycle_split(const gd_pack &P, const c
    * others cover the atom blocks, the leaders place their poses first and are
    * the last wavefronts, since a SIMD issues its oldest first and the blocks
    * last longest; else they are the oldest, take a block like the others and
-   * place the poses behind it. */
-  const bool place_late = Z.nb * share > SPLIT - 2 * share;
+   * place the poses behind it.  Workgroups of 4 or 8 always place first: with
+   * one or two wavefronts a SIMD the rounds are many and the placing fits
+   * beside them (64 replicas of 24 x 300, eight to a replica, behind a block 94
+   * us a cycle, first 88). */
+  const bool place_late = SPLIT == 16 && Z.nb * share > SPLIT - 2 * share;
   const int q = place_late ? role : SPLIT - 1 - role;
   const int j_lead = q >> 1;
   const bool lead = j_lead < share;
@@ -1648,9 +1651,11 @@ gd_mc_kernel(const gd_pack *__restrict__ packs, const gd_task *__restrict__ task
  * replicas sharing them, grid form or persistent as gd_mc_kernel: for launches
  * with too few replicas to give every SIMD several, where one wavefront per
  * replica leaves most of the device idle and every step waits on its own
- * latency. */
+ * latency.  Workgroups of 4 and 8 have one replica each (the engine's rule),
+ * known to the compiler, and registers for four wavefronts a SIMD, so that two
+ * workgroups of 8 fit a CU. */
 template <int SPLIT>
-__global__ void __launch_bounds__(GD_WAVE *SPLIT)
+__global__ void __launch_bounds__(GD_WAVE *SPLIT) __attribute__((amdgpu_waves_per_eu(4, 8)))
 gd_mc_split_kernel(const gd_pack *__restrict__ packs, const gd_task *__restrict__ tasks,
                    int n_tasks, int *queue, int n_cyc, int area_off, int prio)
 {
@@ -1689,7 +1694,7 @@ gd_mc_split_kernel(const gd_pack *__restrict__ packs, const gd_task *__restrict_
       /* (the cycle's first barrier covers the staging) */
       gd_replica_cycle_split<SPLIT>(P, smem, areas, (gd_lds_i32 *) s_ctr, role, task.r_begin,
                                     s0, n_steps,
-                                    gd_split_consts_of(P, task.prt, task.r_count));
+                                    gd_split_consts_of(P, task.prt, SPLIT < 16 ? 1 : task.r_count));
     }
     if (!queue)
       t = -2;

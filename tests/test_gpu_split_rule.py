@@ -53,3 +53,21 @@ def test_split_and_whole_complexes_share_an_engine():
         assert rep["layout"]["split"] == 16 and rep["layout"]["n_classes"] >= 2
         for job, got in zip(jobs, res):
             _same(job, got)
+
+
+@pytest.mark.parametrize("split", [8, 4])
+@pytest.mark.parametrize("lna,steps,spe", [(3, 6, 3), (24, 12, 4), (61, 68, 34)])
+def test_workgroups_of_four_and_eight_share_a_cu(split, lna, steps, spe):
+    """Asked for: one replica a workgroup, and two or more workgroups a CU
+    (registers for four wavefronts a SIMD; LDS allows two of these complexes'
+    or more); fewer atom blocks than wavefronts, and more."""
+    job = _job(lna, 200, 200, 2, 4, steps=steps, spe=spe, seed=lna)
+    E = remc.Engine(arena_bytes=1 << 26, use_graph=0, split=split)
+    h = E.add(job)
+    E.cycles(steps // spe)
+    E.sync()
+    got, _ = E.results(h)
+    _same(job, got)
+    layout = E.layout()
+    assert layout["split"] == split and layout["resident_groups"] >= 2 * 256
+    E.close()
