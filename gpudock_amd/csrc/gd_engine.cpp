@@ -256,7 +256,13 @@ bool gd_engine::can_split(const GdImage &I) const
  * Up to four share one and its staged tables: they take turns on the same
  * SIMDs, but the serial end of a step (sums, decision; some 4,000 cycles) is
  * paid once for all, and a last round of workgroups is not left half empty.
- * So of the shares that fit, the one with the least rounds x (share + 1).
+ * So of the shares that fit, the one with the least rounds x (share + 1).  A
+ * round of two, three, four takes 105, 153, 187 us a cycle at 24 x 300 and two
+ * rounds of one 130 (61 x 1,037: 420, 610, too large for four, and 490): the sum
+ * orders them rightly if it does not scale with them.  At 24 x 300, 34 x 344, 48 x
+ * 800, 16 x 1,500, 96 x 800 and 61 x 1,037, with 264, 400, 592, 768, 1,008, 1,536,
+ * 2,048 and 3,008 replicas each, no other share that was timed beside the
+ * rule's (one, two and four where it fits) was faster.
  * Cycle of 10 steps of 592 replicas of 61 atoms x 1,037 points: one wavefront
  * per replica 2.68 ms, two workgroups of 8 a CU, two rounds 0.82 ms, three
  * replicas a workgroup, one round 0.70 ms; 2,048 of 46 x 800, one wavefront

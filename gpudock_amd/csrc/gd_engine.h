@@ -105,10 +105,10 @@ struct gd_engine {
   size_t packs_off = 0, packs_bytes = 0, tasks_off = 0, tasks_bytes = 0, chains_off = 0,
          chains_bytes = 0;
   int n_cx = 0, n_tasks = 0, n_chain = 0;
-  /* MC launches of a cycle: complexes with as many wavefronts per replica
-   * whose LDS need gives the same workgroups per CU share one launch (tasks [off, off + n) of the task
-   * list, queue counter = class index), so a large pocket does not lower
-   * the occupancy of the small ones */
+  /* MC launches of a cycle: complexes with as many wavefronts and replicas a
+   * workgroup whose LDS need gives the same workgroups per CU share one launch
+   * (tasks [off, off + n) of the task list, queue counter = class index), so a
+   * large pocket does not lower the occupancy of the small ones */
   struct Class {
     int stage, off, n, grid, per_cu, split, share;
   };
@@ -195,13 +195,13 @@ private:
   /* LDS staging bytes of a complex */
   int stage_of(const GdImage &I) const;
   long long replicas() const;
-  /* wavefronts per replica of one complex, n_rep replicas resident in all,
-   * and the most over the resident complexes */
   /* a complex's workgroups: wavefronts (1: one per replica) and replicas */
   struct Split {
     int waves, share;
     int per_replica() const { return waves / share; }
   };
+  /* those of one complex, n_rep replicas resident in all, and the most
+   * wavefronts per replica over the resident complexes */
   Split split_of(const GdImage &I, long long n_rep) const;
   int choose_split() const;
 };

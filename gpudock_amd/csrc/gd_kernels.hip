@@ -560,62 +560,37 @@ __device__ __forceinline__ float gd_lhm_one(const gd_hot &H, float ax0, float ay
   return c > 0 ? gd_uload(H.mcs_tcc + m) * gd_sqrt(s / (float) c) : 0.0f;
 }
 
-/* From the summed terms to the energies: KDE normalisation, the restraint
- * log, the distance term, averaging, normalisation and total
- * (calcenergy_d.cu:276-371); out[] (slot order) and *cmcc uniform.  vdw ..
- * kde are the wave sums of the lane totals. */
 /* distance of the placed centre to the pocket centre (calcenergy_d.cu:276-283) */
 __device__ __forceinline__ float gd_edst(const float pc[3], const float cen[3])
 {
   return gd_sqrt(gd_dist2(cen[0] - pc[0], cen[1] - pc[1], cen[2] - pc[2]));
 }
 
-__device__ __forceinline__ void gd_energy_final_d(const gd_pack &P, float vdw, float ele,
-                                                  float pmf, float hdb, float psp, float ehpc,
-                                                  float kde, float elhm_sum, int tp, int fp,
-                                                  int fn, float edst, float out[GD_E_N],
-                                                  float *cmcc)
+/* From the lane totals to the energies: wave sums, KDE normalisation, the
+ * restraint log, the distance term, averaging, normalisation and total
+ * (calcenergy_d.cu:276-371); out[] (slot order) and *cmcc uniform. */
+__device__ __forceinline__ void gd_energy_tail(const gd_pack &P, const gd_blk &tot,
+                                               float ehpc, float kde_lane, float elhm_sum,
+                                               int tp, int fp, int fn, const float cen[3],
+                                               float out[GD_E_N], float *cmcc)
 {
   const int pos = P.pos;
-  const float ekde = kde / P.kde3;
-  const float elhm = (pos > 0) ? gd_log(elhm_sum / (float) pos) : 0.0f;
   float sums[GD_F_NTERM];
-  sums[GD_F_VDW] = vdw;
-  sums[GD_F_ELE] = ele * P.sc.inv_el1;   /* the pair loop sums el1 g */
-  sums[GD_F_PMF] = pmf;
+  sums[GD_F_VDW] = gd_wave_sum(tot.vdw);
+  sums[GD_F_ELE] = gd_wave_sum(tot.ele) * P.sc.inv_el1;   /* the pair loop sums el1 g */
+  sums[GD_F_PMF] = gd_wave_sum(tot.pmf);
   sums[GD_F_HPC] = ehpc;
-  sums[GD_F_HDB] = hdb;
-  sums[GD_F_DST] = edst;
-  sums[GD_F_PSP] = psp;
-  sums[GD_F_KDE] = ekde;
-  sums[GD_F_LHM] = elhm;
+  sums[GD_F_HDB] = gd_wave_sum(tot.hdb);
+  sums[GD_F_DST] = gd_edst(P.pocket_center, cen);
+  sums[GD_F_PSP] = gd_wave_sum(tot.psp);
+  sums[GD_F_KDE] = gd_wave_sum(kde_lane) / P.kde3;
+  sums[GD_F_LHM] = (pos > 0) ? gd_log(elhm_sum / (float) pos) : 0.0f;
   gd_finalize(sums, (float) P.lna, P.a_para, P.b_para, P.w, P.term_order, P.combine, out);
   *cmcc = 0.0f;
   if (P.mcc_ref) {
     const int tn = P.lna * P.pnp - tp - fp - fn;   /* padding points are never contacts */
     *cmcc = gd_mcc((float) tp, (float) fn, (float) fp, (float) tn);
   }
-}
-
-__device__ __forceinline__ void gd_energy_final(const gd_pack &P, float vdw, float ele,
-                                                float pmf, float hdb, float psp, float ehpc,
-                                                float kde, float elhm_sum, int tp, int fp,
-                                                int fn, const float cen[3], float out[GD_E_N],
-                                                float *cmcc)
-{
-  gd_energy_final_d(P, vdw, ele, pmf, hdb, psp, ehpc, kde, elhm_sum, tp, fp, fn,
-                    gd_edst(P.pocket_center, cen), out, cmcc);
-}
-
-/* The same from the lane totals: their wave sums first. */
-__device__ __forceinline__ void gd_energy_tail(const gd_pack &P, const gd_blk &tot,
-                                               float ehpc, float kde_lane, float elhm_sum,
-                                               int tp, int fp, int fn, const float cen[3],
-                                               float out[GD_E_N], float *cmcc)
-{
-  gd_energy_final(P, gd_wave_sum(tot.vdw), gd_wave_sum(tot.ele), gd_wave_sum(tot.pmf),
-                  gd_wave_sum(tot.hdb), gd_wave_sum(tot.psp), ehpc, gd_wave_sum(kde_lane),
-                  elhm_sum, tp, fp, fn, cen, out, cmcc);
 }
 
 /* One wavefront evaluates every block in order.  On return out[] (slot
@@ -1279,10 +1254,11 @@ static_assert(GD_SPLIT_DRAWS * 2 == GD_WAVE, "one lane per draw call");
 
 /* n_steps MC steps from step s0 of the Z.share replicas r0, r0 + 1, .. on the
  * SPLIT wavefronts of the workgroup, `role` = this wavefront's index.
- * Two wavefronts lead replica j, and the first of them keeps its state.  Per step: the wavefronts take items; barrier; the
- * sums; barrier; the keepers take the decisions; barrier.  The move of step s + 1 never waits for
- * the decision: among their items the two leaders place both poses that step
- * may start from, in the replica's two other buffers (the move from the
+ * Two wavefronts lead replica j, and the first of them keeps its state.  Per
+ * step: the wavefronts take items; barrier; the sums; barrier; the keepers take
+ * the decisions; barrier.  The move of step s + 1 never waits for the decision:
+ * among their items the two leaders place both poses that step may start from,
+ * in the replica's two other buffers (the move from the
  * current pose if this one is rejected, from the proposed one if it is
  * accepted: the same draws and arithmetic as placing it after the decision),
  * and the decision only selects the buffer; the state, the best pose and the
