@@ -379,9 +379,10 @@ int gd_build_image(GdImage &I, const gd_ligand *lig, const gd_protein *prt,
   P.off_kde = al16(P.off_tab + tab_bytes);
   const int with_kde = al16(P.off_kde + (P.pnk + 1) * 16);   /* with the padding point */
   /* the KDE points too, unless that keeps a replica out of a split workgroup:
-   * read through the caches they cost no measurable time (16,384 replicas of
-   * 48 x 800 with 2,000 KDE points 8.43 ms a cycle staged, 8.36 read through
-   * the caches) */
+   * read through the caches they cost little or nothing and leave room for
+   * more wavefronts (16,384 replicas of 48 x 800 with 2,000 KDE points, staged |
+   * read through the caches: 8.43 | 8.36 ms a cycle at the default register
+   * budget, 8.44 | 8.20 at 8 waves a SIMD, 8.31 | 8.53 at 6) */
   auto split_areas = [&](int stage) {
     return std::min(GD_SPLIT_MAX_SHARE,
                     (max_lds - stage - GD_SPLIT_LDS_BYTES(0)) / GD_SPLIT_AREA_BYTES);

@@ -407,7 +407,8 @@ typedef struct gd_engine_config {
                           every choice.  A complex with more than 64 position
                           restraints, or whose staged tables leave no room in
                           LDS for the split area, has one wavefront per
-                          replica whatever is asked */
+                          replica whatever is asked, and so have all in an
+                          arena with no room for the longer task lists */
   int prio;            /* 0-3: issue priority of the MC launches' wavefronts in
                           their SIMD against other streams' launches on the
                           device (s_setprio); 0 = the default */
@@ -535,9 +536,10 @@ typedef struct gd_server_config {
    * queues they did not, but four lanes served no better than three.
    * lane_split[k] > 1 runs lane k with that many wavefronts per replica (4,
    * 8 or 16): a few small jobs then fill the device, so they are done in a
-   * few cycles of their own instead of waiting in a large resident set.  A job that lane cannot split (more than 64
-   * restraints, or its tables do not fit in LDS beside the split area) goes
-   * to the next lane.  0 = split as above.
+   * few cycles of their own instead of waiting in a large resident set.  A
+   * job that lane cannot split (more than 64 restraints, or its tables do not
+   * fit in LDS beside the split area) goes to the next lane.  0 = split as
+   * above.
    * lane_max_jobs[k] > 0: lane k takes a job only while fewer jobs than
    * that are queued or resident on it; the others go to the next lane.  A
    * split lane holds a few jobs at a time at low latency and hands the rest
